@@ -360,3 +360,43 @@ def test_large_tlas_with_clas_overflow():
     tvisit(arr["tlasRoot"])
     assert sorted(seen) == list(range(n))
     compare_hits(gh, oh, gd, od)
+
+
+@pytest.mark.parametrize("layout,num", [("parallel", 1), ("parallel", 4096), ("grazing", 63), ("grazing", 4097),
+                                        ("scattered", 65), ("scattered", 6000)])
+def test_shared_leaf_steps_match_packets(layout, num):
+    """The leaf steps that share blocks over a wave's lanes give the packet
+    traversal's hits (one lane per block) byte for byte: parallel rays onto
+    whole clusters (every lane holds 32 groups, tested per lane), grazing rays
+    in one plane (few lanes hold leaves, many leaves per ray) and scattered
+    rays (blocks of all sizes in one wave: whole clusters and tessellated
+    parts); ragged ray counts leave lanes without a ray; also with the whole
+    stack in private memory."""
+    host = scene.scene_grid_instances(num_instances=4, quads=60, patch_size=8.0, tex_size=256, tess_rate_pixels=6.0)
+    rng = np.random.default_rng(num)
+    rays = np.zeros(num, abi.RAY_DT)
+    if layout == "parallel":
+        rays["origin"] = rng.uniform(0.0, 14.0, (num, 3))
+        rays["origin"][:, 1] = 5.0
+        rays["direction"] = (0.01, -1.0, 0.02)
+    elif layout == "grazing":
+        rays["origin"] = (1.0, 0.35, -2.0)
+        a = rng.uniform(-0.5, 0.5, num)
+        rays["direction"] = np.stack([np.sin(a), rng.uniform(-0.02, 0.005, num), np.cos(a)], 1)
+    else:
+        rays["origin"] = rng.uniform(0.0, 14.0, (num, 3)) * (1.0, 0.1, 1.0) + (0.0, 0.7, 0.0)
+        rays["direction"] = rng.normal(size=(num, 3))
+    rays["tMin"], rays["tMax"] = 0.0, 200.0
+    g = harness.GpuFrame(host, harness.small_config())
+    try:
+        g.run(host.frame(), stages="accel")
+        want = g.trace(0, 0, abi.TRACE_PACKETS, rays=rays)
+        got = [g.trace(0, 0, f, rays=rays) for f in (0, abi.TRACE_PRIVATE_STACK)]
+    finally:
+        g.close()
+    if num > 1000:
+        assert (want[0]["t"] > 0).mean() > 0.05, "rays must meet the surface"
+        assert len(np.unique(want[0]["clusterID"] >> 30)) > 1 or layout != "scattered"
+    for h, d in got:
+        assert np.array_equal(h.view(np.uint8), want[0].view(np.uint8))
+        assert np.array_equal(d.view(np.uint8), want[1].view(np.uint8))

@@ -27,26 +27,30 @@ struct WoopRay {
 // registers (a dynamic index into an array would go through private memory)
 __device__ __forceinline__ float pick3(float x, float y, float z, int k) { return k == 0 ? x : (k == 1 ? y : z); }
 
-__device__ __forceinline__ void setup_ray(WoopRay& r, const float o[3], const float dir[3]) {
-  float d[3];
+// The parts of a ray that box tests read.
+__device__ __forceinline__ void setup_box_ray(WoopRay& r, const float o[3], const float dir[3]) {
   for (int k = 0; k < 3; k++) {
-    d[k] = dir[k];
-    asm volatile("" : "+v"(d[k]));  // register values: the picks below stay selects
-    r.o[k] = o[k], r.d[k] = d[k], r.inv[k] = 1.0f / d[k];
+    float d = dir[k];
+    asm volatile("" : "+v"(d));  // register values: the picks of setup_ray stay selects
+    r.o[k] = o[k], r.d[k] = d, r.inv[k] = 1.0f / d;
   }
-  const float ax = fabsf(d[0]), ay = fabsf(d[1]), az = fabsf(d[2]);
+}
+
+__device__ __forceinline__ void setup_ray(WoopRay& r, const float o[3], const float dir[3]) {
+  setup_box_ray(r, o, dir);
+  const float ax = fabsf(r.d[0]), ay = fabsf(r.d[1]), az = fabsf(r.d[2]);
   r.kz = (ax > ay) ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
   r.kx = r.kz == 2 ? 0 : r.kz + 1;
   r.ky = r.kx == 2 ? 0 : r.kx + 1;
-  if (d[r.kz] < 0.0f) {
+  const float dz = pick3(r.d[0], r.d[1], r.d[2], r.kz);
+  if (dz < 0.0f) {
     const int t = r.kx;
     r.kx = r.ky;
     r.ky = t;
   }
-  const float dz = pick3(d[0], d[1], d[2], r.kz);
-  r.Sx = pick3(d[0], d[1], d[2], r.kx) / dz;
-  r.Sy = pick3(d[0], d[1], d[2], r.ky) / dz;
-  r.Sz = 1.0f / dz;
+  r.Sx = pick3(r.d[0], r.d[1], r.d[2], r.kx) / dz;
+  r.Sy = pick3(r.d[0], r.d[1], r.d[2], r.ky) / dz;
+  r.Sz = pick3(r.inv[0], r.inv[1], r.inv[2], r.kz);  // 1 / dz
 }
 
 // conservative slab test; returns entry distance or +inf
@@ -62,13 +66,14 @@ __device__ __forceinline__ float box_hit(const WoopRay& r, const float lo[3], co
   return tn <= tf * 1.0000005f ? tn : INFINITY;
 }
 
-struct TriHit {
-  float t, u, v;
+struct TriDet {
+  float t, V, W, det;
 };
 
-// Woop et al. 2013 with barycentrics (u: vertex 1, v: vertex 2)
-__device__ __forceinline__ bool tri_hit(const WoopRay& r, const float* p0, const float* p1, const float* p2, bool cullBack,
-                                        float tmin, float tmax, TriHit& h) {
+// Woop et al. 2013 with barycentrics V / det (vertex 1) and W / det
+// (vertex 2), which only a ray's closest hit divides out
+__device__ __forceinline__ bool tri_test(const WoopRay& r, const float* p0, const float* p1, const float* p2, bool cullBack,
+                                         float tmin, float tmax, TriDet& h) {
   const float A0 = p0[0] - r.o[0], A1 = p0[1] - r.o[1], A2 = p0[2] - r.o[2];
   const float B0 = p1[0] - r.o[0], B1 = p1[1] - r.o[1], B2 = p1[2] - r.o[2];
   const float C0 = p2[0] - r.o[0], C1 = p2[1] - r.o[1], C2 = p2[2] - r.o[2];
@@ -93,8 +98,7 @@ __device__ __forceinline__ bool tri_hit(const WoopRay& r, const float* p0, const
   const float t = T / det;
   if (!(t >= tmin && t <= tmax)) return false;
   h.t = t;
-  h.u = V / det;
-  h.v = W / det;
+  h.V = V, h.W = W, h.det = det;
   return true;
 }
 
@@ -219,8 +223,8 @@ __device__ __forceinline__ bool clas_hit(const WoopRay& r, const char* clas, uin
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       if (t0 + j >= nt) break;
-      TriHit th;
-      if (!tri_hit(r, v[j], v[j] + 3, v[j] + 6, cullBack, tmin, best.h.t, th)) continue;
+      TriDet th;
+      if (!tri_test(r, v[j], v[j] + 3, v[j] + 6, cullBack, tmin, best.h.t, th)) continue;
       const uint32_t prim = w[j] >> 24;
       if (anyHit) {
         best.h.t = th.t;
@@ -228,8 +232,8 @@ __device__ __forceinline__ bool clas_hit(const WoopRay& r, const char* clas, uin
       }
       if (key_less(th.t, instanceID, clusterID, prim, best.h)) {
         best.h.t = th.t;
-        best.h.u = th.u;
-        best.h.v = th.v;
+        best.h.u = th.V / th.det;
+        best.h.v = th.W / th.det;
         best.h.instanceID = instanceID;
         best.h.clusterID = clusterID;
         best.h.primitiveID = prim;
@@ -244,19 +248,26 @@ __device__ __forceinline__ bool clas_hit(const WoopRay& r, const char* clas, uin
 }
 
 // Traversal stack of one lane: the first kLdsStack entries in LDS (stride
-// T, the workgroup size), the rest in a private array.  TLAS and BLAS
-// entries share it: the BLAS entries of the instance being walked sit above
-// the stack depth at which it was entered.  Bound: every visited node
-// pushes at most 3 of its 4 slots, and the four-wide view visits every
-// other level, so a ray holds at most 3 * (ceil(dT / 2) + ceil(dB / 2))
-// entries for binary depths dT (TLAS) and dB (BLAS).  A Karras tree's depth
-// is at most its distinct key bits plus the index bits that break ties.
-// TLAS keys are a 30-bit Morton code above the instance index, so dT <=
-// 30 + 16 = 46 (2^16 instances); a BLAS covers one instance's segment,
-// whose keys differ only in the 24-bit Morton code, so dB <= 24 + 23 = 47
-// (2^23 references).  That is at most 3 * (23 + 24) = 141 < kStackDepth.
-constexpr uint32_t kLdsStack = 24;
+// 64), the rest in a private array.  TLAS and BLAS entries share it: a kDone
+// sentinel lies at its bottom and another below the BLAS entries of the
+// instance being walked, so a pop needs no depth test to end a walk.  Bound:
+// every visited node pushes at most 3 of its 4 slots, and the four-wide view
+// visits every other level, so a ray holds at most 3 * (ceil(dT / 2) +
+// ceil(dB / 2)) entries and two sentinels for binary depths dT (TLAS) and dB
+// (BLAS).  A Karras tree's depth is at most its distinct key bits plus the
+// index bits that break ties.  TLAS keys are a 30-bit Morton code above the
+// instance index, so dT <= 30 + 16 = 46 (2^16 instances); a BLAS covers one
+// instance's segment, whose keys differ only in the 24-bit Morton code, so
+// dB <= 24 + 23 = 47 (2^23 references).  That is at most 3 * (23 + 24) + 2 =
+// 143 < kStackDepth.
+constexpr uint32_t kLdsStack = 16;
 constexpr uint32_t kStackDepth = 160;
+// The node loop hands over to a leaf step when fewer lanes than this still
+// search (and some lane holds a leaf): the step costs what its leaves cost,
+// so it need not wait for stragglers.  4107 -> 3950 us at the 3840 x 2160
+// patch frame, 148 -> 131 us at a 320 x 180 icosphere and no difference at
+// grid64 against waiting for all; 16 and more lose at grid64 (488 -> 492-510 us).
+constexpr uint32_t kMinSearch = 8;
 constexpr uint32_t kDone = 0xFFFFFFFFu;
 
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
@@ -264,41 +275,21 @@ typedef __attribute__((address_space(5))) uint32_t private_u32;
 
 // Holds no array itself, so the stack pointer lives in a register; the
 // typed pointers make every access a ds_* or scratch_* instruction.
-template <uint32_t T>
 struct RayStack {
-  lds_u32* lds;         // this lane's first entry, stride T
-  private_u32* spill;   // kStackDepth private entries
-  uint32_t ldsDepth;    // kLdsStack, or 0 with TC_TRACE_PRIVATE_STACK
+  lds_u32* lds;        // this lane's first entry, stride kWave
+  private_u32* spill;  // kStackDepth private entries
+  uint32_t ldsDepth;   // kLdsStack, or 0 with TC_TRACE_PRIVATE_STACK
   uint32_t sp;
   __device__ __forceinline__ void push(uint32_t e) {
     if (sp < ldsDepth)
-      lds[sp * T] = e;
+      lds[sp * kWave] = e;
     else if (sp < kStackDepth)
       spill[sp - ldsDepth] = e;
     sp++;
   }
   __device__ __forceinline__ uint32_t pop() {
     --sp;
-    return sp < ldsDepth ? lds[sp * T] : spill[sp - ldsDepth];
-  }
-  // next entry above stack depth `base`, or kDone
-  __device__ __forceinline__ uint32_t pop_above(uint32_t base) { return sp > base ? pop() : kDone; }
-  // pushes c[3], c[2], c[1] where t[k] < inf, with t ascending (the misses
-  // are a suffix).  With room in LDS every entry is written and only the
-  // pointer advance depends on the hit, so the wave runs no branch.
-  __device__ __forceinline__ void push3(const uint32_t c[4], const float t[4]) {
-    if (sp + 3 <= ldsDepth) {
-      lds[sp * T] = c[3];
-      sp += t[3] != INFINITY;
-      lds[sp * T] = c[2];
-      sp += t[2] != INFINITY;
-      lds[sp * T] = c[1];
-      sp += t[1] != INFINITY;
-    } else {
-      if (t[3] != INFINITY) push(c[3]);
-      if (t[2] != INFINITY) push(c[2]);
-      if (t[1] != INFINITY) push(c[1]);
-    }
+    return sp < ldsDepth ? lds[sp * kWave] : spill[sp - ldsDepth];
   }
 };
 
@@ -340,41 +331,301 @@ __device__ __forceinline__ void node_slots(const tc_bvh4_node* node, const WoopR
   }
 }
 
+// (entry distance, child) of a slot as one double: the distance's bits are
+// the high word, so doubles order as the distances do (negative ones, which
+// only a negative tMin lets in, in reverse; the order of visits is a matter of
+// speed alone), and one v_min_f64 / v_max_f64 pair swaps distance and child
+// together.  A compare and four selects did that before.  The asm keeps
+// fmin / fmax from quieting their operands first (the high words are never
+// those of a NaN: an entry distance is a number or +inf).
+__device__ __forceinline__ double slot_key(float t, uint32_t c) {
+  return __longlong_as_double((long long)(((uint64_t)__float_as_uint(t) << 32) | c));
+}
+__device__ __forceinline__ void sort2(double& a, double& b) {
+  double lo, hi;
+  asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+  asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+  a = lo, b = hi;
+}
+__device__ __forceinline__ float key_t(double k) { return __uint_as_float((uint32_t)((uint64_t)__double_as_longlong(k) >> 32)); }
+__device__ __forceinline__ uint32_t key_child(double k) { return (uint32_t)__double_as_longlong(k); }
+
 // Visits one node: pushes the hit slots but the nearest (farthest first)
-// and returns the nearest one's child, or the next entry above `base`
-// when no slot is hit.
-template <uint32_t T>
+// and returns the nearest one's child, or pops when no slot is hit.  The top
+// of the stack is read ahead of the box tests and every LDS entry is written
+// whether its slot is hit or not; only the pointer advance depends on the
+// hits (h hits move it by h - 1, one pop being -1), so the wave runs no branch.
 __device__ __forceinline__ uint32_t visit_node(const tc_bvh4_node* node, const WoopRay& r, float tmin, float tmax,
-                                               RayStack<T>& stack, uint32_t base) {
+                                               RayStack& stack) {
+  const uint32_t top = stack.lds[min(stack.sp - 1, kLdsStack - 1) * kWave];
   float t[4];
   uint32_t c[4];
   node_slots(node, r, tmin, tmax, t, c);
-  cswap(t, c, 0, 1);
-  cswap(t, c, 2, 3);
-  cswap(t, c, 0, 2);
-  cswap(t, c, 1, 3);
-  cswap(t, c, 1, 2);
-  if (t[0] == INFINITY) return stack.pop_above(base);
-  stack.push3(c, t);
-  return c[0];
+  double k0 = slot_key(t[0], c[0]), k1 = slot_key(t[1], c[1]), k2 = slot_key(t[2], c[2]), k3 = slot_key(t[3], c[3]);
+  sort2(k0, k1);
+  sort2(k2, k3);
+  sort2(k0, k2);
+  sort2(k1, k3);
+  sort2(k1, k2);
+  const uint32_t h0 = key_t(k0) != INFINITY, h1 = key_t(k1) != INFINITY, h2 = key_t(k2) != INFINITY,
+                 h3 = key_t(k3) != INFINITY;
+  if (stack.sp + 3 <= stack.ldsDepth) {
+    uint32_t sp = stack.sp;
+    stack.lds[sp * kWave] = key_child(k3);
+    sp += h3;
+    stack.lds[sp * kWave] = key_child(k2);
+    sp += h2;
+    stack.lds[sp * kWave] = key_child(k1);
+    stack.sp = sp + h1 + h0 - 1;
+    return h0 ? key_child(k0) : top;
+  }
+  if (!h0) return stack.pop();
+  if (h3) stack.push(key_child(k3));
+  if (h2) stack.push(key_child(k2));
+  if (h1) stack.push(key_child(k1));
+  return key_child(k0);
 }
 
-// Full two-level traversal of one ray over the four-wide views.  Returns
-// true if anything was hit.  The TLAS walk stops at each instance whose
-// BLAS has clusters; that BLAS is walked with the object-space ray until
-// the stack is back at the depth it was entered at.
-template <uint32_t T>
-__device__ bool trace_ray(const TraceArgs& a, const float o[3], const float d[3], float tmin, float tmax, bool cullBack,
-                          bool anyHit, RayStack<T>& stack, HitState& best) {
-  best.h.t = tmax;
-  best.h.u = best.h.v = 0.0f;
-  best.h.instanceID = best.h.clusterID = best.h.primitiveID = 0xFFFFFFFFu;
-  best.clas = nullptr;
+// LDS of one wave: the lanes' stacks and the state of a leaf step.
+constexpr uint32_t kLeafQueue = 144;  // 15 left over + 128 of one step, rounded up
+struct WaveLds {
+  uint32_t stack[kLdsStack * kWave];
+  float4 rayO[kWave];          // origin, closest hit so far
+  float4 rayI[kWave];          // inverse direction, tMin
+  float4 rayS[kWave];          // shear, permutation | triangles << 8 | groups << 16
+  uint4 leaf[kWave];           // CLAS address, (ordered t, primitive) of the closest hit
+  float4 won[kWave];           // that hit's V, W, determinant and triangle word
+  uint64_t heads[16];          // bit per group-box pair: the first of its lane
+  uint32_t lanes[kWave];       // lanes with leaves, in order: lane | groups << 8 | first pair << 16
+  uint16_t queue[kLeafQueue];  // groups entered: lane | group << 6
+};
+
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Inclusive sum over the wave's lanes (all active).
+__device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return v;
+}
+
+// Floats as unsigned words of the same order (-0 as 0).
+__device__ __forceinline__ uint32_t ordered(float t) {
+  const uint32_t u = __float_as_uint(t + 0.0f);
+  return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
+}
+__device__ __forceinline__ float from_ordered(uint32_t u) {
+  return __uint_as_float((u & 0x80000000u) ? u ^ 0x80000000u : ~u);
+}
+
+// Closest hit of a ray; barycentrics are V / det and W / det.
+struct BestHit {
+  float t, V, W, det;
+  uint32_t instanceID, clusterID, primitiveID;
+  uint32_t word;     // triangle word
+  const char* clas;  // CLAS block, null: no hit
+};
+
+__device__ __forceinline__ bool key_less(float t, uint32_t i, uint32_t c, uint32_t p, const BestHit& best) {
+  if (t != best.t) return t < best.t;
+  if (i != best.instanceID) return i < best.instanceID;
+  if (c != best.clusterID) return c < best.clusterID;
+  return p < best.primitiveID;
+}
+
+typedef float gfloat3 __attribute__((ext_vector_type(3), aligned(4)));
+__device__ __forceinline__ gfloat3 gload3(const float* p) {
+  return *(const __attribute__((address_space(1))) gfloat3*)p;
+}
+
+// Intersects the CLAS blocks that the wave's lanes hold (`has`), sharing the
+// work over all 64 lanes; the whole wave calls it.  The traversal is bound by
+// VALU issue (82 % busy at grid64), and what it issues is mostly idle lanes:
+// about 22 of 64 lanes arrive with a leaf, their blocks hold 2 to 32 groups,
+// and when each lane tested its own block's triangles 15 of 64 lanes were at
+// work.  So every lane puts its ray in LDS, the group boxes of all blocks are
+// numbered through (pairs of boxes, 48 bytes) and dealt one pair per lane,
+// groups entered go to a queue, and the triangles of 16 queued groups at a
+// time are dealt one per lane.  A candidate enters its ray's (t, primitive)
+// minimum in LDS, so the result is that of testing one triangle after another.
+// Measured against one lane per block (trace launch, same hits): grid64 552 ->
+// 485 us, 500 meshes 1160 -> 856 us, patch field at 3840 x 2160 4975 -> 3850
+// us, icosphere at 320 x 180 161 -> 132 us, parallel rays onto whole clusters
+// (384^2 depth rays) 15.5 -> 17.5 us.
+__device__ __forceinline__ void leaf_step(WaveLds& w, bool has, const char* clas, uint64_t info, const WoopRay& ray,
+                                          float tmin, float tmax, bool cullBack, bool anyHit) {
+  const uint32_t lane = lane_id();
+  const uint32_t nt = (uint32_t)info & 0xFF, ng = ((uint32_t)info >> 16) & 0xFF;
+  const uint32_t npairs = has ? (ng + 1) >> 1 : 0;
+  const uint32_t end = wave_scan_dpp(npairs), first = end - npairs;
+  const uint32_t total = __builtin_amdgcn_readlane(end, 63);
+  if (lane < 16) w.heads[lane] = 0;
+  wave_sync();
+  const uint64_t holders = ballot(has);
+  if (has) {
+    const uint64_t addr = reinterpret_cast<uint64_t>(clas);
+    w.rayO[lane] = make_float4(ray.o[0], ray.o[1], ray.o[2], tmax);
+    w.rayI[lane] = make_float4(ray.inv[0], ray.inv[1], ray.inv[2], tmin);
+    w.rayS[lane] = make_float4(ray.Sx, ray.Sy, ray.Sz,
+                               __uint_as_float((uint32_t)(ray.kx | ray.ky << 2 | ray.kz << 4) | nt << 8 | ng << 16));
+    w.leaf[lane] = make_uint4((uint32_t)addr, (uint32_t)(addr >> 32), ~0u, ~0u);
+    w.lanes[mask_prefix(holders)] = lane | ng << 8 | first << 16;
+    __hip_atomic_fetch_or(reinterpret_cast<uint32_t*>(w.heads) + (first >> 5), 1u << (first & 31), __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_WAVEFRONT);
+  }
+  wave_sync();
+  // Which way the group boxes are tested, by what the two cost in units of
+  // about 50 instructions: each lane its own block (one per pair of the largest
+  // block, in steps of two pairs, and two to queue the groups) or the pairs
+  // dealt out (two per 64 pairs).  Lanes that all hold whole clusters, as
+  // under parallel rays, are better off with their own: 384^2 depth rays take
+  // 17.5 us, 22.8 us with pairs always dealt out; steps of four pairs spill.
+  uint32_t most = npairs;  // the wave's largest, in lane 63
+  most = max(most, (uint32_t)__builtin_amdgcn_update_dpp(0, most, 0x111, 0xf, 0xf, true));
+  most = max(most, (uint32_t)__builtin_amdgcn_update_dpp(0, most, 0x112, 0xf, 0xf, true));
+  most = max(most, (uint32_t)__builtin_amdgcn_update_dpp(0, most, 0x114, 0xf, 0xf, true));
+  most = max(most, (uint32_t)__builtin_amdgcn_update_dpp(0, most, 0x118, 0xf, 0xf, true));
+  most = max(most, (uint32_t)__builtin_amdgcn_update_dpp(0, most, 0x142, 0xa, 0xf, false));
+  most = max(most, (uint32_t)__builtin_amdgcn_update_dpp(0, most, 0x143, 0xc, 0xf, false));
+  most = __builtin_amdgcn_readlane(most, 63);
+  const bool own = (most == 1 ? 1 : (most + 1) & ~1u) + 2 <= 2 * ((total + kWave - 1) / kWave);
+  uint32_t mask = 0;  // own: this lane's groups entered and not queued yet
+  if (own) {
+    const float4* gq = reinterpret_cast<const float4*>(clas + sizeof(tc_clas_header));
+    mask = most == 1 ? group_mask<1>(ray, gq, npairs, tmin, tmax) : group_mask<2>(ray, gq, npairs, tmin, tmax);
+    if (ng < 32) mask &= (1u << ng) - 1u;
+  }
+  uint32_t starts = 0, queued = 0;  // wave-uniform
+  for (uint32_t base = 0;; base += kWave) {
+    bool last;
+    if (own) {
+      const bool in = mask != 0;
+      const uint64_t m = ballot(in);
+      if (in) w.queue[queued + mask_prefix(m)] = (uint16_t)(lane | (uint32_t)__builtin_ctz(mask) << 6);
+      mask &= mask - 1;
+      queued += __popcll(m);
+      last = !ballot(mask != 0);
+    } else {
+      last = base + kWave >= total;
+      // the lane whose block holds pair base + lane: the number of first pairs
+      // up to it
+      const uint64_t heads = uniform64(w.heads[base / kWave]);
+      const uint32_t at = starts + (uint32_t)(heads & 1) + mask_prefix(heads >> 1) - 1;
+      starts += __popcll(heads);
+      const bool valid = base + lane < total;
+      bool in0 = false, in1 = false;
+      uint32_t owner = 0, pair = 0;
+      if (valid) {
+        const uint32_t e = w.lanes[at];
+        owner = e & 63;
+        pair = base + lane - (e >> 16);
+        const float4 ro = w.rayO[owner], ri = w.rayI[owner];
+        const uint2 ca = *reinterpret_cast<const uint2*>(&w.leaf[owner]);
+        const float4* gq =
+            reinterpret_cast<const float4*>((((uint64_t)ca.y << 32) | ca.x) + sizeof(tc_clas_header) + pair * 48ull);
+        const float4 a0 = gload(gq), a1 = gload(gq + 1), a2 = gload(gq + 2);
+        WoopRay br;
+        br.o[0] = ro.x, br.o[1] = ro.y, br.o[2] = ro.z;
+        br.inv[0] = ri.x, br.inv[1] = ri.y, br.inv[2] = ri.z;
+        in0 = group_hit(br, a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, ri.w, ro.w) != 0;
+        in1 = 2 * pair + 1 < ((e >> 8) & 0xFF) && group_hit(br, a1.z, a1.w, a2.x, a2.y, a2.z, a2.w, ri.w, ro.w) != 0;
+      }
+      const uint64_t m0 = ballot(in0), m1 = ballot(in1);
+      if (in0) w.queue[queued + mask_prefix(m0)] = (uint16_t)(owner | (2 * pair) << 6);
+      queued += __popcll(m0);
+      if (in1) w.queue[queued + mask_prefix(m1)] = (uint16_t)(owner | (2 * pair + 1) << 6);
+      queued += __popcll(m1);
+    }
+    wave_sync();
+    // triangles of the queued groups, 16 groups at a time (all that is left
+    // after the last pairs)
+    uint32_t q = 0;
+    for (; q + 16 <= queued || (last && q < queued); q += 16) {
+      const uint32_t k = q + (lane >> 2);
+      uint32_t who = 0;
+      uint64_t key = ~0ull;
+      float V = 0.f, W = 0.f, det = 1.f;
+      uint32_t word = 0;
+      bool hit = false;
+      if (k < queued) {
+        const uint32_t e = w.queue[k];
+        who = e & 63;
+        const uint32_t tri = (e >> 6) * TC_CLAS_GROUP_TRIANGLES + (lane & 3);
+        const float4 rs = w.rayS[who];
+        const uint32_t code = __float_as_uint(rs.w);
+        const uint32_t bnt = (code >> 8) & 0xFF, bng = code >> 16;
+        if (tri < bnt) {
+          const uint2 ca = *reinterpret_cast<const uint2*>(&w.leaf[who]);
+          const char* tris = reinterpret_cast<const char*>(((uint64_t)ca.y << 32) | ca.x) + sizeof(tc_clas_header) +
+                             ((bng * 24u + 15u) & ~15u);
+          word = gload(reinterpret_cast<const uint32_t*>(tris) + tri);
+          const float* verts = reinterpret_cast<const float*>(tris + ((bnt * 4u + 15u) & ~15u));
+          const gfloat3 p0 = gload3(verts + 3 * (word & 0xFF)), p1 = gload3(verts + 3 * ((word >> 8) & 0xFF)),
+                        p2 = gload3(verts + 3 * ((word >> 16) & 0xFF));
+          const float4 ro = w.rayO[who];
+          WoopRay tr;
+          tr.o[0] = ro.x, tr.o[1] = ro.y, tr.o[2] = ro.z;
+          tr.kx = code & 3, tr.ky = (code >> 2) & 3, tr.kz = (code >> 4) & 3;
+          tr.Sx = rs.x, tr.Sy = rs.y, tr.Sz = rs.z;
+          const float q0[3] = {p0.x, p0.y, p0.z}, q1[3] = {p1.x, p1.y, p1.z}, q2[3] = {p2.x, p2.y, p2.z};
+          TriDet h;
+          if (tri_test(tr, q0, q1, q2, cullBack, w.rayI[who].w, ro.w, h)) {
+            hit = true;
+            key = ((uint64_t)ordered(h.t) << 32) | (word >> 24);
+            V = h.V, W = h.W, det = h.det;
+          }
+        }
+      }
+      uint64_t* best = reinterpret_cast<uint64_t*>(&w.leaf[who].z);
+      if (hit) {
+        if (anyHit)
+          *best = 0;
+        else
+          __hip_atomic_fetch_min(best, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+      }
+      wave_sync();
+      if (hit && !anyHit && *best == key) w.won[who] = make_float4(V, W, det, __uint_as_float(word));
+      wave_sync();
+    }
+    if (last) break;
+    // the groups left over move to the front
+    const uint32_t left = queued - q;
+    uint32_t e = 0;
+    if (lane < left) e = w.queue[q + lane];
+    wave_sync();
+    if (lane < left) w.queue[lane] = (uint16_t)e;
+    queued = left;
+    wave_sync();
+  }
+}
+
+// Full two-level traversal of the wave's rays (the lanes with `live`) over
+// the four-wide views; the whole wave calls it.  Returns true in the lanes
+// whose ray hit anything.  The TLAS walk stops at each instance whose BLAS
+// has clusters; that BLAS is walked with the object-space ray until its stack
+// sentinel is popped.
+__device__ __forceinline__ bool trace_wave(const TraceArgs& a, WaveLds& w, RayStack& stack, const float o[3], const float d[3],
+                                           float tmin, float tmax, bool live, bool cullBack, bool anyHit, BestHit& best) {
+  best.t = tmax;
+  best.V = best.W = 0.0f;
+  best.det = 1.0f;
+  best.instanceID = best.clusterID = best.primitiveID = 0xFFFFFFFFu;
   best.word = 0;
+  best.clas = nullptr;
+  bool found = false;
   WoopRay world;
-  setup_ray(world, o, d);
+  setup_box_ray(world, o, d);
   stack.sp = 0;
-  uint32_t e = *a.tlasRoot;
+  stack.push(kDone);
+  uint32_t e = live ? *a.tlasRoot : kDone;
   while (true) {
     // TLAS: find the next instance leaf with clusters
     uint32_t inst = kDone;
@@ -385,37 +636,71 @@ __device__ bool trace_ray(const TraceArgs& a, const float o[3], const float d[3]
           inst = i;
           break;
         }
-        e = stack.pop_above(0);
+        e = stack.pop();
       } else {
-        e = visit_node(a.tlasNodes4 + e, world, tmin, best.h.t, stack, 0);
+        e = visit_node(a.tlasNodes4 + e, world, tmin, best.t, stack);
       }
     }
-    if (inst == kDone) break;
-    const tc_tlas_instance& ti = a.tlasInstances[inst];
+    if (!ballot(inst != kDone)) break;
     WoopRay ray;
-    {
+    const tc_bvh4_node* blas4 = a.blasNodes4;
+    const uint64_t* leafAddr = nullptr;
+    const uint64_t* leafInfo = nullptr;
+    uint32_t b = kDone;
+    if (inst != kDone) {
+      const tc_tlas_instance& ti = a.tlasInstances[inst];
       float ol[3], dl[3];
       xform34(ti.worldToObject, o, 1.0f, ol);
       xform34(ti.worldToObject, d, 0.0f, dl);
       setup_ray(ray, ol, dl);
+      blas4 = a.blasNodes4 + (ti.blasNodes - a.blasNodesBase) / sizeof(tc_bvh_node);
+      leafAddr = reinterpret_cast<const uint64_t*>(ti.blasLeaves);
+      leafInfo = a.blasLeafInfo + (ti.blasLeaves - a.blasLeavesBase) / 8;
+      stack.push(kDone);
+      b = ti.blasRoot;
     }
-    const tc_bvh4_node* blas4 = a.blasNodes4 + (ti.blasNodes - a.blasNodesBase) / sizeof(tc_bvh_node);
-    const uint64_t* blasLeaves = reinterpret_cast<const uint64_t*>(ti.blasLeaves);
-    const uint64_t* leafInfo = a.blasLeafInfo + (ti.blasLeaves - a.blasLeavesBase) / 8;
-    const uint32_t base = stack.sp;
-    uint32_t b = ti.blasRoot;
-    // while-while: every lane walks nodes until it holds a CLAS leaf (or has
-    // finished), then the lanes with leaves intersect them together
-    while (b != kDone) {
-      while (b != kDone && !(b & TC_BVH_LEAF)) b = visit_node(blas4 + b, ray, tmin, best.h.t, stack, base);
-      if (b == kDone) break;
-      const char* clas = reinterpret_cast<const char*>(gload(blasLeaves + (b & ~TC_BVH_LEAF)));
-      if (clas_hit(ray, clas, gload(leafInfo + (b & ~TC_BVH_LEAF)), inst, cullBack, anyHit, tmin, best)) return true;
-      b = stack.pop_above(base);
+    while (true) {
+      // lanes walk nodes until each holds a CLAS leaf or has finished, or too
+      // few still search
+      while (true) {
+        const uint64_t searching = ballot((int32_t)b >= 0);
+        if (!searching) break;
+        if ((uint32_t)__popcll(searching) < kMinSearch && ballot((int32_t)b < 0 && b != kDone)) break;
+        if ((int32_t)b >= 0) b = visit_node(blas4 + b, ray, tmin, best.t, stack);
+      }
+      const bool has = (int32_t)b < 0 && b != kDone;
+      if (!ballot(has)) break;
+      const char* clas = nullptr;
+      uint64_t info = 0;
+      if (has) {
+        clas = reinterpret_cast<const char*>(gload(leafAddr + (b & ~TC_BVH_LEAF)));
+        info = gload(leafInfo + (b & ~TC_BVH_LEAF));
+      }
+      leaf_step(w, has, clas, info, ray, tmin, best.t, cullBack, anyHit);
+      if (has) {
+        const uint32_t lane = lane_id();
+        const uint4 lf = w.leaf[lane];
+        const uint32_t clusterID = (uint32_t)(info >> 32);
+        if ((lf.z & lf.w) != ~0u) {
+          const float t = from_ordered(lf.w);
+          if (anyHit) {
+            found = true;
+          } else if (key_less(t, inst, clusterID, lf.z, best)) {
+            const float4 won = w.won[lane];
+            best.t = t;
+            best.V = won.x, best.W = won.y, best.det = won.z;
+            best.word = __float_as_uint(won.w);
+            best.instanceID = inst, best.clusterID = clusterID, best.primitiveID = lf.z;
+            best.clas = clas;
+          }
+        }
+        b = found ? kDone : stack.pop();
+      }
+      wave_sync();
     }
-    e = stack.pop_above(0);
+    if (inst != kDone) e = found ? kDone : stack.pop();
   }
-  return best.h.instanceID != 0xFFFFFFFFu;
+  return anyHit ? found : best.instanceID != 0xFFFFFFFFu;
 }
 
 // Wave-wide packet traversal: the 64 lanes of a wave walk one shared node
@@ -669,82 +954,100 @@ __device__ void decode_hit(const TraceArgs& a, const HitState& hs, tc_hit_decode
   out.depth = pp[2] / pp[3];
 }
 
-// Four waves per SIMD (at most 128 VGPRs): the batched loads of the CLAS
-// test need the registers, and a frame's time is set by the longest waves
-// (rays with many leaves), which gain more from fewer round trips than from
-// a fifth wave.
+// One ray per lane, 64 rays per wave.  The primary and the shadow walk are
+// two rounds of one loop, so the traversal is one piece of code in the
+// instruction cache.  A wave's lanes stay together through both: lanes without
+// a ray (ragged tiles, rays past the end, misses in the shadow round) help in
+// the leaf steps.
 template <uint32_t T>
 __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_trace(TraceArgs a) {
-  __shared__ uint32_t s_stack[kLdsStack * T];
+  __shared__ WaveLds s_wave[T / kWave];
   uint32_t spill[kStackDepth];
-  RayStack<T> stack;
-  stack.lds = (lds_u32*)(s_stack + threadIdx.x);
+  WaveLds& w = s_wave[threadIdx.x / kWave];
+  const uint32_t lane = lane_id();
+  RayStack stack;
+  stack.lds = (lds_u32*)(w.stack + lane);
   stack.spill = (private_u32*)spill;
   stack.ldsDepth = (a.flags & TC_TRACE_PRIVATE_STACK) ? 0u : kLdsStack;
+  stack.sp = 0;
   const bool cull = (a.flags & TC_TRACE_CULL_BACK) != 0;
   const bool shadows = (a.flags & TC_TRACE_SHADOW) != 0 && a.decoded;
   const uint32_t tilesX = (a.width + 7) / 8, tilesY = (a.height + 7) / 8;
   // tile-row order: the last ranking when it ranked this many rows.  Each
-  // wave's tile time goes to its row, timed from the top of one iteration
-  // to the top of the next (where the wave has reconverged), by an atomic
-  // nobody waits for.
+  // wave's tile time goes to its row by an atomic nobody waits for.
   TraceOrder* ord = !a.rays && a.order && tilesY <= kMaxOrderRows ? a.order : nullptr;
   const uint32_t* rowOrder = ord && ord->rows == tilesY ? ord->order : nullptr;
   if (ord && blockIdx.x == 0 && threadIdx.x == 0) ord->pendingRows = tilesY;
-  constexpr uint32_t kNoRow = 0xFFFFFFFFu;
-  uint32_t timedRow = kNoRow;
-  uint64_t t0 = 0;
-  for (uint32_t item = blockIdx.x * T + threadIdx.x; item < a.numItems; item += gridDim.x * T) {
-    if (ord) {
-      if (timedRow != kNoRow && lane_id() == 0)
-        time_tile_row(ord, timedRow, t0);
-      timedRow = kNoRow;
-      t0 = __builtin_amdgcn_s_memrealtime();
-    }
-    float o[3], d[3], tmin, tmax;
-    uint32_t r = item;
+  const uint32_t waves = gridDim.x * (T / kWave), numWaves = (a.numItems + kWave - 1) / kWave;
+  for (uint32_t wave = uniform(blockIdx.x * (T / kWave) + threadIdx.x / kWave); wave < numWaves; wave += waves) {
+    const uint64_t t0 = ord ? __builtin_amdgcn_s_memrealtime() : 0;
+    float o[3] = {0.f, 0.f, 0.f}, d[3] = {0.f, 0.f, 1.f}, tmin = 0.f, tmax = 0.f;
+    bool live = false;
+    uint32_t r = 0, timedRow = 0;
     if (a.rays) {
-      const tc_ray ray = a.rays[r];
-      for (int k = 0; k < 3; k++) o[k] = ray.origin[k], d[k] = ray.direction[k];
-      tmin = ray.tMin;
-      tmax = ray.tMax;
+      r = wave * kWave + lane;
+      live = r < a.numItems;
+      if (live) {
+        const tc_ray ray = a.rays[r];
+        for (int k = 0; k < 3; k++) o[k] = ray.origin[k], d[k] = ray.direction[k];
+        tmin = ray.tMin;
+        tmax = ray.tMax;
+      }
     } else {
       uint32_t tx, ty;
-      if (!strip_tile(item >> 6, T / kWave, tilesX, tilesY, rowOrder, tx, ty)) continue;
+      if (!strip_tile(wave, T / kWave, tilesX, tilesY, rowOrder, tx, ty)) continue;
       timedRow = ty;
-      const uint32_t in = item & 63, x = tx * 8 + (in & 7), y = ty * 8 + (in >> 3);
-      if (x >= a.width || y >= a.height) continue;
-      r = y * a.width + x;
-      primary_ray(a.view, x, y, a.width, a.height, o, d);
-      tmin = a.view->nearPlane;
-      tmax = a.view->farPlane;
-    }
-    HitState hs;
-    trace_ray(a, o, d, tmin, tmax, cull, false, stack, hs);
-    tc_hit hit = hs.h;
-    if (hit.instanceID == 0xFFFFFFFFu) hit.t = -1.0f;
-    if (a.hits) a.hits[r] = hit;
-    if (a.hitVertices) {
-      uint4 hv = make_uint4(~0u, ~0u, ~0u, ~0u);
-      if (hs.clas) {
-        const uint32_t base = reinterpret_cast<const tc_clas_header*>(hs.clas)->vertexBase;
-        hv = make_uint4(base + (hs.word & 0xFF), base + ((hs.word >> 8) & 0xFF), base + ((hs.word >> 16) & 0xFF), 0u);
+      const uint32_t x = tx * 8 + (lane & 7), y = ty * 8 + (lane >> 3);
+      live = x < a.width && y < a.height;
+      if (live) {
+        r = y * a.width + x;
+        primary_ray(a.view, x, y, a.width, a.height, o, d);
+        tmin = a.view->nearPlane;
+        tmax = a.view->farPlane;
       }
-      reinterpret_cast<uint4*>(a.hitVertices)[r] = hv;
     }
-    if (!a.decoded) continue;
-    tc_hit_decoded dec;
-    decode_hit(a, hs, dec);
-    if (shadows && hit.instanceID != 0xFFFFFFFFu) {
-      // render_shading.glsl:263-274: opaque, terminate on first hit
-      const float* sun = a.view->skyParams.sunDirection;
-      const float sd[3] = {sun[0], sun[1], sun[2]};
-      HitState sh;
-      dec.shadowed = trace_ray(a, dec.wPos, sd, 0.001f, 10000000.0f, false, true, stack, sh) ? 1u : 0u;
+#pragma nounroll
+    for (uint32_t round = 0; round < 2; round++) {
+      BestHit best;
+      const bool any = trace_wave(a, w, stack, o, d, tmin, tmax, live, cull && round == 0, round != 0, best);
+      if (round != 0) {
+        // render_shading.glsl:263-274: opaque, terminated on the first hit
+        if (live && any) a.decoded[r].shadowed = 1u;
+        break;
+      }
+      HitState hs;
+      hs.h.t = any ? best.t : -1.0f;
+      hs.h.u = best.V / best.det, hs.h.v = best.W / best.det;
+      hs.h.instanceID = best.instanceID, hs.h.clusterID = best.clusterID, hs.h.primitiveID = best.primitiveID;
+      hs.clas = best.clas, hs.word = best.word;
+      bool shade = false;
+      if (live) {
+        if (a.hits) a.hits[r] = hs.h;
+        if (a.hitVertices) {
+          uint4 hv = make_uint4(~0u, ~0u, ~0u, ~0u);
+          if (hs.clas) {
+            const uint32_t base = reinterpret_cast<const tc_clas_header*>(hs.clas)->vertexBase;
+            hv = make_uint4(base + (hs.word & 0xFF), base + ((hs.word >> 8) & 0xFF), base + ((hs.word >> 16) & 0xFF), 0u);
+          }
+          reinterpret_cast<uint4*>(a.hitVertices)[r] = hv;
+        }
+        if (a.decoded) {
+          tc_hit_decoded dec;
+          decode_hit(a, hs, dec);
+          a.decoded[r] = dec;
+          shade = shadows && any;
+          for (int k = 0; k < 3; k++) o[k] = dec.wPos[k];
+        }
+      }
+      if (!ballot(shade)) break;
+      // the shadow ray of every hit
+      live = shade;
+      for (int k = 0; k < 3; k++) d[k] = a.view->skyParams.sunDirection[k];
+      tmin = 0.001f;
+      tmax = 10000000.0f;
     }
-    a.decoded[r] = dec;
+    if (ord && lane == 0) time_tile_row(ord, timedRow, t0);
   }
-  if (ord && timedRow != kNoRow && lane_id() == 0) time_tile_row(ord, timedRow, t0);
 }
 
 // Packet form of k_trace: one wave per 64 work items (an 8 x 8 pixel tile
