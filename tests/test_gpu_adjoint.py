@@ -126,3 +126,38 @@ def test_adam_fit_200_steps():
     assert all(np.isfinite(losses))
     assert losses[-1] < 0.05 * losses[0]
     assert np.isfinite(heights.cpu().numpy()).all()
+
+
+@pytest.mark.parametrize("rays", [32, 33, 256])
+def test_gradient_of_scattered_rays(rays):
+    """The adjoint sums a workgroup's 1024 rays per texel in LDS before it
+    adds them to the map.  Rays in row order (many rays per texel) and the
+    same rays in random order (more texels per workgroup than the table has
+    slots) give one gradient: exactly 1024 rays (on the grid's own lines, where
+    most miss and the table stays nearly empty), a remainder of 65, and 64
+    workgroups.  Tolerance: each texel is a sum of at most K = 12 * rays^2 /
+    texels * 16 (sixteen times the mean) or 256 float32 terms of one sign,
+    so two orders differ by at most 2 K 2^-24 of the sum's size."""
+    import torch
+    from vk_tessellated_clusters_amd import diff, scene
+    heights = torch.from_numpy((0.5 * scene.fbm_height(SIZE, 7, 4)).astype(np.float32)).cuda()
+    r = diff.DepthRenderer(heights, rays=rays)
+    try:
+        t = r.render()
+        gen = torch.Generator().manual_seed(rays)
+        g = (torch.rand(rays * rays, generator=gen) + 0.5).cuda()
+        want = r.adjoint(g)
+        perm = torch.randperm(rays * rays, generator=gen).cuda()
+        for name, width in (("rays", abi.RAY_DT.itemsize), ("hits", abi.HIT_DT.itemsize)):
+            b = getattr(r, name).view(-1, width)
+            b.copy_(b[perm].clone())
+        hv = r.hit_vertices.view(-1, 4)
+        hv.copy_(hv[perm].clone())
+        got = r.adjoint(g[perm])
+        torch.cuda.synchronize()
+    finally:
+        r.close()
+    want, got = want.double().cpu().numpy(), got.double().cpu().numpy()
+    assert rays == 32 or np.count_nonzero(want) > rays * rays / 4
+    k = max(256.0, 12.0 * rays * rays / SIZE ** 2 * 16)
+    assert (np.abs(got - want) <= 2 * k * 2.0 ** -24 * np.abs(want) + 1e-30).all()
