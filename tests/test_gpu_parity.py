@@ -352,3 +352,21 @@ def test_device_fbm_matches_numpy():
         torch.cuda.synchronize()
         got = out.cpu().numpy().view(ref.dtype).reshape(size, size)
         assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("instances,quads", [(1, 24), (131, 64), (258, 64)])
+def test_classify_tile_sizes(instances, quads):
+    """Classify's tiles hold 8 clusters in small frames and up to 64 in large
+    ones: 9 clusters (a full and a ragged tile of 8), 8384 (tiles of 16) and
+    16,512 (tiles of 32, the last ragged) equal the oracle bit for bit."""
+    host = scene.scene_grid_instances(num_instances=instances, quads=quads, patch_size=8.0, tex_size=64)
+    cfg = harness.small_config(maxVisibleClusters=1 << 15, maxGeneratedClusters=1 << 17, maxPartTriangles=1 << 17)
+    of = harness.OracleFrame(host, cfg)
+    of.run(host.frame(), nthreads=8)
+    g = harness.GpuFrame(host, cfg)
+    try:
+        g.run(host.frame())
+        res = g.results()
+    finally:
+        g.close()
+    harness.compare(res, of.results())

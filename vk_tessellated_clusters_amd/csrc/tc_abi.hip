@@ -479,7 +479,7 @@ static void launch_prologue(const KArgs& a, int setupMode, uint32_t stage, hipSt
 
 static tc_status launch_classify(const KArgs& a, tc_config config, int setupMode, hipStream_t st) {
   launch_prologue(a, setupMode, 0, st);
-  uint32_t tiles = (config.maxVisibleClusters + kClassifyTile - 1) / kClassifyTile;
+  uint32_t tiles = (config.maxVisibleClusters + kClassifyMinTile - 1) / kClassifyMinTile;
   uint32_t grid = std::min<uint32_t>(tiles, (uint32_t)num_cu() * tuning_snapshot().classifyBlocksPerCU);
   if (config.flags & TC_FLAG_2X_TRANSIENT) {
     hipLaunchKernelGGL((k_cluster_classify<true, true>), dim3(grid), dim3(kClassifyWaves * kWave), 0, st, a);

@@ -320,6 +320,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   WsHeader* h = a.ws;
   const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
   const uint32_t epoch = h->epoch, numTiles = h->numTiles, numItems = h->itemEnd;
+  const uint32_t tileItems = h->tileItems;
   const uint64_t B0 = h->base[0], B1 = h->base[1], B2 = h->base[2], B3 = h->base[3], B4 = h->base[4], B5 = h->base[5];
   const uint64_t B6 = h->base[6], B7 = h->base[7];
   const ViewParams vp = view_params(a);
@@ -336,8 +337,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     __syncthreads();
     const uint32_t tile = s_tile;
     if (tile >= numTiles) break;
-    const uint32_t tileBase = tile * kClassifyTile;
-    const uint32_t cnt = min(kClassifyTile, numItems - tileBase);
+    const uint32_t tileBase = tile * tileItems;
+    const uint32_t cnt = min(tileItems, numItems - tileBase);
 
     // ---- 0. cluster and instance records (:150-176)
     if (threadIdx.x < cnt) {

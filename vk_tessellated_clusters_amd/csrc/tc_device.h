@@ -560,7 +560,8 @@ struct WsHeader {
   uint32_t numTiles;  // tiles of the current launch
   uint32_t itemBegin; // first item of the current launch
   uint32_t itemEnd;   // end of the items of the current launch
-  uint32_t _pad[3];
+  uint32_t tileItems; // items per tile, where the stage varies them (classify)
+  uint32_t _pad[2];
   uint64_t base[8];   // counter values at launch start
 };
 constexpr uint64_t kWsHeaderBytes = 1024;

@@ -38,7 +38,10 @@ __device__ void prologue_body(const KArgs& a, uint32_t stage) {
   h->ticket = 0;
   if (stage == kStageClassify) {
     const uint32_t n = min(b->visibleClusterCounter, a.cfg.maxVisibleClusters);
-    h->numTiles = min((n + kClassifyTile - 1) / kClassifyTile, a.maxTiles);
+    uint32_t ts = kClassifyTile;
+    while (ts > kClassifyMinTile && n < ts * kClassifyTiles && (n + ts / 2 - 1) / (ts / 2) <= a.maxTiles) ts /= 2;
+    h->tileItems = ts;
+    h->numTiles = min((n + ts - 1) / ts, a.maxTiles);
     h->itemBegin = 0;
     h->itemEnd = n;
     h->base[0] = (uint32_t)b->splitTriangleCounter;

@@ -8,7 +8,15 @@ namespace tc {
 enum Stage : uint32_t { kStageClassify = 0, kStageSplit = 1, kStageInstantiate = 2 };
 
 constexpr uint32_t kClassifyWaves = 4;   // waves per classify workgroup
-constexpr uint32_t kClassifyTile = 64;   // visible clusters per classify tile
+constexpr uint32_t kClassifyTile = 64;   // visible clusters per classify tile, at most
+// A tile's four waves take its clusters one after another, so a frame with
+// fewer clusters than fill the chip 64 at a time takes smaller tiles: halved
+// down to 8 while that leaves fewer than kClassifyTiles tiles.  64 clusters of
+// 81 vertices: 72 us in one tile of 64, 21 us in eight of 8; 245 clusters with
+// ripple 62 -> 30 us.  Tiles of 4, and 256 or 1024 tiles, measure the same; 2048
+// tiles (of 32, at 65,536 clusters) make the frame 1082 -> 1120 us.
+constexpr uint32_t kClassifyMinTile = 8;
+constexpr uint32_t kClassifyTiles = 512;
 constexpr uint32_t kVertCache = 128;     // vertices per wave a classify cluster caches
 constexpr uint32_t kInstWaves = 4;       // waves per instantiate workgroup
 constexpr uint32_t kInstTile = kInstWaves * 4 * 64;  // part triangles per instantiate tile (4 per lane)
