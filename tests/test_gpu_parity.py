@@ -370,3 +370,47 @@ def test_classify_tile_sizes(instances, quads):
     finally:
         g.close()
     harness.compare(res, of.results())
+
+
+@pytest.mark.parametrize("quads,rate,stride", [(8, 4000.0, 12), (40, 3.0, 12), (40, 3.0, 16), (64, 1.0, 12)])
+def test_clas_runs_and_rounds(quads, rate, stride):
+    """CLAS blocks are built in runs of records whose rounds hold what fits
+    LDS: one whole cluster alone, whole clusters (ragged ones among them)
+    beside parts of every size, mostly parts of up to 121 triangles.  Blocks,
+    sizes and padding equal the oracle byte for byte; vertex buffers with a
+    stride of 16 bytes give the same blocks."""
+    host = scene.scene_grid_instances(num_instances=1 if quads == 8 else 3, quads=quads, patch_size=6.0, tex_size=64,
+                                      tess_rate_pixels=rate)
+    cfg = harness.small_config()
+    of = harness.OracleFrame(host, cfg)
+    of.run(host.frame(), nthreads=8)
+    g = harness.GpuFrame(host, cfg)
+    try:
+        g.run(host.frame())
+        res = g.results()
+        if stride != 12:
+            # the same vertices spread to 16 bytes in a second buffer
+            import torch
+            nv = res.arrays["genVertices"].shape[0]
+            wide = torch.zeros(nv, 4, dtype=torch.float32, device="cuda")
+            wide[:, :3] = torch.from_numpy(res.arrays["genVertices"].copy()).cuda()
+            sb = g.r.scene_building()
+            n = sb.tempInstantiateCounter
+            ti = g.r.copy(sb.tempInstantiations, 32 * n).view(abi.TEMPLATE_INSTANTIATE_INFO).copy()
+            base = np.uint64(sb.genVertices)
+            ti["vertexBufferAddress"] = np.uint64(wide.data_ptr()) + (ti["vertexBufferAddress"] - base) // np.uint64(12) * np.uint64(16)
+            ti["vertexBufferStride"] = 16
+            torch.cuda.synchronize()
+            L = abi.lib()
+            abi.check(L.tc_memcpy(C.c_void_p(sb.tempInstantiations), ti.ctypes.data, ti.nbytes), "tc_memcpy")
+            abi.check(L.tc_clas_instantiate(C.byref(g.r.bindings), cfg, None), "tc_clas_instantiate")
+            again = g.results()
+            want, got = (x.arrays["clasBlocks"].view(np.uint32).copy() for x in (res, again))
+            # the header's vertexBase names a source outside genVertices
+            at = (res.arrays["tempClusterOffsets"].astype(np.int64) - int(res.arrays["tempClusterOffsets"][0])) // 4 + 8
+            want[at] = got[at] = 0
+            assert np.array_equal(want, got)
+            assert np.array_equal(res.arrays["tempClusterSizes"], again.arrays["tempClusterSizes"])
+    finally:
+        g.close()
+    harness.compare(res, of.results())

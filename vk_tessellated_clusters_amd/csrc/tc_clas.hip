@@ -96,193 +96,277 @@ __device__ __forceinline__ uint32_t vertex_base(const tc_scene_building* b, uint
   return vbuf >= b->genVertices ? (uint32_t)((vbuf - b->genVertices) / 12u) : 0xFFFFFFFFu;
 }
 
-// Templates of at most kSubTris triangles and kSubVerts vertices (the
-// tessellated parts and the whole clusters of up to 128 triangles) are
-// built by 16-lane subgroups, four per wave, each staging its block in a
-// quarter of the wave's LDS; larger ones by the whole wave.  Both paths
-// write the same bytes (box min / max are exact in any order).
-constexpr uint32_t kSub = 16;
-constexpr uint32_t kSubTris = 128;
-constexpr uint32_t kSubVerts = 128;
-constexpr uint32_t kSubsPerWave = kWave / kSub;
-constexpr uint32_t kWaveFloatsPerLane = (kMaxClusterVerts * 3 + kWave - 1) / kWave;
-constexpr uint32_t kWaveTrisPerLane = (kMaxClusterTris + kWave - 1) / kWave;
-constexpr uint32_t kSubFloatsPerLane = (kSubVerts * 3 + kSub - 1) / kSub;
-constexpr uint32_t kSubTrisPerLane = (kSubTris + kSub - 1) / kSub;
+// Sum over the lanes of this lane's row of 16 up to it (all lanes active).
+__device__ __forceinline__ uint32_t row_scan(uint32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);  // row_shr:8
+  return v;
+}
+
+// Value of the lane whose index differs in bit 0 / bit 1 (within four lanes).
+template <int CTRL>
+__device__ __forceinline__ float quad_swap(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
+
+// A wave builds a run of up to kBatch records in rounds.  A round takes as
+// many of them as fit its LDS (whole clusters of 81 vertices: three;
+// tessellated parts of a few triangles: all 16) and works flat over their
+// vertices, triangle words and groups, 64 at a time.  With 16 lanes to a
+// record the launch was bound by its instructions and their waits, not by
+// memory: a part of 7 triangles left most lanes idle in unrolled copies sized
+// for 128 triangles.  Now its stores bound it (of 791 us at the 3840 x 2160
+// patch field, 1.6 GB of blocks, 244 remain without them).  Measured: patch
+// field 1218 -> 791 us (2.9 TB/s), 500 meshes 139 -> 109 us, grid64 112 -> 73 us,
+// 8192 parts of 75 triangles 10 -> 9.5 us.  Rounds of 320 vertices and 512
+// triangles (four workgroups per CU instead of five) took 857, and prefetching
+// the next run's records 751 us there but 77 at grid64 and 112 at 500 meshes.
+constexpr uint32_t kBatch = 16;
+constexpr uint32_t kRoundVerts = 256;  // at least kMaxClusterVerts
+constexpr uint32_t kRoundTris = 384;
+constexpr uint32_t kRoundGroups = 96;
+constexpr uint32_t kMaxTemplateTris = 256;  // tc_cluster_template_order's limit
 constexpr uint32_t kClasWaves = 4;
+constexpr uint32_t kClasResident = 16;  // waves of a CU that a short frame's records are dealt over
+static_assert(kRoundVerts >= kMaxClusterVerts && kRoundTris >= kMaxTemplateTris &&
+                  kRoundGroups >= kMaxTemplateTris / TC_CLAS_GROUP_TRIANGLES,
+              "a record fits a round");
 
-__device__ __forceinline__ float sub_min(float v) {
-#pragma unroll
-  for (int d = 1; d < (int)kSub; d <<= 1) v = fminf(v, __shfl_xor(v, d, kWave));
-  return v;
-}
-__device__ __forceinline__ float sub_max(float v) {
-#pragma unroll
-  for (int d = 1; d < (int)kSub; d <<= 1) v = fmaxf(v, __shfl_xor(v, d, kWave));
-  return v;
+// A record of the round.  Addresses are those item 0 of the round would
+// have if the record began there, so item k of the round is at base + k *
+// size.
+struct ClasRecord {
+  uint64_t src;    // vertices in genVertices, `stride` bytes apart
+  uint64_t verts;  // vertices of the block
+  uint64_t words;  // template's triangle words
+  uint64_t tris;   // triangle words of the block
+  uint64_t boxes;  // group boxes of the block
+  uint32_t stride;
+  uint16_t firstVert, firstTri, firstGroup;  // in the round
+  uint16_t nt, ng;
+};
+
+struct ClasWave {
+  float v[kRoundVerts * 3];
+  uint32_t t[kRoundTris];
+  float box[kRoundGroups * 6];
+  ClasRecord rec[kBatch];
+  // per kind of item: a bit for every first item of a record, and the
+  // records that have items, in order
+  uint64_t headV[(kRoundVerts + 63) / 64], headT[(kRoundTris + 63) / 64], headG[(kRoundGroups + 63) / 64];
+  uint8_t listV[kBatch], listT[kBatch], listG[kBatch];
+};
+
+// The record that item 64 * j + lane of a kind belongs to; `before` counts
+// the first items in earlier words.
+__device__ __forceinline__ uint32_t item_record(const uint64_t* heads, const uint8_t* list, uint32_t j, uint32_t& before) {
+  const uint64_t h = uniform64(heads[j]);
+  const uint32_t k = before + (uint32_t)(h & 1) + mask_prefix(h >> 1) - 1;
+  before += __popcll(h);
+  return list[k & (kBatch - 1)];
 }
 
-// Each wave takes 4 consecutive records per step (one per subgroup),
-// grid-stride over tempInstantiateCounter.
-__global__ __launch_bounds__(kClasWaves * kWave) void k_clas_instantiate(KArgs a) {
-  // per wave: four subgroup quarters, or one whole-wave block (at most
-  // kMaxClusterVerts vertices and kMaxClusterTris triangles)
-  static_assert(kSubsPerWave * kSubVerts >= kMaxClusterVerts && kSubsPerWave * kSubTris >= kMaxClusterTris, "LDS per wave");
-  __shared__ float s_vall[kClasWaves][kSubsPerWave * kSubVerts * 3];
-  __shared__ uint32_t s_tall[kClasWaves][kSubsPerWave * kSubTris];
+__device__ __forceinline__ void mark_head(uint64_t* heads, uint32_t first) {
+  __hip_atomic_fetch_or(reinterpret_cast<uint32_t*>(heads) + (first >> 5), 1u << (first & 31), __ATOMIC_RELAXED,
+                        __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
+// Runs of records, grid-stride over tempInstantiateCounter; a frame with
+// fewer than kBatch records for each of the chip's resident waves takes
+// shorter runs (8192 records in runs of 1 on 40 waves a CU: 14 us, of 2 on 16
+// waves: 9.5 us).
+__global__ __launch_bounds__(kClasWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_clas_instantiate(KArgs a, uint32_t residentWaves) {
+  __shared__ ClasWave s_wave[kClasWaves];
   const tc_scene_building* b = a.build;
   const uint32_t n = min(b->tempInstantiateCounter, a.cfg.maxGeneratedClusters);
-  const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
-  const uint32_t sub = lane / kSub, sl = lane % kSub;
-  float* s_v = s_vall[wave];
-  uint32_t* s_t = s_tall[wave];
-  // a subgroup stages its small block in its quarter of the wave's LDS
-  float* s_sv = s_v + sub * (kSubVerts * 3);
-  uint32_t* s_st = s_t + sub * kSubTris;
+  const uint32_t lane = lane_id();
+  ClasWave& w = s_wave[threadIdx.x / kWave];
   const tc_template_instantiate_info* infos = ptr<const tc_template_instantiate_info>(b->tempInstantiations);
   const uint64_t* dsts = ptr<const uint64_t>(b->tempClusterAddresses);
   uint32_t* sizes = ptr<uint32_t>(b->tempClusterSizes);
-  const uint32_t perStep = kWave / kSub, stride = gridDim.x * kClasWaves * perStep;
-  // two-stage prefetch along the grid-stride loop: while a record is built,
-  // the next record's template (its info is already here) and the info of
-  // the record after it load, so a step waits on its vertex loads alone
-  // instead of the info -> template -> vertices chain
-  uint32_t base = (blockIdx.x * kClasWaves + wave) * perStep;
-  tc_template_instantiate_info info1{}, info2{};
-  tc_clas_template T1{};
-  if (base + sub < n) {
-    info1 = gld_record(infos + base + sub);
-    T1 = gld_record(ptr<const tc_clas_template>(info1.clusterTemplateAddress));
-  }
-  if (base + stride + sub < n) info2 = gld_record(infos + base + stride + sub);
-  for (; base < n; base += stride) {
-    const uint32_t i = base + sub;
-    const bool valid = i < n;
-    const tc_template_instantiate_info info = info1;
-    const tc_clas_template T = T1;
-    info1 = info2;
-    if (i + stride < n) T1 = gld_record(ptr<const tc_clas_template>(info1.clusterTemplateAddress));
-    if (i + 2 * stride < n) info2 = gld_record(infos + i + 2 * stride);
-    const bool small = valid && T.numTriangles <= kSubTris && T.numVertices <= kSubVerts;
-    const uint32_t nt = small ? T.numTriangles : 0u, nv = small ? T.numVertices : 0u;
+  const uint32_t waves = gridDim.x * kClasWaves;
+  const uint32_t run = min(kBatch, max(1u, (n + residentWaves - 1) / residentWaves));
+  for (uint32_t r0 = uniform(blockIdx.x * kClasWaves + threadIdx.x / kWave) * run; r0 < n; r0 += waves * run) {
+    const uint32_t cnt = min(run, n - r0);
+    // lanes 0 .. cnt - 1 hold the run's records
+    const bool held = lane < cnt;
+    uint64_t dst = 0, src = 0, words = 0;
+    uint32_t stride = 12, nv = 0, nt = 0, clusterID = 0;
+    if (held) {
+      const tc_template_instantiate_info info = gld_record(infos + r0 + lane);
+      dst = gld(dsts + r0 + lane);
+      const tc_clas_template T = gld_record(ptr<const tc_clas_template>(info.clusterTemplateAddress));
+      src = info.vertexBufferAddress;
+      stride = (uint32_t)info.vertexBufferStride;
+      words = T.triangles;
+      nv = min(T.numVertices, kMaxClusterVerts);
+      nt = min(T.numTriangles, kMaxTemplateTris);
+      clusterID = T.clusterID + info.clusterIdOffset;
+    }
     const uint32_t ng = (nt + TC_CLAS_GROUP_TRIANGLES - 1) / TC_CLAS_GROUP_TRIANGLES;
-    char* dst = small ? ptr<char>(gld(dsts + i)) : nullptr;
-    const char* src = small ? ptr<const char>(info.vertexBufferAddress) : nullptr;
-    if (small) {
-      uint32_t* tris = reinterpret_cast<uint32_t*>(dst + sizeof(tc_clas_header) + r16(ng * 24u));
-      float* verts = reinterpret_cast<float*>(dst + sizeof(tc_clas_header) + r16(ng * 24u) + r16(nt * 4u));
-      // every load of the block is issued before the first is used, so the
-      // copy waits for one round trip rather than one per element; packed
-      // vertices (stride 12, what the instantiation records carry) are read
-      // from one base, other strides element by element
-      const uint32_t nf = nv * 3;
-      if (info.vertexBufferStride == 12u) {
-        const float* vs = reinterpret_cast<const float*>(src) + sl;
-        float vf[kSubFloatsPerLane];
-#pragma unroll
-        for (uint32_t j = 0; j < kSubFloatsPerLane; j++) vf[j] = sl + j * kSub < nf ? gld(vs + j * kSub) : 0.0f;
-#pragma unroll
-        for (uint32_t j = 0; j < kSubFloatsPerLane; j++) {
-          const uint32_t k = sl + j * kSub;
-          if (k < nf) s_sv[k] = vf[j], gst(verts + k, vf[j]);
-        }
-      } else {
-        for (uint32_t k = sl; k < nf; k += kSub) {
-          const uint32_t v = k / 3, c = k - v * 3;
-          const float f = gld(reinterpret_cast<const float*>(src + (uint64_t)v * info.vertexBufferStride) + c);
-          s_sv[k] = f;
-          gst(verts + k, f);
-        }
-      }
-      const uint32_t* ts = ptr<const uint32_t>(T.triangles) + sl;
-      uint32_t tw[kSubTrisPerLane];
-#pragma unroll
-      for (uint32_t j = 0; j < kSubTrisPerLane; j++) tw[j] = sl + j * kSub < nt ? gld(ts + j * kSub) : 0u;
-#pragma unroll
-      for (uint32_t j = 0; j < kSubTrisPerLane; j++) {
-        const uint32_t t = sl + j * kSub;
-        if (t < nt) s_st[t] = tw[j], gst(tris + t, tw[j]);
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (uint32_t g = sl; small && g < ng; g += kSub) {
-      float glo[3] = {INFINITY, INFINITY, INFINITY}, ghi[3] = {-INFINITY, -INFINITY, -INFINITY};
-      const uint32_t t1 = min(nt, (g + 1) * TC_CLAS_GROUP_TRIANGLES);
-      for (uint32_t t = g * TC_CLAS_GROUP_TRIANGLES; t < t1; t++) {
-        const uint32_t w = s_st[t];
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-          const uint32_t vi = (w >> (8 * k)) & 0xFF;
-#pragma unroll
-          for (int c = 0; c < 3; c++) glo[c] = fminf(glo[c], s_sv[vi * 3 + c]), ghi[c] = fmaxf(ghi[c], s_sv[vi * 3 + c]);
+    const uint32_t oT = (uint32_t)sizeof(tc_clas_header) + r16(ng * 24u), oV = oT + r16(nt * 4u), size = oV + r16(nv * 12u);
+    for (uint32_t done = 0; done < cnt;) {
+      // the records of this round: done .. done + k - 1
+      const bool left = held && lane >= done;
+      const uint32_t ev = row_scan(left ? nv : 0u), et = row_scan(left ? nt : 0u), eg = row_scan(left ? ng : 0u);
+      const uint64_t fit = ballot(left && ev <= kRoundVerts && et <= kRoundTris && eg <= kRoundGroups);
+      const uint32_t k = __popcll(fit), lastLane = done + k - 1;
+      const uint32_t numV = __builtin_amdgcn_readlane(ev, lastLane), numT = __builtin_amdgcn_readlane(et, lastLane),
+                     numG = __builtin_amdgcn_readlane(eg, lastLane);
+      const bool in = left && lane < done + k;
+      constexpr uint32_t kHeads = (kRoundVerts + 63) / 64 + (kRoundTris + 63) / 64 + (kRoundGroups + 63) / 64;
+      if (lane < kHeads) w.headV[lane] = 0;  // headV, headT and headG in a row
+      wave_sync();
+      {
+        const uint64_t mv = ballot(in && nv), mt = ballot(in && nt);
+        const uint32_t fv = ev - nv, ft = et - nt, fg = eg - ng;
+        if (in) {
+          ClasRecord& r = w.rec[lane];
+          r.src = src - (uint64_t)fv * stride;
+          r.verts = dst + oV - 12ull * fv;
+          r.words = words - 4ull * ft;
+          r.tris = dst + oT - 4ull * ft;
+          r.boxes = dst + sizeof(tc_clas_header) - 24ull * fg;
+          r.stride = stride;
+          r.firstVert = (uint16_t)fv, r.firstTri = (uint16_t)ft, r.firstGroup = (uint16_t)fg;
+          r.nt = (uint16_t)nt, r.ng = (uint16_t)ng;
+          if (nv) w.listV[mask_prefix(mv)] = (uint8_t)lane, mark_head(w.headV, fv);
+          if (nt) {
+            w.listT[mask_prefix(mt)] = (uint8_t)lane, mark_head(w.headT, ft);
+            w.listG[mask_prefix(mt)] = (uint8_t)lane, mark_head(w.headG, fg);
+          }
         }
       }
-      tc_aabb box;
+      wave_sync();
+      // vertices and triangle words: every load of the round, then LDS, then
+      // the block.  Lanes past the end repeat the last item (into LDS that
+      // nobody reads), so that no branch lies between the loads, and stores
+      // start when no load is outstanding: either would make a load wait for
+      // the one before it, or for stores.
+      float vx[kRoundVerts / 64][3];
+      uint32_t tw[kRoundTris / 64];
+      uint32_t vq[kRoundVerts / 64], tq[kRoundTris / 64];
+      uint32_t before = 0;
+      if (numV != 0 && numT != 0) {
 #pragma unroll
-      for (int c = 0; c < 3; c++) box.lo[c] = glo[c], box.hi[c] = ghi[c], lo[c] = fminf(lo[c], glo[c]), hi[c] = fmaxf(hi[c], ghi[c]);
-      gst_record(reinterpret_cast<tc_aabb*>(dst + sizeof(tc_clas_header)) + g, box);
-    }
+        for (uint32_t j = 0; j < kRoundVerts / 64; j++) {
+          vq[j] = item_record(w.headV, w.listV, j, before);
+          const ClasRecord& r = w.rec[vq[j]];
+          const gfloat3 f = gld3(ptr<const float>(r.src + (uint64_t)min(64 * j + lane, numV - 1) * r.stride));
+          vx[j][0] = f.x, vx[j][1] = f.y, vx[j][2] = f.z;
+        }
+        before = 0;
 #pragma unroll
-    for (int c = 0; c < 3; c++) lo[c] = sub_min(lo[c]), hi[c] = sub_max(hi[c]);
-    if (small) {
-      // zero the 16-byte padding after each part
-      uint32_t* w32 = reinterpret_cast<uint32_t*>(dst);
-      const uint32_t g0 = (uint32_t)sizeof(tc_clas_header) + ng * 24u, g1 = (uint32_t)sizeof(tc_clas_header) + r16(ng * 24u);
-      const uint32_t t0 = g1 + nt * 4u, t1 = g1 + r16(nt * 4u), v0 = t1 + nv * 12u, v1 = t1 + r16(nv * 12u);
-      const uint32_t na = (g1 - g0) / 4, nb = na + (t1 - t0) / 4, nc = nb + (v1 - v0) / 4;
-      for (uint32_t q = sl; q < nc; q += kSub)
-        gst(w32 + (q < na ? g0 + 4 * q : (q < nb ? t0 + 4 * (q - na) : v0 + 4 * (q - nb))) / 4, 0u);
-      if (sl == 0) {
-        tc_clas_header h;
-        h.lo[0] = lo[0], h.lo[1] = lo[1], h.lo[2] = lo[2];
-        h.hi[0] = hi[0], h.hi[1] = hi[1], h.hi[2] = hi[2];
-        h.clusterID = T.clusterID + info.clusterIdOffset;
-        h.counts = nt | (nv << 8) | (ng << 16);
-        h.vertexBase = vertex_base(b, info.vertexBufferAddress);
-        h._pad[0] = h._pad[1] = h._pad[2] = 0;
-        gst_record(reinterpret_cast<tc_clas_header*>(dst), h);
-        gst(sizes + i, (uint32_t)sizeof(tc_clas_header) + r16(ng * 24u) + r16(nt * 4u) + r16(nv * 12u));
+        for (uint32_t j = 0; j < kRoundTris / 64; j++) {
+          tq[j] = item_record(w.headT, w.listT, j, before);
+          tw[j] = gld(ptr<const uint32_t>(w.rec[tq[j]].words) + min(64 * j + lane, numT - 1));
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kRoundVerts / 64; j++) {
+          float* l = w.v + 3 * (64 * j + lane);
+          l[0] = vx[j][0], l[1] = vx[j][1], l[2] = vx[j][2];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kRoundTris / 64; j++) w.t[64 * j + lane] = tw[j];
+        wave_sync();
+#pragma unroll
+        for (uint32_t j = 0; j < kRoundVerts / 64; j++) {
+          const uint32_t i = 64 * j + lane;
+          if (i < numV) {
+            float* g = ptr<float>(w.rec[vq[j]].verts) + 3 * i;
+            gst(g, vx[j][0]), gst(g + 1, vx[j][1]), gst(g + 2, vx[j][2]);
+          }
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kRoundTris / 64; j++) {
+          const uint32_t i = 64 * j + lane;
+          if (i < numT) gst(ptr<uint32_t>(w.rec[tq[j]].tris) + i, tw[j]);
+        }
       }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    // large templates: the whole wave, one at a time
-    uint64_t big = ballot(valid && !small && sl == 0);
-    while (big) {
-      const uint32_t ij = base + (uint32_t)__builtin_ctzll(big) / kSub;
-      big &= big - 1;
-      const tc_template_instantiate_info bi = gld_record(infos + ij);
-      const tc_clas_template BT = gld_record(ptr<const tc_clas_template>(bi.clusterTemplateAddress));
-      const uint32_t bnt = BT.numTriangles, bnv = BT.numVertices, bng = BT.numGroups;
-      char* bdst = ptr<char>(gld(dsts + ij));
-      uint32_t* tris = reinterpret_cast<uint32_t*>(bdst + sizeof(tc_clas_header) + r16(bng * 24u));
-      float* verts = reinterpret_cast<float*>(bdst + sizeof(tc_clas_header) + r16(bng * 24u) + r16(bnt * 4u));
-      const char* bsrc = ptr<const char>(bi.vertexBufferAddress);
-      for (uint32_t k = lane; k < bnv * 3; k += kWave) {
-        const uint32_t v = k / 3, c = k - v * 3;
-        const float f = gld(reinterpret_cast<const float*>(bsrc + (uint64_t)v * bi.vertexBufferStride) + c);
-        s_v[k] = f;
-        gst(verts + k, f);
+      wave_sync();
+      // group boxes
+      before = 0;
+#pragma unroll
+      for (uint32_t j = 0; j < (kRoundGroups + 63) / 64; j++) {
+        if (64 * j >= numG) continue;
+        const uint32_t i = 64 * j + lane, q = item_record(w.headG, w.listG, j, before);
+        if (i < numG) {
+          const ClasRecord& r = w.rec[q];
+          const uint32_t t0 = (i - r.firstGroup) * TC_CLAS_GROUP_TRIANGLES, tEnd = r.nt - 1;
+          const uint32_t* t = w.t + r.firstTri;
+          const float* v = w.v + 3 * r.firstVert;
+          float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+          for (uint32_t m = 0; m < TC_CLAS_GROUP_TRIANGLES; m++) {
+            const uint32_t word = t[min(t0 + m, tEnd)];  // the last one again past the end
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+              const float* p = v + 3 * ((word >> (8 * c)) & 0xFF);
+#pragma unroll
+              for (int x = 0; x < 3; x++) lo[x] = fminf(lo[x], p[x]), hi[x] = fmaxf(hi[x], p[x]);
+            }
+          }
+          tc_aabb box;
+#pragma unroll
+          for (int x = 0; x < 3; x++) {
+            box.lo[x] = w.box[6 * i + x] = lo[x];
+            box.hi[x] = w.box[6 * i + 3 + x] = hi[x];
+          }
+          gst_record(ptr<tc_aabb>(r.boxes) + i, box);
+        }
       }
-      for (uint32_t t = lane; t < bnt; t += kWave) {
-        const uint32_t w = gld(ptr<const uint32_t>(BT.triangles) + t);
-        s_t[t] = w;
-        gst(tris + t, w);
+      wave_sync();
+      // headers, four lanes to a record, and the zeros after each part
+      {
+        const uint32_t q = lane >> 2, sl = lane & 3;
+        const bool mine = q >= done && q < done + k;
+        float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+        if (mine) {
+          const ClasRecord& r = w.rec[q];
+          for (uint32_t g = sl; g < r.ng; g += 4) {
+            const float* bx = w.box + 6 * (r.firstGroup + g);
+#pragma unroll
+            for (int x = 0; x < 3; x++) lo[x] = fminf(lo[x], bx[x]), hi[x] = fmaxf(hi[x], bx[3 + x]);
+          }
+        }
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+          lo[x] = fminf(lo[x], quad_swap<kSwap1>(lo[x])), hi[x] = fmaxf(hi[x], quad_swap<kSwap1>(hi[x]));
+          lo[x] = fminf(lo[x], quad_swap<kSwap2>(lo[x])), hi[x] = fmaxf(hi[x], quad_swap<kSwap2>(hi[x]));
+        }
+        const uint64_t rdst = shfl64(dst, q), rsrc = shfl64(src, q);
+        const uint32_t rnt = shfl(nt, q), rnv = shfl(nv, q), rng = shfl(ng, q), rid = shfl(clusterID, q);
+        const uint32_t roT = shfl(oT, q), roV = shfl(oV, q), rsize = shfl(size, q);
+        if (mine) {
+          const uint32_t g0 = (uint32_t)sizeof(tc_clas_header) + rng * 24u, t0 = roT + rnt * 4u, v0 = roV + rnv * 12u;
+          char* base = ptr<char>(rdst);
+          if (g0 + 4 * sl < roT) gst(reinterpret_cast<uint32_t*>(base + g0 + 4 * sl), 0u);
+          if (t0 + 4 * sl < roV) gst(reinterpret_cast<uint32_t*>(base + t0 + 4 * sl), 0u);
+          if (v0 + 4 * sl < rsize) gst(reinterpret_cast<uint32_t*>(base + v0 + 4 * sl), 0u);
+          if (sl == 0) {
+            tc_clas_header h;
+            h.lo[0] = lo[0], h.lo[1] = lo[1], h.lo[2] = lo[2];
+            h.hi[0] = hi[0], h.hi[1] = hi[1], h.hi[2] = hi[2];
+            h.clusterID = rid;
+            h.counts = rnt | (rnv << 8) | (rng << 16);
+            h.vertexBase = vertex_base(b, rsrc);
+            h._pad[0] = h._pad[1] = h._pad[2] = 0;
+            gst_record(reinterpret_cast<tc_clas_header*>(base), h);
+            gst(sizes + r0 + q, rsize);
+          }
+        }
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const uint32_t size = finish_block(bdst, s_v, s_t, bnt, bnv, BT.clusterID + bi.clusterIdOffset,
-                                         vertex_base(b, bi.vertexBufferAddress));
-      if (lane == 0) gst(sizes + ij, size);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
+      done += k;
     }
   }
 }
+
+constexpr uint32_t kWaveFloatsPerLane = (kMaxClusterVerts * 3 + kWave - 1) / kWave;
+constexpr uint32_t kWaveTrisPerLane = (kMaxClusterTris + kWave - 1) / kWave;
 
 // Transient builds (stands for the NV transient CLAS build,
 // renderer_raytrace_clusters_tess.cpp:625-655): triangles in record order
@@ -364,7 +448,8 @@ extern "C" tc_status tc_clas_instantiate(const tc_bindings* b, tc_config config,
   const uint32_t waves = std::min<uint32_t>((config.maxGeneratedClusters + 3) / 4,
                                             (uint32_t)num_cu_public() * tuning_snapshot().clasWavesPerCU);
   const uint32_t grid = (waves + kClasWaves - 1) / kClasWaves;
-  hipLaunchKernelGGL(k_clas_instantiate, dim3(grid), dim3(kClasWaves * kWave), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(k_clas_instantiate, dim3(grid), dim3(kClasWaves * kWave), 0, (hipStream_t)stream, a,
+                     (uint32_t)num_cu_public() * kClasResident);
   return hipGetLastError() == hipSuccess ? TC_OK : TC_ERROR_LAUNCH;
 }
 

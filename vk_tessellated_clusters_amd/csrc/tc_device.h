@@ -109,6 +109,12 @@ __device__ __forceinline__ void gst_record(T* p, const T& v) {
   for (uint32_t i = 0; i < sizeof(T) / 4; i++) gst(d + i, s[i]);
 }
 
+// Three floats at any 4-byte boundary in one load.
+typedef float gfloat3 __attribute__((ext_vector_type(3), aligned(4)));
+__device__ __forceinline__ gfloat3 gld3(const float* p) {
+  return *(const __attribute__((address_space(1))) gfloat3*)p;
+}
+
 __device__ __forceinline__ v3 ld3(uint64_t base, uint32_t i) {
   const float* f = ptr<const float>(base) + 3ull * i;
   return mk(gld(f), gld(f + 1), gld(f + 2));
@@ -500,6 +506,14 @@ __device__ __forceinline__ uint32_t shfl(uint32_t v, uint32_t src) { return (uin
 __device__ __forceinline__ uint64_t shfl64(uint64_t v, uint32_t src) {
   uint32_t lo = shfl((uint32_t)v, src), hi = shfl((uint32_t)(v >> 32), src);
   return ((uint64_t)hi << 32) | lo;
+}
+
+// Orders LDS accesses of one wave's lanes (the hardware runs a wave's LDS
+// operations in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // inclusive wave scan (Hillis-Steele over 64 lanes)

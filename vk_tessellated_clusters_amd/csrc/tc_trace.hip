@@ -400,12 +400,6 @@ struct WaveLds {
   uint16_t queue[kLeafQueue];  // groups entered: lane | group << 6
 };
 
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Inclusive sum over the wave's lanes (all active).
 __device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1
@@ -439,11 +433,6 @@ __device__ __forceinline__ bool key_less(float t, uint32_t i, uint32_t c, uint32
   if (i != best.instanceID) return i < best.instanceID;
   if (c != best.clusterID) return c < best.clusterID;
   return p < best.primitiveID;
-}
-
-typedef float gfloat3 __attribute__((ext_vector_type(3), aligned(4)));
-__device__ __forceinline__ gfloat3 gload3(const float* p) {
-  return *(const __attribute__((address_space(1))) gfloat3*)p;
 }
 
 // Intersects the CLAS blocks that the wave's lanes hold (`has`), sharing the
@@ -568,8 +557,8 @@ __device__ __forceinline__ void leaf_step(WaveLds& w, bool has, const char* clas
                              ((bng * 24u + 15u) & ~15u);
           word = gload(reinterpret_cast<const uint32_t*>(tris) + tri);
           const float* verts = reinterpret_cast<const float*>(tris + ((bnt * 4u + 15u) & ~15u));
-          const gfloat3 p0 = gload3(verts + 3 * (word & 0xFF)), p1 = gload3(verts + 3 * ((word >> 8) & 0xFF)),
-                        p2 = gload3(verts + 3 * ((word >> 16) & 0xFF));
+          const gfloat3 p0 = gld3(verts + 3 * (word & 0xFF)), p1 = gld3(verts + 3 * ((word >> 8) & 0xFF)),
+                        p2 = gld3(verts + 3 * ((word >> 16) & 0xFF));
           const float4 ro = w.rayO[who];
           WoopRay tr;
           tr.o[0] = ro.x, tr.o[1] = ro.y, tr.o[2] = ro.z;
