@@ -8,6 +8,8 @@
 //   tc_clas_header | group boxes | triangle words | vertices
 // and tempClusterSizes[i] receives its size.  Transient build records
 // (ClasBuildInfo, 1X clusters) produce the same block format.
+#include <stddef.h>
+
 #include <algorithm>
 
 #include "tc_kernels.h"
@@ -114,65 +116,59 @@ constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
 
 // A wave builds a run of up to kBatch records in rounds.  A round takes as
 // many of them as fit its LDS (whole clusters of 81 vertices: three;
-// tessellated parts of a few triangles: all 16) and works flat over their
+// tessellated parts of a few triangles: about 14) and works flat over their
 // vertices, triangle words and groups, 64 at a time.  With 16 lanes to a
 // record the launch was bound by its instructions and their waits, not by
 // memory: a part of 7 triangles left most lanes idle in unrolled copies sized
-// for 128 triangles.  Now its stores bound it (of 791 us at the 3840 x 2160
-// patch field, 1.6 GB of blocks, 244 remain without them).  Measured: patch
-// field 1218 -> 791 us (2.9 TB/s), 500 meshes 139 -> 109 us, grid64 112 -> 73 us,
-// 8192 parts of 75 triangles 10 -> 9.5 us.  Rounds of 320 vertices and 512
-// triangles (four workgroups per CU instead of five) took 857, and prefetching
-// the next run's records 751 us there but 77 at grid64 and 112 at 500 meshes.
+// for 128 triangles.  The blocks are put together in LDS and leave in 16-byte
+// stores, 1 KB a step: written piece by piece, the stores took 550 of 791 us
+// at the 3840 x 2160 patch field (1.6 GB of blocks).  Measured: patch field
+// 1218 -> 610 us (3.9 TB/s), 500 meshes 139 -> 107 us, grid64 112 -> 73 us, 8192
+// parts of 75 triangles 10 -> 9.2 us.  VALU is then 57 % busy.  Prefetching the
+// next run's records gained 5 % at the patch field and lost as much at grid64;
+// five waves per SIMD instead of four measured no difference.
 constexpr uint32_t kBatch = 16;
 constexpr uint32_t kRoundVerts = 256;  // at least kMaxClusterVerts
 constexpr uint32_t kRoundTris = 384;
-constexpr uint32_t kRoundGroups = 96;
+constexpr uint32_t kRoundGroups = 128;
+constexpr uint32_t kRoundBytes = 7168;      // blocks of the round
 constexpr uint32_t kMaxTemplateTris = 256;  // tc_cluster_template_order's limit
 constexpr uint32_t kClasWaves = 4;
 constexpr uint32_t kClasResident = 16;  // waves of a CU that a short frame's records are dealt over
 static_assert(kRoundVerts >= kMaxClusterVerts && kRoundTris >= kMaxTemplateTris &&
-                  kRoundGroups >= kMaxTemplateTris / TC_CLAS_GROUP_TRIANGLES,
+                  kRoundGroups >= kMaxTemplateTris / TC_CLAS_GROUP_TRIANGLES &&
+                  kRoundBytes >= sizeof(tc_clas_header) + kMaxTemplateTris * 10 + kMaxClusterVerts * 12 + 48,
               "a record fits a round");
 
-// A record of the round.  Addresses are those item 0 of the round would
-// have if the record began there, so item k of the round is at base + k *
-// size.
-struct ClasRecord {
-  uint64_t src;    // vertices in genVertices, `stride` bytes apart
-  uint64_t verts;  // vertices of the block
-  uint64_t words;  // template's triangle words
-  uint64_t tris;   // triangle words of the block
-  uint64_t boxes;  // group boxes of the block
-  uint32_t stride;
-  uint16_t firstVert, firstTri, firstGroup;  // in the round
-  uint16_t nt, ng;
-};
-
 struct ClasWave {
-  float v[kRoundVerts * 3];
-  uint32_t t[kRoundTris];
-  float box[kRoundGroups * 6];
-  ClasRecord rec[kBatch];
-  // per kind of item: a bit for every first item of a record, and the
-  // records that have items, in order
-  uint64_t headV[(kRoundVerts + 63) / 64], headT[(kRoundTris + 63) / 64], headG[(kRoundGroups + 63) / 64];
-  uint8_t listV[kBatch], listT[kBatch], listG[kBatch];
+  // the round's blocks as they go to memory, one after another; in words and
+  // in the 16-byte chunks they are written by
+  union {
+    uint32_t u[kRoundBytes / 4];
+    float f[kRoundBytes / 4];
+    uint4 chunk[kRoundBytes / 16];
+  };
+  // the round's records, one 16-byte read per kind of item.  Addresses and
+  // offsets are those that item 0 of the round would have if the record began
+  // with it (modulo 2^64 and 2^16), so item i lies at base + i * its size.
+  uint4 vert[kBatch];   // source address, stride, word offset of the vertices
+  uint4 tri[kBatch];    // template words' address, word offset of the triangles
+  uint4 group[kBatch];  // first group | triangles << 16, word offsets: triangles | vertices << 16, boxes,
+                        // groups | vertices << 16
+  uint4 block[kBatch];  // block address, cluster ID, counts
+  uint2 head[kBatch];   // vertexBase, first chunk | chunks << 16
+  // a bit for every first item of a record: vertices, triangles, groups, chunks
+  uint64_t heads[kRoundVerts / 64 + kRoundTris / 64 + kRoundGroups / 64 + kRoundBytes / 16 / 64];
 };
-
-// The record that item 64 * j + lane of a kind belongs to; `before` counts
-// the first items in earlier words.
-__device__ __forceinline__ uint32_t item_record(const uint64_t* heads, const uint8_t* list, uint32_t j, uint32_t& before) {
-  const uint64_t h = uniform64(heads[j]);
-  const uint32_t k = before + (uint32_t)(h & 1) + mask_prefix(h >> 1) - 1;
-  before += __popcll(h);
-  return list[k & (kBatch - 1)];
-}
+constexpr uint32_t kHeadT = kRoundVerts / 64, kHeadG = kHeadT + kRoundTris / 64, kHeadC = kHeadG + kRoundGroups / 64,
+                   kHeads = kHeadC + kRoundBytes / 16 / 64;
 
 __device__ __forceinline__ void mark_head(uint64_t* heads, uint32_t first) {
   __hip_atomic_fetch_or(reinterpret_cast<uint32_t*>(heads) + (first >> 5), 1u << (first & 31), __ATOMIC_RELAXED,
                         __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
+
+__device__ __forceinline__ uint64_t u64(uint32_t lo, uint32_t hi) { return ((uint64_t)hi << 32) | lo; }
 
 // Runs of records, grid-stride over tempInstantiateCounter; a frame with
 // fewer than kBatch records for each of the chip's resident waves takes
@@ -208,114 +204,106 @@ __global__ __launch_bounds__(kClasWaves * kWave) __attribute__((amdgpu_waves_per
     }
     const uint32_t ng = (nt + TC_CLAS_GROUP_TRIANGLES - 1) / TC_CLAS_GROUP_TRIANGLES;
     const uint32_t oT = (uint32_t)sizeof(tc_clas_header) + r16(ng * 24u), oV = oT + r16(nt * 4u), size = oV + r16(nv * 12u);
+    // a record without vertices or triangles takes a round of its own, so
+    // that a round's first items are its records
+    const bool empty = ballot(held && (nv == 0 || nt == 0)) != 0;
     for (uint32_t done = 0; done < cnt;) {
       // the records of this round: done .. done + k - 1
-      const bool left = held && lane >= done;
-      const uint32_t ev = row_scan(left ? nv : 0u), et = row_scan(left ? nt : 0u), eg = row_scan(left ? ng : 0u);
-      const uint64_t fit = ballot(left && ev <= kRoundVerts && et <= kRoundTris && eg <= kRoundGroups);
+      const bool left = held && lane >= done && !(empty && lane > done);
+      const uint32_t ev = row_scan(left ? nv : 0u), et = row_scan(left ? nt : 0u), eg = row_scan(left ? ng : 0u),
+                     es = row_scan(left ? size : 0u);
+      const uint64_t fit = ballot(left && ev <= kRoundVerts && et <= kRoundTris && eg <= kRoundGroups && es <= kRoundBytes);
       const uint32_t k = __popcll(fit), lastLane = done + k - 1;
       const uint32_t numV = __builtin_amdgcn_readlane(ev, lastLane), numT = __builtin_amdgcn_readlane(et, lastLane),
-                     numG = __builtin_amdgcn_readlane(eg, lastLane);
+                     numG = __builtin_amdgcn_readlane(eg, lastLane), numC = __builtin_amdgcn_readlane(es, lastLane) / 16;
       const bool in = left && lane < done + k;
-      constexpr uint32_t kHeads = (kRoundVerts + 63) / 64 + (kRoundTris + 63) / 64 + (kRoundGroups + 63) / 64;
-      if (lane < kHeads) w.headV[lane] = 0;  // headV, headT and headG in a row
+      if (lane < kHeads) w.heads[lane] = 0;
       wave_sync();
-      {
-        const uint64_t mv = ballot(in && nv), mt = ballot(in && nt);
-        const uint32_t fv = ev - nv, ft = et - nt, fg = eg - ng;
-        if (in) {
-          ClasRecord& r = w.rec[lane];
-          r.src = src - (uint64_t)fv * stride;
-          r.verts = dst + oV - 12ull * fv;
-          r.words = words - 4ull * ft;
-          r.tris = dst + oT - 4ull * ft;
-          r.boxes = dst + sizeof(tc_clas_header) - 24ull * fg;
-          r.stride = stride;
-          r.firstVert = (uint16_t)fv, r.firstTri = (uint16_t)ft, r.firstGroup = (uint16_t)fg;
-          r.nt = (uint16_t)nt, r.ng = (uint16_t)ng;
-          if (nv) w.listV[mask_prefix(mv)] = (uint8_t)lane, mark_head(w.headV, fv);
-          if (nt) {
-            w.listT[mask_prefix(mt)] = (uint8_t)lane, mark_head(w.headT, ft);
-            w.listG[mask_prefix(mt)] = (uint8_t)lane, mark_head(w.headG, fg);
-          }
-        }
+      if (in) {
+        const uint32_t fv = ev - nv, ft = et - nt, fg = eg - ng, fs = es - size;
+        const uint64_t sa = src - (uint64_t)fv * stride, wa = words - 4ull * ft, da = dst - fs;
+        const uint32_t bT = (fs + oT) / 4, bV = (fs + oV) / 4, bG = (fs + (uint32_t)sizeof(tc_clas_header)) / 4;
+        w.vert[lane] = make_uint4((uint32_t)sa, (uint32_t)(sa >> 32), stride, bV - 3 * fv);
+        w.tri[lane] = make_uint4((uint32_t)wa, (uint32_t)(wa >> 32), bT - ft, 0u);
+        w.group[lane] = make_uint4(fg | nt << 16, bT | bV << 16, bG, ng | nv << 16);
+        w.block[lane] = make_uint4((uint32_t)da, (uint32_t)(da >> 32), clusterID, nt | (nv << 8) | (ng << 16));
+        w.head[lane] = make_uint2(vertex_base(b, src), fs / 16 | (size / 16) << 16);
+        mark_head(w.heads, fv);
+        mark_head(w.heads + kHeadT, ft);
+        mark_head(w.heads + kHeadG, fg);
+        mark_head(w.heads + kHeadC, fs / 16);
       }
       wave_sync();
-      // vertices and triangle words: every load of the round, then LDS, then
-      // the block.  Lanes past the end repeat the last item (into LDS that
-      // nobody reads), so that no branch lies between the loads, and stores
-      // start when no load is outstanding: either would make a load wait for
-      // the one before it, or for stores.
-      float vx[kRoundVerts / 64][3];
-      uint32_t tw[kRoundTris / 64];
-      uint32_t vq[kRoundVerts / 64], tq[kRoundTris / 64];
-      uint32_t before = 0;
+      // word j of the heads in lane j; the record of item 64 * j + lane of a
+      // kind, `before` counting the first items in earlier words
+      const uint64_t headWord = lane < kHeads ? w.heads[lane] : 0ull;
+      auto record = [&](uint32_t word, uint32_t& before) {
+        const uint64_t h = u64(__builtin_amdgcn_readlane((uint32_t)headWord, word),
+                               __builtin_amdgcn_readlane((uint32_t)(headWord >> 32), word));
+        const uint32_t q = before + (uint32_t)(h & 1) + mask_prefix(h >> 1) - 1;
+        before += __popcll(h);
+        return q & (kBatch - 1);
+      };
+      // vertices and triangle words: every load of the round, then the image.
+      // Lanes past the end repeat the last item, so that no branch lies
+      // between the loads (one would make a load wait for the one before).
       if (numV != 0 && numT != 0) {
+        float vx[kRoundVerts / 64][3];
+        uint32_t tw[kRoundTris / 64], va[kRoundVerts / 64], ta[kRoundTris / 64];
+        uint32_t before = done;
 #pragma unroll
         for (uint32_t j = 0; j < kRoundVerts / 64; j++) {
-          vq[j] = item_record(w.headV, w.listV, j, before);
-          const ClasRecord& r = w.rec[vq[j]];
-          const gfloat3 f = gld3(ptr<const float>(r.src + (uint64_t)min(64 * j + lane, numV - 1) * r.stride));
+          const uint4 r = w.vert[record(j, before)];
+          const uint32_t i = min(64 * j + lane, numV - 1);
+          const gfloat3 f = gld3(ptr<const float>(u64(r.x, r.y) + (uint64_t)i * r.z));
           vx[j][0] = f.x, vx[j][1] = f.y, vx[j][2] = f.z;
+          va[j] = r.w + 3 * i;
         }
-        before = 0;
+        before = done;
 #pragma unroll
         for (uint32_t j = 0; j < kRoundTris / 64; j++) {
-          tq[j] = item_record(w.headT, w.listT, j, before);
-          tw[j] = gld(ptr<const uint32_t>(w.rec[tq[j]].words) + min(64 * j + lane, numT - 1));
+          const uint4 r = w.tri[record(kHeadT + j, before)];
+          const uint32_t i = min(64 * j + lane, numT - 1);
+          tw[j] = gld(ptr<const uint32_t>(u64(r.x, r.y)) + i);
+          ta[j] = r.z + i;
         }
 #pragma unroll
-        for (uint32_t j = 0; j < kRoundVerts / 64; j++) {
-          float* l = w.v + 3 * (64 * j + lane);
-          l[0] = vx[j][0], l[1] = vx[j][1], l[2] = vx[j][2];
-        }
+        for (uint32_t j = 0; j < kRoundVerts / 64; j++)
+          w.f[va[j]] = vx[j][0], w.f[va[j] + 1] = vx[j][1], w.f[va[j] + 2] = vx[j][2];
 #pragma unroll
-        for (uint32_t j = 0; j < kRoundTris / 64; j++) w.t[64 * j + lane] = tw[j];
-        wave_sync();
-#pragma unroll
-        for (uint32_t j = 0; j < kRoundVerts / 64; j++) {
-          const uint32_t i = 64 * j + lane;
-          if (i < numV) {
-            float* g = ptr<float>(w.rec[vq[j]].verts) + 3 * i;
-            gst(g, vx[j][0]), gst(g + 1, vx[j][1]), gst(g + 2, vx[j][2]);
-          }
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < kRoundTris / 64; j++) {
-          const uint32_t i = 64 * j + lane;
-          if (i < numT) gst(ptr<uint32_t>(w.rec[tq[j]].tris) + i, tw[j]);
-        }
+        for (uint32_t j = 0; j < kRoundTris / 64; j++) w.u[ta[j]] = tw[j];
       }
       wave_sync();
       // group boxes
-      before = 0;
+      {
+        uint32_t before = done;
 #pragma unroll
-      for (uint32_t j = 0; j < (kRoundGroups + 63) / 64; j++) {
-        if (64 * j >= numG) continue;
-        const uint32_t i = 64 * j + lane, q = item_record(w.headG, w.listG, j, before);
-        if (i < numG) {
-          const ClasRecord& r = w.rec[q];
-          const uint32_t t0 = (i - r.firstGroup) * TC_CLAS_GROUP_TRIANGLES, tEnd = r.nt - 1;
-          const uint32_t* t = w.t + r.firstTri;
-          const float* v = w.v + 3 * r.firstVert;
-          float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+        for (uint32_t j = 0; j < kRoundGroups / 64; j++) {
+          if (64 * j >= numG) continue;
+          const uint32_t i = 64 * j + lane, q = record(kHeadG + j, before);
+          if (i < numG) {
+            const uint4 r = w.group[q];
+            const uint32_t g = i - (r.x & 0xFFFF), t0 = g * TC_CLAS_GROUP_TRIANGLES, rnt = r.x >> 16;
+            const uint4 w4 = *reinterpret_cast<const uint4*>(w.u + (r.y & 0xFFFF) + t0);
+            // past the last triangle the one before again
+            uint32_t word[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
-          for (uint32_t m = 0; m < TC_CLAS_GROUP_TRIANGLES; m++) {
-            const uint32_t word = t[min(t0 + m, tEnd)];  // the last one again past the end
+            for (uint32_t m = 1; m < TC_CLAS_GROUP_TRIANGLES; m++) word[m] = t0 + m < rnt ? word[m] : word[m - 1];
+            const float* v = w.f + (r.y >> 16);
+            float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-              const float* p = v + 3 * ((word >> (8 * c)) & 0xFF);
+            for (uint32_t m = 0; m < TC_CLAS_GROUP_TRIANGLES; m++) {
 #pragma unroll
-              for (int x = 0; x < 3; x++) lo[x] = fminf(lo[x], p[x]), hi[x] = fmaxf(hi[x], p[x]);
+              for (int c = 0; c < 3; c++) {
+                const float* p = v + 3 * ((word[m] >> (8 * c)) & 0xFF);
+#pragma unroll
+                for (int x = 0; x < 3; x++) lo[x] = fminf(lo[x], p[x]), hi[x] = fmaxf(hi[x], p[x]);
+              }
             }
-          }
-          tc_aabb box;
+            float* box = w.f + r.z + 6 * g;
 #pragma unroll
-          for (int x = 0; x < 3; x++) {
-            box.lo[x] = w.box[6 * i + x] = lo[x];
-            box.hi[x] = w.box[6 * i + 3 + x] = hi[x];
+            for (int x = 0; x < 3; x++) box[x] = lo[x], box[3 + x] = hi[x];
           }
-          gst_record(ptr<tc_aabb>(r.boxes) + i, box);
         }
       }
       wave_sync();
@@ -324,38 +312,49 @@ __global__ __launch_bounds__(kClasWaves * kWave) __attribute__((amdgpu_waves_per
         const uint32_t q = lane >> 2, sl = lane & 3;
         const bool mine = q >= done && q < done + k;
         float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-        if (mine) {
-          const ClasRecord& r = w.rec[q];
-          for (uint32_t g = sl; g < r.ng; g += 4) {
-            const float* bx = w.box + 6 * (r.firstGroup + g);
+        const uint4 r = w.group[q];
+        const uint32_t rng = mine ? r.w & 0xFFFF : 0u;
+        for (uint32_t g = sl; g < rng; g += 4) {
+          const float* bx = w.f + r.z + 6 * g;
 #pragma unroll
-            for (int x = 0; x < 3; x++) lo[x] = fminf(lo[x], bx[x]), hi[x] = fmaxf(hi[x], bx[3 + x]);
-          }
+          for (int x = 0; x < 3; x++) lo[x] = fminf(lo[x], bx[x]), hi[x] = fmaxf(hi[x], bx[3 + x]);
         }
 #pragma unroll
         for (int x = 0; x < 3; x++) {
           lo[x] = fminf(lo[x], quad_swap<kSwap1>(lo[x])), hi[x] = fmaxf(hi[x], quad_swap<kSwap1>(hi[x]));
           lo[x] = fminf(lo[x], quad_swap<kSwap2>(lo[x])), hi[x] = fmaxf(hi[x], quad_swap<kSwap2>(hi[x]));
         }
-        const uint64_t rdst = shfl64(dst, q), rsrc = shfl64(src, q);
-        const uint32_t rnt = shfl(nt, q), rnv = shfl(nv, q), rng = shfl(ng, q), rid = shfl(clusterID, q);
-        const uint32_t roT = shfl(oT, q), roV = shfl(oV, q), rsize = shfl(size, q);
         if (mine) {
-          const uint32_t g0 = (uint32_t)sizeof(tc_clas_header) + rng * 24u, t0 = roT + rnt * 4u, v0 = roV + rnv * 12u;
-          char* base = ptr<char>(rdst);
-          if (g0 + 4 * sl < roT) gst(reinterpret_cast<uint32_t*>(base + g0 + 4 * sl), 0u);
-          if (t0 + 4 * sl < roV) gst(reinterpret_cast<uint32_t*>(base + t0 + 4 * sl), 0u);
-          if (v0 + 4 * sl < rsize) gst(reinterpret_cast<uint32_t*>(base + v0 + 4 * sl), 0u);
-          if (sl == 0) {
-            tc_clas_header h;
-            h.lo[0] = lo[0], h.lo[1] = lo[1], h.lo[2] = lo[2];
-            h.hi[0] = hi[0], h.hi[1] = hi[1], h.hi[2] = hi[2];
-            h.clusterID = rid;
-            h.counts = rnt | (rnv << 8) | (rng << 16);
-            h.vertexBase = vertex_base(b, rsrc);
-            h._pad[0] = h._pad[1] = h._pad[2] = 0;
-            gst_record(reinterpret_cast<tc_clas_header*>(base), h);
-            gst(sizes + r0 + q, rsize);
+          const uint4 bl = w.block[q];
+          const uint2 hd = w.head[q];
+          const uint32_t bT = r.y & 0xFFFF, bV = r.y >> 16, rnv = r.w >> 16;
+          const uint32_t g0 = r.z + 6 * rng + sl, t0 = bT + (r.x >> 16) + sl, end = ((hd.y & 0xFFFF) + (hd.y >> 16)) * 4;
+          if (g0 < bT) w.u[g0] = 0;
+          if (t0 < bV) w.u[t0] = 0;
+          if (bV + 3 * rnv + sl < end) w.u[bV + 3 * rnv + sl] = 0;
+          uint4 h = make_uint4(hd.x, 0u, 0u, 0u);
+          if (sl == 0) h = make_uint4(__float_as_uint(lo[0]), __float_as_uint(lo[1]), __float_as_uint(lo[2]), bl.z);
+          if (sl == 1) h = make_uint4(__float_as_uint(hi[0]), __float_as_uint(hi[1]), __float_as_uint(hi[2]), bl.w);
+          if (sl < 3) w.chunk[(hd.y & 0xFFFF) + sl] = h;
+        }
+      }
+      static_assert(sizeof(tc_clas_header) == 48 && offsetof(tc_clas_header, clusterID) == 12 &&
+                        offsetof(tc_clas_header, counts) == 28 && offsetof(tc_clas_header, vertexBase) == 32,
+                    "the header as three chunks");
+      wave_sync();
+      // the image to memory, 1 KB a step
+      if (in) gst(sizes + r0 + lane, size);
+      {
+        uint32_t before = done;
+#pragma unroll
+        for (uint32_t j = 0; j < kRoundBytes / 16 / 64; j++) {
+          if (64 * j >= numC) continue;
+          const uint32_t i = 64 * j + lane, q = record(kHeadC + j, before);
+          if (i < numC) {
+            const uint4 c = w.chunk[i];
+            const uint2 d = *reinterpret_cast<const uint2*>(&w.block[q]);
+            typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(4)));
+            gst(ptr<u4>(u64(d.x, d.y)) + i, u4{c.x, c.y, c.z, c.w});
           }
         }
       }
