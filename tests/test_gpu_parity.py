@@ -414,3 +414,48 @@ def test_clas_runs_and_rounds(quads, rate, stride):
     finally:
         g.close()
     harness.compare(res, of.results())
+
+
+@pytest.mark.parametrize("instances,quads,rate,flags", [
+    (1, 16, 0.25, 0), (2, 64, 1.5, 0), (4, 96, 0.6, 0), (4, 64, 1.0, abi.FLAG_1X_TRANSIENT | abi.FLAG_2X_TRANSIENT)])
+def test_frame_sequence_tiles(instances, quads, rate, flags):
+    """The frame sequence takes its stages' counters, tickets and epochs from
+    the launches before them, and tiles of a size by the number of items
+    (split: 16 to 64, instantiation: 256 to 1024 parts): few and many split
+    triangles and parts equal the oracle, as do two frames in a row and the
+    stage entry points with a prologue each."""
+    host = scene.scene_grid_instances(num_instances=instances, quads=quads, patch_size=6.0, tex_size=64,
+                                      tess_rate_pixels=rate)
+    cfg = harness.small_config(maxPartTriangles=1 << 20, maxGeneratedClusters=(1 << 14) + (1 << 20), maxSplitTriangles=1 << 17,
+                               maxGeneratedVertices=1 << 25, maxGeneratedClusterMegs=2048)
+    cfg.flags |= flags
+    of = harness.OracleFrame(host, cfg)
+    of.run(host.frame(), nthreads=8)
+    ref = of.results()
+    print("split", ref.counters["splitWriteCounter"], "parts", ref.counters["partTriangleCounter"], flush=True)
+    assert ref.counters["splitWriteCounter"] > 0
+    g = harness.GpuFrame(host, cfg)
+    L, b = abi.lib(), C.byref(g.r.bindings)
+    try:
+        g.run(host.frame())
+        g.run(host.frame())
+        harness.compare(g.results(), ref)
+        abi.check(L.tc_renderer_begin_frame(g.r.handle, C.byref(host.frame()), None))
+        abi.check(L.tc_instances_classify(b, cfg, None))
+        abi.check(L.tc_clusters_cull(b, cfg, None))
+        abi.check(L.tc_build_setup(b, cfg, abi.BUILD_SETUP_CLASSIFY, None))
+        abi.check(L.tc_cluster_classify(b, cfg, None))
+        abi.check(L.tc_build_setup(b, cfg, abi.BUILD_SETUP_SPLIT, None))
+        passes = L.tc_num_split_passes(cfg.maxSplitFactor)
+        for p in range(passes):
+            abi.check(L.tc_triangle_split(b, cfg, None))
+            if p + 1 < passes:
+                abi.check(L.tc_build_setup(b, cfg, abi.BUILD_SETUP_SPLIT_PASS, None))
+        abi.check(L.tc_build_setup(b, cfg, abi.BUILD_SETUP_INSTANTIATE_TESS, None))
+        abi.check(L.tc_triangle_tess_template_instantiate(b, cfg, None))
+        abi.check(L.tc_build_setup(b, cfg, abi.BUILD_SETUP_BUILD_BLAS, None))
+        g.r.clas_and_blas()
+        abi.check(L.tc_device_synchronize(), "synchronize")
+        harness.compare(g.results(), ref)
+    finally:
+        g.close()

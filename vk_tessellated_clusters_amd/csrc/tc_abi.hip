@@ -477,8 +477,7 @@ static void launch_prologue(const KArgs& a, int setupMode, uint32_t stage, hipSt
     hipLaunchKernelGGL(k_prologue, dim3(1), dim3(256), 0, st, a, stage);
 }
 
-static tc_status launch_classify(const KArgs& a, tc_config config, int setupMode, hipStream_t st) {
-  launch_prologue(a, setupMode, 0, st);
+static tc_status launch_classify(const KArgs& a, tc_config config, hipStream_t st) {
   uint32_t tiles = (config.maxVisibleClusters + kClassifyMinTile - 1) / kClassifyMinTile;
   uint32_t grid = std::min<uint32_t>(tiles, (uint32_t)num_cu() * tuning_snapshot().classifyBlocksPerCU);
   if (config.flags & TC_FLAG_2X_TRANSIENT) {
@@ -499,21 +498,24 @@ tc_status tc_cluster_classify(const tc_bindings* b, tc_config config, tc_stream 
   KArgs a;
   tc_status s = make_args(b, config, a);
   if (s != TC_OK) return s;
-  return launch_classify(a, config, -1, (hipStream_t)stream);
+  launch_prologue(a, -1, 0, (hipStream_t)stream);
+  return launch_classify(a, config, (hipStream_t)stream);
 }
 
 // One split pass, or with TC_FLAG_PERSISTENT_SPLIT all `passes` passes in
 // one persistent launch (renderer_raytrace_clusters_tess.cpp:510-513).
-static tc_status launch_split(const KArgs& a, tc_config config, uint32_t passes, hipStream_t st, int setupMode = -1) {
+// `pass` >= 0: that pass of the frame sequence, without a prologue.
+static tc_status launch_split(const KArgs& a, tc_config config, uint32_t passes, hipStream_t st, int setupMode = -1,
+                              int pass = -1) {
   if ((config.flags & TC_FLAG_PERSISTENT_SPLIT) && passes > kMaxSplitPasses) return TC_ERROR_UNSUPPORTED;
-  launch_prologue(a, setupMode, 1, st);
+  if (pass < 0) launch_prologue(a, setupMode, 1, st);
   uint32_t tiles = (config.maxSplitTriangles + kWave - 1) / kWave;
   uint32_t grid = std::max<uint32_t>(1u, std::min<uint32_t>(tiles, (uint32_t)num_cu() * tuning_snapshot().splitBlocksPerCU));
   if (config.flags & TC_FLAG_PERSISTENT_SPLIT) {
     hipLaunchKernelGGL(k_split_queue_init, dim3(1), dim3(256), 0, st, a, passes, tuning_snapshot().splitWaitLimit);
     hipLaunchKernelGGL(k_triangle_split_persistent, dim3(grid), dim3(64), 0, st, a);
   } else {
-    hipLaunchKernelGGL(k_triangle_split, dim3(grid), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(k_triangle_split, dim3(grid), dim3(64), 0, st, a, pass, passes);
   }
   return launched();
 }
@@ -525,17 +527,19 @@ tc_status tc_triangle_split(const tc_bindings* b, tc_config config, tc_stream st
   return launch_split(a, config, tc_num_split_passes(config.maxSplitFactor), (hipStream_t)stream);
 }
 
-static tc_status launch_instantiate(const KArgs& a, tc_config config, int setupMode, hipStream_t st) {
-  launch_prologue(a, setupMode, 2, st);
+// `passes` > 0: in the frame sequence of that many split passes, without a
+// prologue and with its setups.
+static tc_status launch_instantiate(const KArgs& a, tc_config config, int setupMode, hipStream_t st, uint32_t passes = 0) {
+  if (!passes) launch_prologue(a, setupMode, 2, st);
   uint32_t tiles = (config.maxPartTriangles + kInstTile - 1) / kInstTile;
   uint32_t grid = std::min<uint32_t>(tiles, (uint32_t)num_cu() * tuning_snapshot().instantiateBlocksPerCU);
-  hipLaunchKernelGGL(k_instantiate, dim3(grid), dim3(kInstWaves * kWave), 0, st, a);
+  hipLaunchKernelGGL(k_instantiate, dim3(grid), dim3(kInstWaves * kWave), 0, st, a, passes);
   // vertices: four waves per workgroup, each taking 64 parts at a time
   const uint32_t vgrid = std::min<uint32_t>((config.maxPartTriangles + kInstTile - 1) / kInstTile, (uint32_t)num_cu() * 8u);
   if (config.flags & TC_FLAG_PN)
-    hipLaunchKernelGGL(k_instantiate_vertices<true>, dim3(vgrid), dim3(kInstWaves * kWave), 0, st, a);
+    hipLaunchKernelGGL(k_instantiate_vertices<true>, dim3(vgrid), dim3(kInstWaves * kWave), 0, st, a, passes);
   else
-    hipLaunchKernelGGL(k_instantiate_vertices<false>, dim3(vgrid), dim3(kInstWaves * kWave), 0, st, a);
+    hipLaunchKernelGGL(k_instantiate_vertices<false>, dim3(vgrid), dim3(kInstWaves * kWave), 0, st, a, passes);
   return launched();
 }
 
@@ -589,24 +593,41 @@ tc_status tc_blas_clusters_insert(const tc_bindings* b, tc_config config, int tr
   return launched();
 }
 
-// renderer_raytrace_clusters_tess.cpp:467-582 on a prepared argument block;
-// each build_setup that precedes a stage runs in that stage's prologue
-// launch
-static tc_status frame_tessellate(const KArgs& a, tc_config config, uint32_t numSplitPasses, hipStream_t st) {
+// renderer_raytrace_clusters_tess.cpp:467-582 on a prepared argument block.
+// The frame sequence: one prologue launch opens every stage's epoch and ticket
+// (and classifies the instances, when `instances`), and each build_setup is
+// made by the stage launch next to it, from what the launch before left in the
+// workspace header.  A small launch takes 3 to 4.5 us between two others
+// whatever it does, and the chain had eight of them (six prologues, the last
+// build_setup, the instances).  The persistent split keeps its prologues: its
+// passes hand over within one launch, through the same header.
+static tc_status frame_tessellate(const KArgs& a, tc_config config, uint32_t numSplitPasses, hipStream_t st,
+                                  bool instances = false) {
   tc_status s;
   if (numSplitPasses == 0) numSplitPasses = tc_num_split_passes(config.maxSplitFactor);
-  if ((s = launch_classify(a, config, TC_BUILD_SETUP_CLASSIFY, st)) != TC_OK) return s;
-  if (config.flags & TC_FLAG_PERSISTENT_SPLIT) {
-    // every pass, with its SPLIT_PASS setup, in one launch
-    if ((s = launch_split(a, config, numSplitPasses, st, TC_BUILD_SETUP_SPLIT)) != TC_OK) return s;
-  } else {
-    for (uint32_t p = 0; p < numSplitPasses; p++)
-      if ((s = launch_split(a, config, numSplitPasses, st, p == 0 ? TC_BUILD_SETUP_SPLIT : TC_BUILD_SETUP_SPLIT_PASS)) != TC_OK)
-        return s;
+  if ((config.flags & TC_FLAG_PERSISTENT_SPLIT) || numSplitPasses > kMaxSplitPasses) {
+    if (instances)
+      hipLaunchKernelGGL(k_instances_classify, dim3((a.numInstances + 63) / 64), dim3(64), 0, st, a);
+    launch_prologue(a, TC_BUILD_SETUP_CLASSIFY, 0, st);
+    if ((s = launch_classify(a, config, st)) != TC_OK) return s;
+    if (config.flags & TC_FLAG_PERSISTENT_SPLIT) {
+      // every pass, with its SPLIT_PASS setup, in one launch
+      if ((s = launch_split(a, config, numSplitPasses, st, TC_BUILD_SETUP_SPLIT)) != TC_OK) return s;
+    } else {
+      for (uint32_t p = 0; p < numSplitPasses; p++)
+        if ((s = launch_split(a, config, numSplitPasses, st, p == 0 ? TC_BUILD_SETUP_SPLIT : TC_BUILD_SETUP_SPLIT_PASS)) != TC_OK)
+          return s;
+    }
+    if ((s = launch_instantiate(a, config, TC_BUILD_SETUP_INSTANTIATE_TESS, st)) != TC_OK) return s;
+    hipLaunchKernelGGL(k_build_setup, dim3(1), dim3(1), 0, st, a, (int)TC_BUILD_SETUP_BUILD_BLAS);
+    return launched();
   }
-  if ((s = launch_instantiate(a, config, TC_BUILD_SETUP_INSTANTIATE_TESS, st)) != TC_OK) return s;
-  hipLaunchKernelGGL(k_build_setup, dim3(1), dim3(1), 0, st, a, (int)TC_BUILD_SETUP_BUILD_BLAS);
-  return launched();
+  hipLaunchKernelGGL(k_frame_prologue, dim3(1 + (instances ? (a.numInstances + 255) / 256 : 0)), dim3(256), 0, st, a,
+                     numSplitPasses);
+  if ((s = launch_classify(a, config, st)) != TC_OK) return s;
+  for (uint32_t p = 0; p < numSplitPasses; p++)
+    if ((s = launch_split(a, config, numSplitPasses, st, -1, (int)p)) != TC_OK) return s;
+  return launch_instantiate(a, config, -1, st, numSplitPasses);
 }
 
 tc_status tc_frame_tessellate(const tc_bindings* b, tc_config config, uint32_t numSplitPasses, tc_stream stream) {
@@ -615,6 +636,17 @@ tc_status tc_frame_tessellate(const tc_bindings* b, tc_config config, uint32_t n
   if (s != TC_OK) return s;
   return frame_tessellate(a, config, numSplitPasses, (hipStream_t)stream);
 }
+
+}  // extern "C"
+
+tc_status tc::frame_tessellate_instances(const tc_bindings* b, tc_config config, bool instances, tc_stream stream) {
+  KArgs a;
+  tc_status s = make_args(b, config, a);
+  if (s != TC_OK) return s;
+  return frame_tessellate(a, config, 0, (hipStream_t)stream, instances);
+}
+
+extern "C" {
 
 // ---------------------------------------------- allocation-free variant
 //

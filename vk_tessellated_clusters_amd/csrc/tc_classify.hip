@@ -319,8 +319,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 
   WsHeader* h = a.ws;
   const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
-  const uint32_t epoch = h->epoch, numTiles = h->numTiles, numItems = h->itemEnd;
+  const uint32_t epoch = h->epoch0, numTiles = h->numTiles, numItems = h->itemEnd;
   const uint32_t tileItems = h->tileItems;
+  if (blockIdx.x >= numTiles) return;  // at most numTiles workgroups take tickets
   const uint64_t B0 = h->base[0], B1 = h->base[1], B2 = h->base[2], B3 = h->base[3], B4 = h->base[4], B5 = h->base[5];
   const uint64_t B6 = h->base[6], B7 = h->base[7];
   const ViewParams vp = view_params(a);
@@ -701,6 +702,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
           b->genVertexCounter = (uint32_t)(B3 + excl[3] + agg[3]);
           b->genClusterDataCounter = B4 + excl[4] + agg[4];
           b->dualPartTriangleCounter = ((B6 + excl[5] + agg[5]) << 32) | (uint32_t)(B1 + excl[1] + agg[1]);
+          // frame sequence: split pass 0 (build_setup SPLIT)
+          SplitPass& p0 = split_queue(h)->pass[0];
+          p0.itemBegin = 0;
+          p0.itemEnd = min((uint32_t)(B0 + excl[0] + agg[0]), cfg.maxSplitTriangles);
+          p0.b0 = p0.itemEnd;
+          p0.b1 = (uint32_t)(B1 + excl[1] + agg[1]);
         }
       }
     }

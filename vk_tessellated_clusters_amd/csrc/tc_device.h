@@ -575,13 +575,23 @@ struct WsHeader {
   uint32_t itemBegin; // first item of the current launch
   uint32_t itemEnd;   // end of the items of the current launch
   uint32_t tileItems; // items per tile, where the stage varies them (classify)
-  uint32_t _pad[2];
+  uint32_t epoch0;    // frame sequence: classify's epoch (split pass p takes epoch0 + 1 + p, ...)
+  uint32_t _pad;
   uint64_t base[8];   // counter values at launch start
+  // The frame sequence (multipass split) opens the epochs of all its stages
+  // and resets their tickets in its first launch, and the stages take what
+  // they start from out of these fields, so no launch lies between them.
+  uint32_t splitTicket[16];
+  uint32_t instTicket;
+  uint32_t _pad1;
+  uint64_t instBase[4];  // generated clusters, vertices, CLAS bytes, instantiations before the parts
 };
 constexpr uint64_t kWsHeaderBytes = 1024;
+static_assert(sizeof(WsHeader) <= 256, "the split passes follow at byte 256");
 
-// Pass table of the persistent split kernel (TC_FLAG_PERSISTENT_SPLIT),
-// after the header: pass p covers global tickets [tileBegin, tileBegin +
+// Pass table of the split, after the header.  In the frame sequence pass p
+// finds its items and counters in entry p, written by the launch before it.
+// For the persistent kernel (TC_FLAG_PERSISTENT_SPLIT) pass p covers global tickets [tileBegin, tileBegin +
 // numTiles); a pass is published (passReady > p) once the pass before it
 // has completed, and `finished` is set when no pass with tiles is left.
 constexpr uint32_t kMaxSplitPasses = 16;
@@ -626,9 +636,9 @@ __device__ __forceinline__ uint32_t take_ticket(WsHeader* h) {
 // nothing to split: thousands of them) leave without an atomic on the one
 // ticket word.  The read costs a round trip per tile, so launches that
 // always have work take tickets directly.  One thread.
-__device__ __forceinline__ uint32_t take_ticket_below(WsHeader* h, uint32_t numTiles) {
-  if (__hip_atomic_load(&h->ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= numTiles) return numTiles;
-  return __hip_atomic_fetch_add(&h->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ uint32_t take_ticket_below(uint32_t* ticket, uint32_t numTiles) {
+  if (__hip_atomic_load(ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= numTiles) return numTiles;
+  return __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Decoupled look-back over N counters for `tile`, executed by one full

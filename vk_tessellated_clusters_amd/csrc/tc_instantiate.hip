@@ -1,8 +1,8 @@
 // tc_instantiate.hip -- triangle_tess_template_instantiate.comp.glsl:126-373
 // on gfx950, as two launches.
 //
-// k_instantiate allocates: a workgroup of four waves owns a tile of 256 part
-// triangles, and the allocation of every part (generated cluster, vertices,
+// k_instantiate allocates: a workgroup of four waves owns a tile of 256 to 1024
+// part triangles, and the allocation of every part (generated cluster, vertices,
 // CLAS bytes) is a prefix sum over parts in index order: wave-level scans, a
 // workgroup combine and one decoupled look-back per tile.  It writes the
 // instantiation records and the BLAS reference counts.  Its tiles carry no
@@ -20,9 +20,14 @@
 
 namespace tc {
 
-// Parts per lane of the allocation kernel: a wave covers kPartsPerLane x 64
-// consecutive parts, a tile kInstWaves such runs (kInstTile parts).
-constexpr uint32_t kPartsPerLane = kInstTile / (kInstWaves * kWave);
+// Parts per lane of the allocation kernel, at most: a wave covers that many
+// times 64 consecutive parts, a tile kInstWaves such runs (kInstTile parts).
+// Halved down to one while a frame's parts make fewer than kInstTiles tiles:
+// 1280 parts 14.5 -> 10 us, 26,000 parts 16.6 -> 12.8 us (64 to 128 tiles the
+// same; 512 tiles make 246,000 parts take 35 us instead of 22).
+constexpr uint32_t kInstLanes = kInstWaves * kWave;
+constexpr uint32_t kPartsPerLane = kInstTile / kInstLanes;
+constexpr uint32_t kInstTiles = 128;
 // Parts a wave stages at a time in the vertex kernel.
 constexpr uint32_t kVertChunk = 32;
 
@@ -60,7 +65,12 @@ __device__ __forceinline__ tc_tess_triangle_info load_part(const KArgs& a, uint3
 // prefix: the owner of the first rejected part, or of the last part when
 // none is rejected.  It alone writes tempInstantiateCounter = T0 + A and
 // adds the prefix's triangles to the readback.
-__global__ __launch_bounds__(256) void k_instantiate(KArgs a) {
+// After a prologue (numPasses 0) it starts from the header's snapshot; in the
+// frame sequence of numPasses split passes every workgroup takes the parts
+// and bases from what the launches before left, and the first one makes the
+// split's and the instantiation's setups (the counters it clamps there are
+// clamped by every reader, so either value gives the same parts).
+__global__ __launch_bounds__(256) void k_instantiate(KArgs a, uint32_t numPasses) {
   __shared__ uint64_t s_wave[kInstWaves][4];
   __shared__ uint64_t s_excl[4];
   __shared__ uint32_t s_tile;
@@ -68,22 +78,39 @@ __global__ __launch_bounds__(256) void k_instantiate(KArgs a) {
 
   WsHeader* h = a.ws;
   const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
-  const uint32_t epoch = h->epoch, numTiles = h->numTiles, numParts = h->itemEnd;
-  const uint64_t G0 = h->base[0], V0 = h->base[1], D0 = h->base[2], T0 = h->base[3];
-  const TableView T = load_table(a.tessTable);
   tc_scene_building* b = a.build;
   const tc_config cfg = a.cfg;
+  const uint64_t* base0 = numPasses ? h->instBase : h->base;
+  const uint64_t G0 = base0[0], V0 = base0[1], D0 = base0[2], T0 = base0[3];
+  uint32_t epoch = h->epoch, numTiles, numParts = h->itemEnd;
+  uint32_t* ticket = &h->ticket;
+  if (numPasses) {
+    epoch = h->epoch0 + 1 + numPasses;
+    ticket = &h->instTicket;
+    numParts = accepted_parts(a);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      split_state_one(a, numPasses);
+      build_setup_one(a, TC_BUILD_SETUP_INSTANTIATE_TESS);
+    }
+  }
+  // few parts go to smaller tiles: fewer parts per lane
+  uint32_t ppl = kPartsPerLane;
+  while (ppl > 1 && numParts < ppl * kInstLanes * kInstTiles && (numParts + ppl * kInstLanes / 2 - 1) / (ppl * kInstLanes / 2) <= a.maxTiles)
+    ppl /= 2;
+  numTiles = min((numParts + ppl * kInstLanes - 1) / (ppl * kInstLanes), a.maxTiles);
+  if (blockIdx.x >= numTiles) return;  // at most numTiles workgroups take tickets
+  const TableView T = load_table(a.tessTable);
   const uint64_t maxData = max_data_bytes(cfg);
   tc_blas_build_info* infos = ptr<tc_blas_build_info>(b->blasBuildInfos);
 
   while (true) {
-    if (threadIdx.x == 0) s_tile = __hip_atomic_fetch_add(&h->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) s_tile = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     const uint32_t tile = s_tile;
     if (tile >= numTiles) break;
 
     // this lane's parts: base + k * 64, k < kPartsPerLane (coalesced rounds)
-    const uint32_t base = tile * kInstTile + wave * (kPartsPerLane * kWave) + lane;
+    const uint32_t base = tile * ppl * kInstLanes + wave * (ppl * kWave) + lane;
     tc_tess_triangle_info ti[kPartsPerLane];
     uint32_t nv[kPartsPerLane], nt[kPartsPerLane];
     uint64_t ds[kPartsPerLane];
@@ -92,7 +119,7 @@ __global__ __launch_bounds__(256) void k_instantiate(KArgs a) {
       const uint32_t p = base + k * kWave;
       nv[k] = nt[k] = 0;
       ds[k] = 0;
-      if (p < numParts) {
+      if (k < ppl && p < numParts) {
         ti[k] = load_part(a, p);
         const uint32_t cf = ti[k].subTriangle.triangleID_config >> 16;
         const tc_tess_table_entry e = cfg_entry(T, cf);
@@ -106,6 +133,7 @@ __global__ __launch_bounds__(256) void k_instantiate(KArgs a) {
     uint64_t excl[kPartsPerLane][4];
 #pragma unroll
     for (uint32_t k = 0; k < kPartsPerLane; k++) {
+      if (k >= ppl) break;
       const uint32_t g = base + k * kWave < numParts ? 1u : 0u;
       const uint32_t gi = wave_incl_scan(g), vi = wave_incl_scan(nv[k]), ti3 = wave_incl_scan(nt[k]);
       const uint64_t di = wave_incl_scan64(ds[k]);
@@ -150,6 +178,7 @@ __global__ __launch_bounds__(256) void k_instantiate(KArgs a) {
     bool single = true;
 #pragma unroll
     for (uint32_t k = 0; k < kPartsPerLane; k++) {
+      if (k >= ppl) break;
       const uint32_t p = base + k * kWave;
       const bool valid = p < numParts;
       const uint64_t genOffset = G0 + wb[0] + excl[k][0];
@@ -222,14 +251,17 @@ __global__ __launch_bounds__(256) void k_instantiate(KArgs a) {
 // k_instantiate wrote to tempInstantiateCounter above its start value.
 // Waves take kVertChunk parts at a time, grid-stride.
 template <bool PN>
-__global__ __launch_bounds__(256) void k_instantiate_vertices(KArgs a) {
+__global__ __launch_bounds__(256) void k_instantiate_vertices(KArgs a, uint32_t numPasses) {
   __shared__ PartBase s_parts[kInstWaves][kVertChunk];
   __shared__ PNBasis s_pn[PN ? kInstWaves : 1][PN ? kVertChunk : 1];
   __shared__ uint32_t s_start[kInstWaves][kVertChunk];
 
   const WsHeader* h = a.ws;
   const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
-  const uint32_t T0 = (uint32_t)h->base[3];
+  const uint32_t T0 = (uint32_t)(numPasses ? h->instBase[3] : h->base[3]);
+  // frame sequence: build_setup BUILD_BLAS (accepted parts fit
+  // maxGeneratedClusters, so its clamp leaves the counter as it is)
+  if (numPasses && blockIdx.x == 0 && threadIdx.x == 0) build_setup_one(a, TC_BUILD_SETUP_BUILD_BLAS);
   const TableView T = load_table(a.tessTable);
   const tc_scene_building* b = a.build;
   const uint32_t accepted = b->tempInstantiateCounter - T0;
@@ -312,7 +344,7 @@ __global__ __launch_bounds__(256) void k_instantiate_vertices(KArgs a) {
   }
 }
 
-template __global__ void k_instantiate_vertices<false>(KArgs);
-template __global__ void k_instantiate_vertices<true>(KArgs);
+template __global__ void k_instantiate_vertices<false>(KArgs, uint32_t);
+template __global__ void k_instantiate_vertices<true>(KArgs, uint32_t);
 
 }  // namespace tc

@@ -70,6 +70,9 @@ WsLayout ws_layout(const tc_config& cfg, uint32_t numInstances);
 tc_status make_args_public(const tc_bindings* b, const tc_config& cfg, KArgs& a);
 int num_cu_public();
 tc_tuning tuning_snapshot();
+// tc_frame_tessellate, with the instances classified in its first launch when
+// `instances` (tc_instances_classify before it)
+tc_status frame_tessellate_instances(const tc_bindings* b, tc_config config, bool instances, tc_stream stream);
 
 __global__ void k_prologue(KArgs a, uint32_t stage);
 __global__ void k_build_setup(KArgs a, int mode);
@@ -77,12 +80,13 @@ __global__ void k_setup_prologue(KArgs a, int mode, uint32_t stage);
 template <bool TWO_X, bool TRANS>
 __global__ void k_cluster_classify(KArgs a);
 __global__ void k_mini_vertices(KArgs a);
-__global__ void k_triangle_split(KArgs a);
+__global__ void k_frame_prologue(KArgs a, uint32_t numPasses);
+__global__ void k_triangle_split(KArgs a, int pass, uint32_t numPasses);
 __global__ void k_split_queue_init(KArgs a, uint32_t numPasses, uint32_t waitLimit);
 __global__ void k_triangle_split_persistent(KArgs a);
-__global__ void k_instantiate(KArgs a);
+__global__ void k_instantiate(KArgs a, uint32_t numPasses);
 template <bool PN>
-__global__ void k_instantiate_vertices(KArgs a);
+__global__ void k_instantiate_vertices(KArgs a, uint32_t numPasses);
 __global__ void k_blas_setup_insertion(KArgs a);
 __global__ void k_instances_classify(KArgs a);
 __global__ void k_clusters_cull_scan(KArgs a, uint32_t* offsets);

@@ -15,14 +15,15 @@ namespace tc {
 
 // Opens a new look-back launch: bumps the epoch (clearing stale status
 // words when it wraps), resets the ticket and snapshots the counters the
-// stage advances.  One workgroup.
-__device__ void prologue_body(const KArgs& a, uint32_t stage) {
+// stage advances.  `more` further epochs are taken for the stages that follow
+// without a prologue (the frame sequence).  One workgroup.
+__device__ void prologue_body(const KArgs& a, uint32_t stage, uint32_t more = 0) {
   __shared__ uint32_t s_epoch;
   WsHeader* h = a.ws;
   tc_scene_building* b = a.build;
   if (threadIdx.x == 0) {
     uint32_t e = h->epoch + 1;
-    s_epoch = e >= (1u << kEpochBits) ? 0u : e;
+    s_epoch = e + more >= (1u << kEpochBits) ? 0u : e;
   }
   __syncthreads();
   uint32_t e = s_epoch;
@@ -34,7 +35,8 @@ __device__ void prologue_body(const KArgs& a, uint32_t stage) {
   }
   __syncthreads();
   if (threadIdx.x != 0) return;
-  h->epoch = e;
+  h->epoch = e + more;
+  h->epoch0 = e;
   h->ticket = 0;
   if (stage == kStageClassify) {
     const uint32_t n = min(b->visibleClusterCounter, a.cfg.maxVisibleClusters);
@@ -76,82 +78,6 @@ __device__ void prologue_body(const KArgs& a, uint32_t stage) {
 __global__ __launch_bounds__(256) void k_prologue(KArgs a, uint32_t stage) { prologue_body(a, stage); }
 
 // ---------------------------------------------------------- build_setup
-
-// build_setup.comp.glsl:102-264 (transient builds with TC_FLAG_1X_TRANSIENT
-// or TC_FLAG_2X_TRANSIENT).  One thread.
-__device__ void build_setup_one(const KArgs& a, int mode) {
-  tc_scene_building* b = a.build;
-  tc_readback* rb = a.readback;
-  const tc_config& cfg = a.cfg;
-  if (mode == TC_BUILD_SETUP_CLASSIFY) {
-    uint32_t counter = b->visibleClusterCounter;
-    rb->numVisibleClusters = counter;
-    counter = min(counter, cfg.maxVisibleClusters);
-    b->visibleClusterCounter = counter;
-    b->dispatchClassify = tc_dispatch_indirect{counter, 1, 1};
-  } else if (mode == TC_BUILD_SETUP_DRAW_TESS) {
-    uint32_t full = b->fullClusterCounter, part = b->partTriangleCounter;
-    rb->numFullClusters = full;
-    rb->numPartTriangles = part;
-    rb->numSplitTriangles = b->splitWriteCounter;
-    full = min(full, cfg.maxVisibleClusters);
-    part = min(part, cfg.maxPartTriangles);
-    b->drawFullClusters = tc_draw_mesh_tasks_indirect{full, 0};
-    b->drawPartTriangles = tc_draw_mesh_tasks_indirect{(part + 31) / 32, 0};
-    rb->numBlasClusters = full;
-  } else if (mode == TC_BUILD_SETUP_SPLIT) {
-    uint32_t count = min((uint32_t)b->splitTriangleCounter, cfg.maxSplitTriangles);
-    b->splitWriteCounter = count;
-    b->splitTriangleCounter = (int32_t)count;
-    b->splitPassStart = 0;
-    b->splitPassEnd = count;
-    b->dispatchTriangleSplit = tc_dispatch_indirect{(count + 63) / 64, 1, 1};
-  } else if (mode == TC_BUILD_SETUP_SPLIT_PASS) {
-    b->splitPass = b->splitPass + 1;
-    uint32_t start = min(b->splitPassEnd, cfg.maxSplitTriangles);
-    uint32_t end = min(b->splitWriteCounter, cfg.maxSplitTriangles);
-    b->splitPassStart = start;
-    b->splitPassEnd = end;
-    b->dispatchTriangleSplit = tc_dispatch_indirect{(end - start + 63) / 64, 1, 1};
-  } else if (mode == TC_BUILD_SETUP_BUILD_BLAS) {
-    const bool trans = transient_builds(cfg.flags);
-    uint32_t temp = b->tempInstantiateCounter;
-    uint32_t tr = trans ? b->transBuildCounter : 0u;
-    rb->numBlasClusters = temp + tr;
-    if (trans) rb->numTransBuilds = tr;
-    rb->numTempInstantiations = temp;
-    rb->numGenDatas = b->genClusterDataCounter;
-    rb->numGenVertices = b->genVertexCounter;
-    rb->numBlasReservedSizes = b->numBlasReservedSizes;
-    temp = min(cfg.maxGeneratedClusters, temp);
-    b->tempInstantiateCounter = temp;
-    rb->numActualTempInstantiations = temp;
-    b->dispatchBlasTempInsert = tc_dispatch_indirect{(temp + 63) / 64, 1, 1};
-    if (trans) {
-      tr = min(cfg.maxGeneratedClusters, temp + tr) - temp;
-      b->transBuildCounter = tr;
-      rb->numActualTransBuilds = tr;
-      b->dispatchBlasTransInsert = tc_dispatch_indirect{(tr + 63) / 64, 1, 1};
-    }
-  } else if (mode == TC_BUILD_SETUP_INSTANTIATE_TESS) {
-    uint32_t part = b->partTriangleCounter;
-    rb->numSplitTriangles = b->splitWriteCounter;
-    if (transient_builds(cfg.flags)) {
-      // :240-253: the instantiated parts are the accepted prefix
-      // x + y + 2 <= MAX_PART_TRIANGLES of the lower counter
-      const uint32_t y = (uint32_t)(b->dualPartTriangleCounter >> 32);
-      rb->numPartTriangles = part + y;
-      rb->numTransPartTriangles = y;
-      const uint32_t cap = cfg.maxPartTriangles > y + 1 ? cfg.maxPartTriangles - y - 1 : 0u;
-      part = min(part, cap);
-    } else {
-      rb->numPartTriangles = part;
-      part = min(part, cfg.maxPartTriangles);
-    }
-    b->partTriangleCounter = part;
-    b->dispatchTriangleInstantiate = tc_dispatch_indirect{(part + 31) / 32, 1, 1};
-  }
-}
 
 __global__ void k_build_setup(KArgs a, int mode) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
@@ -197,20 +123,54 @@ __device__ __forceinline__ void split_child(const TableView& T, const SplitItem&
 }
 
 
+// Whether a child with factors f splits again; its factors become those of
+// that split (at most TC_TESSTABLE_SIZE either way).
+__device__ __forceinline__ bool final_factors(uint32_t f[3], uint32_t maxSplitFactor) {
+  if (umax3(f[0], f[1], f[2]) <= TC_TESSTABLE_SIZE) return false;
+#pragma unroll
+  for (int k = 0; k < 3; k++) f[k] = split_factor(f[k], maxSplitFactor);
+  return true;
+}
+
+// Children of a tile whose phase A results phase B finds in LDS (4 KB): a
+// tile of 64 items has 128 and more children).  Computing them again made the
+// four passes of 2300 split triangles take 58 us instead of 53, of 166,000 279
+// instead of 269.
+constexpr uint32_t kSplitKeep = 256;
+
+// Items per tile of a frame-sequence pass, at least and at most: a wave walks
+// its tile's children 64 at a time, so a pass of few items takes tiles of
+// fewer, halved while there are fewer than kSplitTiles tiles (2300 items in
+// four passes 46 -> 31 us).  Passes of more items keep 64: 2048 tiles would make
+// 166,000 items take 302 us instead of 206.
+constexpr uint32_t kSplitMinTile = 16;
+constexpr uint32_t kSplitTiles = 128;
+
+// The split pass after one that ended at item `end` with the given counters
+// (build_setup SPLIT_PASS, build_setup.comp.glsl:168-190).
+__device__ __forceinline__ SplitPass next_split_pass(const KArgs& a, uint32_t end, uint32_t written, uint32_t parts) {
+  SplitPass p{};
+  p.itemBegin = min(end, a.cfg.maxSplitTriangles);
+  p.itemEnd = min(written, a.cfg.maxSplitTriangles);
+  p.b0 = written;
+  p.b1 = parts;
+  return p;
+}
+
 // triangle_split.comp.glsl:598-632 + processAllSubTasks :350-472 for one
 // tile of 64 split items (one wave); children packed densely over the wave.
 // Counters: 0 split, 1 part.  The last tile of a pass writes the pass's
 // split / part totals to SceneBuilding.
 __device__ __forceinline__ void split_tile(const KArgs& a, const TableView& T, const ViewParams& vp, SplitItem* s_items,
-                                           uint32_t* s_start, uint32_t tile, uint32_t numTiles, uint32_t epoch,
+                                           uint32_t* s_start, uint4* s_keep, uint32_t tile, uint32_t numTiles, uint32_t epoch,
                                            uint32_t itemBegin, uint32_t itemEnd, uint64_t B0, uint64_t B1, uint64_t transY,
-                                           const uint32_t* abort = nullptr) {
+                                           const uint32_t* abort = nullptr, SplitPass* next = nullptr, uint32_t ts = kWave) {
   const uint32_t lane = lane_id();
   tc_scene_building* b = a.build;
   const tc_config& cfg = a.cfg;
   // setupTask + fillBaseVertices (:146-199) once per item
-  const uint32_t idx = itemBegin + tile * kWave + lane;
-  bool valid = idx < itemEnd;
+  const uint32_t idx = itemBegin + tile * ts + lane;
+  bool valid = lane < ts && idx < itemEnd;
   uint32_t count = 0;
   {
     SplitItem it;
@@ -247,7 +207,9 @@ __device__ __forceinline__ void split_tile(const KArgs& a, const TableView& T, c
   const uint32_t total = shfl(wave_incl_scan(count), kWave - 1);
   __syncthreads();
 
-  // phase A: count children going to the split and part lists
+  // phase A: count children going to the split and part lists; the corners
+  // and final factors of the first kSplitKeep stay in LDS for phase B (each
+  // takes a chain of table reads)
   uint32_t ns = 0, np = 0;
   for (uint32_t t0 = 0; t0 < total; t0 += kWave) {
     const uint32_t t = t0 + lane;
@@ -256,9 +218,9 @@ __device__ __forceinline__ void split_tile(const KArgs& a, const TableView& T, c
       const SplitItem& it = s_items[find_owner(s_start, t)];
       uint32_t vtx[3], f[3];
       split_child(T, it, t - it.start, vp, vtx, f);
-      uint32_t mx = umax3(f[0], f[1], f[2]);
-      needSplit = mx > TC_TESSTABLE_SIZE;
+      needSplit = final_factors(f, cfg.maxSplitFactor);
       needPart = !needSplit;
+      if (t < kSplitKeep) s_keep[t] = make_uint4(vtx[0], vtx[1], vtx[2], f[0] | f[1] << 8 | f[2] << 16 | (needSplit ? 1u << 31 : 0u));
     }
     ns += __popcll(ballot(needSplit));
     np += __popcll(ballot(needPart));
@@ -275,9 +237,15 @@ __device__ __forceinline__ void split_tile(const KArgs& a, const TableView& T, c
     const SplitItem* itp = nullptr;
     if (t < total) {
       itp = &s_items[find_owner(s_start, t)];
-      split_child(T, *itp, t - itp->start, vp, vtx, f);
-      uint32_t mx = umax3(f[0], f[1], f[2]);
-      needSplit = mx > TC_TESSTABLE_SIZE;
+      if (t < kSplitKeep) {
+        const uint4 k = s_keep[t];
+        vtx[0] = k.x, vtx[1] = k.y, vtx[2] = k.z;
+        f[0] = k.w & 0xFF, f[1] = (k.w >> 8) & 0xFF, f[2] = (k.w >> 16) & 0xFF;
+        needSplit = (k.w >> 31) != 0;
+      } else {
+        split_child(T, *itp, t - itp->start, vp, vtx, f);
+        needSplit = final_factors(f, cfg.maxSplitFactor);
+      }
       needPart = !needSplit;
     }
     uint64_t vs = ballot(needSplit), vpm = ballot(needPart);
@@ -286,11 +254,6 @@ __device__ __forceinline__ void split_tile(const KArgs& a, const TableView& T, c
     runSplit += __popcll(vs);
     runPart += __popcll(vpm);
     if (needSplit || needPart) {
-      if (needSplit) {
-        f[0] = split_factor(f[0], cfg.maxSplitFactor);
-        f[1] = split_factor(f[1], cfg.maxSplitFactor);
-        f[2] = split_factor(f[2], cfg.maxSplitFactor);
-      }
       uint32_t cf = get_config(f, vtx);
       tc_tess_triangle_info ti;
       ti.cluster = itp->cluster;
@@ -314,25 +277,63 @@ __device__ __forceinline__ void split_tile(const KArgs& a, const TableView& T, c
     b->splitWriteCounter = (uint32_t)(B0 + excl[0] + agg[0]);
     b->partTriangleCounter = (uint32_t)(B1 + excl[1] + agg[1]);
     b->dualPartTriangleCounter = (transY << 32) | (uint32_t)(B1 + excl[1] + agg[1]);
+    // frame sequence: what the next pass starts from
+    if (next) *next = next_split_pass(a, itemEnd, (uint32_t)(B0 + excl[0] + agg[0]), (uint32_t)(B1 + excl[1] + agg[1]));
   }
   __syncthreads();
 }
 
 // One split pass (multipass form, the reference default): tiles by ticket.
-__global__ __launch_bounds__(64) void k_triangle_split(KArgs a) {
+// After a prologue (pass < 0) it starts from the header's snapshot; pass p of
+// the frame sequence starts from entry p of the pass table and leaves entry
+// p + 1 (its last tile does, or the first workgroup of an empty pass).
+__global__ __launch_bounds__(64) void k_triangle_split(KArgs a, int pass, uint32_t numPasses) {
   __shared__ SplitItem s_items[kWave];
   __shared__ uint32_t s_start[kWave];
+  __shared__ uint4 s_keep[kSplitKeep];
   WsHeader* h = a.ws;
-  const uint32_t epoch = h->epoch, numTiles = h->numTiles, itemBegin = h->itemBegin, itemEnd = h->itemEnd;
-  const uint64_t B0 = h->base[0], B1 = h->base[1], transY = h->base[2];
+  tc_scene_building* b = a.build;
+  uint32_t epoch, numTiles, itemBegin, itemEnd, ts = kWave;
+  uint32_t* ticket;
+  uint64_t B0, B1, transY;
+  SplitPass* next = nullptr;
+  if (pass < 0) {
+    epoch = h->epoch, numTiles = h->numTiles, itemBegin = h->itemBegin, itemEnd = h->itemEnd;
+    B0 = h->base[0], B1 = h->base[1], transY = h->base[2];
+    ticket = &h->ticket;
+  } else {
+    SplitQueue* q = split_queue(h);
+    const SplitPass& P = q->pass[pass];
+    itemBegin = P.itemBegin, itemEnd = P.itemEnd, B0 = P.b0, B1 = P.b1;
+    transY = b->dualPartTriangleCounter >> 32;
+    epoch = h->epoch0 + 1 + (uint32_t)pass;
+    ticket = &h->splitTicket[pass];
+    const uint32_t n = itemEnd > itemBegin ? itemEnd - itemBegin : 0u;
+    while (ts > kSplitMinTile && n < ts * kSplitTiles && (n + ts / 2 - 1) / (ts / 2) <= a.maxTiles) ts /= 2;
+    numTiles = min((n + ts - 1) / ts, a.maxTiles);
+    if ((uint32_t)pass + 1 < numPasses) next = &q->pass[pass + 1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      if (numTiles == 0 && next) *next = next_split_pass(a, itemEnd, (uint32_t)B0, (uint32_t)B1);
+      if (pass == 0) {
+        if (numTiles == 0) b->splitWriteCounter = (uint32_t)B0;
+        h->instBase[0] = b->genClusterCounter;
+        h->instBase[1] = b->genVertexCounter;
+        h->instBase[2] = b->genClusterDataCounter;
+        h->instBase[3] = b->tempInstantiateCounter;
+      }
+    }
+  }
+  // At most numTiles workgroups take tickets: 2048 workgroups queueing atomics
+  // on one word cost a pass of few tiles 10 to 20 us.
+  if (blockIdx.x >= numTiles) return;
   const ViewParams vp = view_params(a);
   const TableView T = load_table(a.tessTable);
   while (true) {
     uint32_t tile = 0;
-    if (lane_id() == 0) tile = take_ticket_below(h, numTiles);
+    if (lane_id() == 0) tile = take_ticket_below(ticket, numTiles);
     tile = uniform(tile);
     if (tile >= numTiles) break;
-    split_tile(a, T, vp, s_items, s_start, tile, numTiles, epoch, itemBegin, itemEnd, B0, B1, transY);
+    split_tile(a, T, vp, s_items, s_start, s_keep, tile, numTiles, epoch, itemBegin, itemEnd, B0, B1, transY, nullptr, next, ts);
   }
 }
 
@@ -435,6 +436,7 @@ __global__ __launch_bounds__(256) void k_split_queue_init(KArgs a, uint32_t numP
 __global__ __launch_bounds__(64) void k_triangle_split_persistent(KArgs a) {
   __shared__ SplitItem s_items[kWave];
   __shared__ uint32_t s_start[kWave];
+  __shared__ uint4 s_keep[kSplitKeep];
   WsHeader* h = a.ws;
   SplitQueue* q = split_queue(h);
   const uint32_t lane = lane_id();
@@ -497,7 +499,7 @@ __global__ __launch_bounds__(64) void k_triangle_split_persistent(KArgs a) {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     const SplitPass& Q = q->pass[p];
     const uint32_t tileBegin = ld_agent(&Q.tileBegin), numTiles = ld_agent(&Q.numTiles);
-    split_tile(a, T, vp, s_items, s_start, g - tileBegin, numTiles, ld_agent(&Q.epoch), ld_agent(&Q.itemBegin),
+    split_tile(a, T, vp, s_items, s_start, s_keep, g - tileBegin, numTiles, ld_agent(&Q.epoch), ld_agent(&Q.itemBegin),
                ld_agent(&Q.itemEnd), ld_agent(&Q.b0), ld_agent(&Q.b1), transY, &q->error);
     // completion: this tile's lists and counters are visible before it counts
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
@@ -569,9 +571,7 @@ __device__ __forceinline__ void xform4(const float* m, const float p[4], float o
 
 // instances_classify.comp.glsl:100-127 with culling.glsl:30-90 (frustum and
 // size test; there is no HiZ pyramid, so the occlusion test passes)
-__global__ void k_instances_classify(KArgs a) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.numInstances) return;
+__device__ void classify_instance(const KArgs& a, uint32_t i) {
   const tc_render_instance& inst = a.instances[i];
   const tc_frame_constants* vw = a.viewLast;  // culling.glsl reads viewLast
   float wvp[16];
@@ -617,6 +617,33 @@ __global__ void k_instances_classify(KArgs a) {
   const bool visible = inFrustum && (!clipValid || (sizeOk && hizOk));
   ptr<uint32_t>(a.build->instanceStates)[i] = (inFrustum ? TC_INSTANCE_FRUSTUM_BIT : 0u) | (visible ? TC_INSTANCE_VISIBLE_BIT : 0u);
   ptr<tc_blas_build_info>(a.build->blasBuildInfos)[i].clusterReferencesCount = 0;
+}
+
+__global__ void k_instances_classify(KArgs a) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < a.numInstances) classify_instance(a, i);
+}
+
+// First launch of the frame sequence.  Workgroup 0: build_setup CLASSIFY, the
+// classify prologue with the epochs and tickets of all stages, and split pass
+// 0 as a classify of no clusters leaves it.  The other workgroups (when the
+// sequence starts with them) classify the instances.
+__global__ __launch_bounds__(256) void k_frame_prologue(KArgs a, uint32_t numPasses) {
+  if (blockIdx.x != 0) {
+    const uint32_t i = (blockIdx.x - 1) * blockDim.x + threadIdx.x;
+    if (i < a.numInstances) classify_instance(a, i);
+    return;
+  }
+  WsHeader* h = a.ws;
+  if (threadIdx.x == 0) build_setup_one(a, TC_BUILD_SETUP_CLASSIFY);
+  if (threadIdx.x < 16) h->splitTicket[threadIdx.x] = 0;
+  if (threadIdx.x == 16) {
+    h->instTicket = 0;
+    const uint32_t split = min((uint32_t)a.build->splitTriangleCounter, a.cfg.maxSplitTriangles);
+    split_queue(h)->pass[0] = next_split_pass(a, 0, split, a.build->partTriangleCounter);
+  }
+  __syncthreads();
+  prologue_body(a, kStageClassify, numPasses + 1);
 }
 
 // clusters_cull.comp.glsl:112-161 in ray-tracing mode (every cluster of

@@ -583,9 +583,8 @@ static tc_status tessellate(tc_renderer* rr, const tc_frame_constants* frameHost
   if ((s = begin_frame(r, frameHost, (hipStream_t)stream, fetchView, listed)) != TC_OK) return s;
   tc_bindings b;
   tc_renderer_get_bindings(rr, &b);
-  if ((s = tc_instances_classify(&b, r->cfg, stream)) != TC_OK) return s;
   if (!listed && (s = tc_clusters_cull(&b, r->cfg, stream)) != TC_OK) return s;
-  return tc_frame_tessellate(&b, r->cfg, 0, stream);
+  return frame_tessellate_instances(&b, r->cfg, true, stream);
 }
 
 extern "C" {

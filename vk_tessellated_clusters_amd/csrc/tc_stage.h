@@ -112,4 +112,102 @@ __device__ __forceinline__ void add_blas_reference_counts(tc_blas_build_info* in
   }
 }
 
+// Parts that are instantiated: the accepted prefix of the list.  With
+// transient builds (build_setup.comp.glsl:240-253) x + y + 2 <=
+// MAX_PART_TRIANGLES of the lower counter x.
+__device__ __forceinline__ uint32_t accepted_parts(const KArgs& a) {
+  uint32_t cap = a.cfg.maxPartTriangles;
+  if (transient_builds(a.cfg.flags)) {
+    const uint32_t y = (uint32_t)(a.build->dualPartTriangleCounter >> 32);
+    cap = cap > y + 1 ? cap - y - 1 : 0u;
+  }
+  return min(a.build->partTriangleCounter, cap);
+}
+
+// build_setup.comp.glsl:102-264 (transient builds with TC_FLAG_1X_TRANSIENT
+// or TC_FLAG_2X_TRANSIENT).  One thread.
+__device__ __forceinline__ void build_setup_one(const KArgs& a, int mode) {
+  tc_scene_building* b = a.build;
+  tc_readback* rb = a.readback;
+  const tc_config& cfg = a.cfg;
+  if (mode == TC_BUILD_SETUP_CLASSIFY) {
+    uint32_t counter = b->visibleClusterCounter;
+    rb->numVisibleClusters = counter;
+    counter = min(counter, cfg.maxVisibleClusters);
+    b->visibleClusterCounter = counter;
+    b->dispatchClassify = tc_dispatch_indirect{counter, 1, 1};
+  } else if (mode == TC_BUILD_SETUP_DRAW_TESS) {
+    uint32_t full = b->fullClusterCounter, part = b->partTriangleCounter;
+    rb->numFullClusters = full;
+    rb->numPartTriangles = part;
+    rb->numSplitTriangles = b->splitWriteCounter;
+    full = min(full, cfg.maxVisibleClusters);
+    part = min(part, cfg.maxPartTriangles);
+    b->drawFullClusters = tc_draw_mesh_tasks_indirect{full, 0};
+    b->drawPartTriangles = tc_draw_mesh_tasks_indirect{(part + 31) / 32, 0};
+    rb->numBlasClusters = full;
+  } else if (mode == TC_BUILD_SETUP_SPLIT) {
+    uint32_t count = min((uint32_t)b->splitTriangleCounter, cfg.maxSplitTriangles);
+    b->splitWriteCounter = count;
+    b->splitTriangleCounter = (int32_t)count;
+    b->splitPassStart = 0;
+    b->splitPassEnd = count;
+    b->dispatchTriangleSplit = tc_dispatch_indirect{(count + 63) / 64, 1, 1};
+  } else if (mode == TC_BUILD_SETUP_SPLIT_PASS) {
+    b->splitPass = b->splitPass + 1;
+    uint32_t start = min(b->splitPassEnd, cfg.maxSplitTriangles);
+    uint32_t end = min(b->splitWriteCounter, cfg.maxSplitTriangles);
+    b->splitPassStart = start;
+    b->splitPassEnd = end;
+    b->dispatchTriangleSplit = tc_dispatch_indirect{(end - start + 63) / 64, 1, 1};
+  } else if (mode == TC_BUILD_SETUP_BUILD_BLAS) {
+    const bool trans = transient_builds(cfg.flags);
+    uint32_t temp = b->tempInstantiateCounter;
+    uint32_t tr = trans ? b->transBuildCounter : 0u;
+    rb->numBlasClusters = temp + tr;
+    if (trans) rb->numTransBuilds = tr;
+    rb->numTempInstantiations = temp;
+    rb->numGenDatas = b->genClusterDataCounter;
+    rb->numGenVertices = b->genVertexCounter;
+    rb->numBlasReservedSizes = b->numBlasReservedSizes;
+    temp = min(cfg.maxGeneratedClusters, temp);
+    b->tempInstantiateCounter = temp;
+    rb->numActualTempInstantiations = temp;
+    b->dispatchBlasTempInsert = tc_dispatch_indirect{(temp + 63) / 64, 1, 1};
+    if (trans) {
+      tr = min(cfg.maxGeneratedClusters, temp + tr) - temp;
+      b->transBuildCounter = tr;
+      rb->numActualTransBuilds = tr;
+      b->dispatchBlasTransInsert = tc_dispatch_indirect{(tr + 63) / 64, 1, 1};
+    }
+  } else if (mode == TC_BUILD_SETUP_INSTANTIATE_TESS) {
+    const uint32_t part = b->partTriangleCounter;
+    rb->numSplitTriangles = b->splitWriteCounter;
+    if (transient_builds(cfg.flags)) {
+      const uint32_t y = (uint32_t)(b->dualPartTriangleCounter >> 32);
+      rb->numPartTriangles = part + y;
+      rb->numTransPartTriangles = y;
+    } else {
+      rb->numPartTriangles = part;
+    }
+    const uint32_t ok = accepted_parts(a);
+    b->partTriangleCounter = ok;
+    b->dispatchTriangleInstantiate = tc_dispatch_indirect{(ok + 31) / 32, 1, 1};
+  }
+}
+
+// The split's setups of the frame sequence, once its passes are done:
+// SceneBuilding's split state as build_setup SPLIT and the SPLIT_PASSes leave
+// it.  One thread.
+__device__ __forceinline__ void split_state_one(const KArgs& a, uint32_t numPasses) {
+  tc_scene_building* b = a.build;
+  const SplitQueue* q = split_queue(a.ws);
+  const SplitPass first = q->pass[0], last = q->pass[numPasses - 1];
+  b->splitTriangleCounter = (int32_t)first.itemEnd;
+  b->splitPass = b->splitPass + numPasses - 1;
+  b->splitPassStart = last.itemBegin;
+  b->splitPassEnd = last.itemEnd;
+  b->dispatchTriangleSplit = tc_dispatch_indirect{(last.itemEnd - last.itemBegin + 63) / 64, 1, 1};
+}
+
 }  // namespace tc
