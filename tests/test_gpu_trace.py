@@ -400,3 +400,42 @@ def test_shared_leaf_steps_match_packets(layout, num):
     for h, d in got:
         assert np.array_equal(h.view(np.uint8), want[0].view(np.uint8))
         assert np.array_equal(d.view(np.uint8), want[1].view(np.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("num", [64, 1000])
+def test_ordered_and_general_slab_tests_agree(num):
+    """Waves of regular rays load a node's planes in the order the ray meets
+    them; a wave with a ray parallel to an axis, or with an origin that is not
+    finite, takes the general slab test.  Rays of all eight octants give the
+    same bytes both ways, and the irregular rays those of the packet traversal
+    (which has only the general test)."""
+    host = scene.scene_grid_instances(num_instances=4, quads=24, patch_size=8.0, tex_size=64, tess_rate_pixels=6.0)
+    rng = np.random.default_rng(num)
+    rays = np.zeros(num, abi.RAY_DT)
+    target = rng.uniform(1.0, 13.0, (num, 3)) * (1.0, 0.02, 1.0)
+    rays["direction"] = rng.choice([-1.0, 1.0], (num, 3)) * rng.uniform(0.1, 1.0, (num, 3))
+    rays["origin"] = target - 3.0 * rays["direction"]
+    rays["tMin"], rays["tMax"] = 0.0, 200.0
+    mixed = rays.copy()
+    odd = np.arange(0, num, 16)  # one or more in every wave
+    mixed["direction"][odd, 1] = np.where(odd % 32 == 0, -1.0, mixed["direction"][odd, 1])
+    mixed["direction"][odd[::2], 0] = 0.0
+    mixed["direction"][odd[::4], 2] = -0.0
+    mixed["origin"][odd[1::4], 1] = np.inf
+    mixed["origin"][odd[3::4], 0] = np.nan
+    g = harness.GpuFrame(host, harness.small_config())
+    try:
+        g.run(host.frame(), stages="accel")
+        regular, _ = g.trace(0, 0, 0, rays=rays)
+        general, _ = g.trace(0, 0, 0, rays=mixed)
+        packets = [g.trace(0, 0, abi.TRACE_PACKETS, rays=r)[0] for r in (rays, mixed)]
+    finally:
+        g.close()
+    if num == 1000:
+        assert (regular["t"] > 0).mean() > 0.3, "rays must meet the surface"
+    same = np.ones(num, bool)
+    same[odd] = False
+    assert np.array_equal(regular[same].view(np.uint8), general[same].view(np.uint8))
+    assert np.array_equal(regular.view(np.uint8), packets[0].view(np.uint8))
+    assert np.array_equal(general.view(np.uint8), packets[1].view(np.uint8))
