@@ -50,6 +50,33 @@ def test_hiz_build_matches_oracle(w, h, stride):
     assert L.tc_hiz_build(C.byref(abi.Hiz()), C.c_void_p(dev.data_ptr()), 4, None) == abi.TC_ERROR_INVALID_ARGUMENT
 
 
+@pytest.mark.parametrize("w,h", [(6, 6), (9, 6), (64, 64), (66, 40), (128, 127), (130, 130), (2050, 6), (7, 4097)])
+def test_hiz_tiles_match_oracle(w, h):
+    """Pyramids of 3 to 13 levels: smaller than, equal to and just above one
+    tile of 32 texels, and one, two and three launches of six levels, with
+    infinities and zeros of both signs; texels past the pyramid stay."""
+    import torch
+    print("case", w, h, flush=True)
+    rng = np.random.default_rng(w + h)
+    depth = (rng.random((h, w), np.float32) * 4.0 - 3.0).astype(np.float32)
+    depth[rng.random((h, w)) < 0.05] = np.inf
+    depth[rng.random((h, w)) < 0.05] = -np.inf
+    depth[rng.random((h, w)) < 0.05] = 0.0
+    hz, nbytes, _, _ = hiz_setup(w, h)
+    dev = torch.from_numpy(depth).cuda()
+    tex = torch.full((nbytes // 4 + 64,), -7.0, dtype=torch.float32, device="cuda")
+    hz.texels = tex.data_ptr()
+    abi.check(abi.lib().tc_hiz_build(C.byref(hz), C.c_void_p(dev.data_ptr()), 4, None), "tc_hiz_build")
+    torch.cuda.synchronize()
+    ref = np.zeros(nbytes // 4, np.float32)
+    hr = abi.Hiz.from_buffer_copy(hz)
+    hr.texels = ref.ctypes.data
+    oracle().oracle_hiz_build(C.byref(hr), depth.ctypes.data, 4)
+    got = tex.cpu().numpy()
+    assert np.array_equal(got[:nbytes // 4], ref)
+    assert (got[nbytes // 4:] == -7.0).all()
+
+
 def wall_scene(width=320, height=180):
     """A vertical wall 8 units in front of the camera and grid patches
     behind it (hidden), plus one patch in front of it (seen)."""
