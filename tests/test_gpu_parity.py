@@ -459,3 +459,49 @@ def test_frame_sequence_tiles(instances, quads, rate, flags):
         harness.compare(g.results(), ref)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("instances,flags,capacity", [
+    (1, 0, 0), (2, 0, 0), (256, 0, 0), (257, 0, 0), (600, 0, 0), (2, "trans", 0), (300, "trans", 0), (40, 0, 300),
+    (300, "trans", 600)])
+def test_insertion_with_keys_matches_stages(instances, flags, capacity):
+    """tc_renderer_build_accel inserts and sorts in one sort whose digit bases
+    come from the reference counts; the stage entry points (setup, insertion of
+    both lists, keys, sort) give the same lists, counts, totals and trees: one
+    and two instance digits and their borders, both CLAS lists, and a CLAS
+    capacity that cuts the frame."""
+    from test_gpu_trace import lattice_scene
+    host = lattice_scene(instances)
+    host.tess_rate_pixels /= 8.0  # eight parts a patch, or transient builds
+    over = {"maxGeneratedClusters": capacity} if capacity else {}
+    if flags:
+        over["flags"] = (abi.FLAG_DISPLACEMENT | abi.FLAG_CULLING | abi.FLAG_1X_TRANSIENT | abi.FLAG_2X_TRANSIENT)
+    g = harness.GpuFrame(host, harness.small_config(**over))
+    L = abi.lib()
+    out = []
+    try:
+        for staged in (False, True):
+            g.r.tessellate(host.frame())
+            if staged:
+                g.r.clas_and_blas()
+                accel, xforms = g.r.accel()
+                abi.check(L.tc_accel_build(C.byref(g.r.bindings), g.cfg, C.byref(accel), C.c_void_p(xforms), None),
+                          "tc_accel_build")
+            else:
+                g.r.build_accel()
+            abi.check(L.tc_device_synchronize(), "synchronize")
+            arr, rb = g.accel_arrays(), g.r.readback()
+            sb = arr["sb"]
+            keep = np.zeros(len(arr["blasNodes"]), bool)
+            for info in arr["infos"]:
+                first = int(info["clusterReferences"] - sb.blasClusterAddresses) // 8
+                keep[first:first + max(0, int(info["clusterReferencesCount"]) - 1)] = True
+            out.append([arr["refs"], arr["infos"], arr["blasLeaves"], arr["blasLeafInfo"], arr["blasNodes"][keep],
+                        arr["blasNodes4"][keep], arr["tlasNodes"][:instances - 1], arr["tlasInstances"],
+                        np.array([sb.blasClusterCounter, sb.tempInstantiateCounter, sb.transBuildCounter,
+                                  rb.numBlasActualSizes, rb.numGenActualDatas])])
+    finally:
+        g.close()
+    assert out[0][8][0] >= (capacity or instances) and bool(flags) == (out[0][8][2] > 0)
+    for x, y in zip(*out):
+        assert x.tobytes() == y.tobytes()

@@ -50,6 +50,24 @@ struct AccelLayout {
   uint64_t total;
 };
 
+// 24-bit Morton code (8 bits per axis) of the box centre, normalised to
+// [lo, hi]: the BLAS key below the instance, three radix digits
+__device__ __forceinline__ uint32_t morton24_of(const float* blo, const float* bhi, const float* lo, const float* hi) {
+  uint32_t code = 0;
+  for (int k = 0; k < 3; k++) {
+    const float c = (blo[k] + bhi[k]) * 0.5f;
+    const float ext = hi[k] - lo[k];
+    float n = ext > 0.0f ? (c - lo[k]) / ext : 0.5f;
+    n = fminf(fmaxf(n, 0.0f), 1.0f);
+    uint32_t q = (uint32_t)(n * 255.0f + 0.5f);
+    q = (q | (q << 8)) & 0x0300F00Fu;
+    q = (q | (q << 4)) & 0x030C30C3u;
+    q = (q | (q << 2)) & 0x09249249u;
+    code |= q << k;
+  }
+  return code;
+}
+
 AccelLayout accel_layout(uint32_t capacity, uint32_t numInstances);
 
 }  // namespace tc

@@ -19,6 +19,7 @@
 #include <algorithm>
 
 #include "tc_bvh.h"
+#include "tc_insert.h"
 
 namespace tc {
 
@@ -41,24 +42,6 @@ __host__ __device__ __forceinline__ uint32_t morton_of(const float* blo, const f
     n = fminf(fmaxf(n, 0.0f), 1.0f);
     uint32_t q = (uint32_t)(n * 1023.0f + 0.5f);
     q = (q | (q << 16)) & 0x030000FFu;
-    q = (q | (q << 8)) & 0x0300F00Fu;
-    q = (q | (q << 4)) & 0x030C30C3u;
-    q = (q | (q << 2)) & 0x09249249u;
-    code |= q << k;
-  }
-  return code;
-}
-
-// 24-bit Morton code (8 bits per axis) of the box centre, normalised to
-// [lo, hi]: the BLAS key below the instance, three radix digits
-__device__ __forceinline__ uint32_t morton24_of(const float* blo, const float* bhi, const float* lo, const float* hi) {
-  uint32_t code = 0;
-  for (int k = 0; k < 3; k++) {
-    const float c = (blo[k] + bhi[k]) * 0.5f;
-    const float ext = hi[k] - lo[k];
-    float n = ext > 0.0f ? (c - lo[k]) / ext : 0.5f;
-    n = fminf(fmaxf(n, 0.0f), 1.0f);
-    uint32_t q = (uint32_t)(n * 255.0f + 0.5f);
     q = (q | (q << 8)) & 0x0300F00Fu;
     q = (q | (q << 4)) & 0x030C30C3u;
     q = (q | (q << 2)) & 0x09249249u;
@@ -826,8 +809,11 @@ tc_status tc_accel_bind(void* memory, uint64_t bytes, uint32_t capacity, uint32_
   return TC_OK;
 }
 
-tc_status tc_accel_build(const tc_bindings* b, tc_config config, const tc_accel* accel, const float* instanceXforms,
-                         tc_stream stream) {
+}  // extern "C"
+
+// `inserted`: the keys and the digit counts are those insert_clusters left.
+static tc_status accel_build(const tc_bindings* b, tc_config config, const tc_accel* accel, const float* instanceXforms,
+                             tc_stream stream, bool inserted) {
   KArgs ka;
   tc_status s = make_args_public(b, config, ka);
   if (s != TC_OK) return s;
@@ -881,12 +867,13 @@ tc_status tc_accel_build(const tc_bindings* b, tc_config config, const tc_accel*
 
   const uint32_t grid = std::min<uint32_t>((capacity + 255) / 256, (uint32_t)num_cu_public() * tuning_snapshot().bvhBlocksPerCU);
   // BLAS: keys, sort by (instance, Morton), hierarchy, refit
-  hipLaunchKernelGGL(k_blas_keys, dim3(grid), dim3(256), 0, st, a);
-  uint32_t instBits = 1;
-  while ((1u << instBits) < a.numInstances) instBits++;
+  if (!inserted) hipLaunchKernelGGL(k_blas_keys, dim3(grid), dim3(256), 0, st, a);
   uint32_t res = 0;
-  // digits 0-2: the 24-bit Morton code; digits 4-5: the instance
-  radix_sort_digits(sb, &b->build->blasClusterCounter, 0x7u | (instBits > 8 ? 0x30u : 0x10u), st, &res);
+  // digits 0-2: the 24-bit Morton code; digits 4-5: the instance, where there
+  // is more than one
+  const InsertPlan ip = insert_plan(b, config);
+  radix_sort_digits(sb, &b->build->blasClusterCounter, 0x7u | ((1u << ip.instancePasses) - 1u) << 4, st, &res,
+                    inserted ? ip.insertPasses : 0);
   a.sortedKeys = sb.keys[res];
   a.sortedVals = sb.vals[res];
   hipLaunchKernelGGL(k_blas_hierarchy, dim3(grid), dim3(256), 0, st, a);
@@ -924,4 +911,12 @@ tc_status tc_accel_build(const tc_bindings* b, tc_config config, const tc_accel*
   return hipGetLastError() == hipSuccess ? TC_OK : TC_ERROR_LAUNCH;
 }
 
-}  // extern "C"
+tc_status tc::accel_build_inserted(const tc_bindings* b, tc_config config, const tc_accel* accel, const float* instanceXforms,
+                                   tc_stream stream) {
+  return accel_build(b, config, accel, instanceXforms, stream, true);
+}
+
+extern "C" tc_status tc_accel_build(const tc_bindings* b, tc_config config, const tc_accel* accel, const float* instanceXforms,
+                                    tc_stream stream) {
+  return accel_build(b, config, accel, instanceXforms, stream, false);
+}

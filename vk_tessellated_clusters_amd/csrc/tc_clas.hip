@@ -13,6 +13,8 @@
 #include <algorithm>
 
 #include "tc_kernels.h"
+#include "tc_bvh.h"
+#include "tc_insert.h"
 
 namespace tc {
 
@@ -31,13 +33,13 @@ __host__ __device__ __forceinline__ uint32_t r16(uint32_t v) { return (v + 15u) 
 
 // Group boxes and header of a block whose triangle words (s_t) and
 // vertices (s_v) are in LDS and already copied to the block; returns the
-// block size.  One wave.
+// block size and the block's box.  One wave.
 __device__ __forceinline__ uint32_t finish_block(char* dst, const float* s_v, const uint32_t* s_t, uint32_t nt, uint32_t nv,
-                                                 uint32_t clusterID, uint32_t vertexBase) {
+                                                 uint32_t clusterID, uint32_t vertexBase, float lo[3], float hi[3]) {
   const uint32_t lane = lane_id();
   const uint32_t ng = (nt + TC_CLAS_GROUP_TRIANGLES - 1) / TC_CLAS_GROUP_TRIANGLES;
   tc_aabb* groups = reinterpret_cast<tc_aabb*>(dst + sizeof(tc_clas_header));
-  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  for (int c = 0; c < 3; c++) lo[c] = INFINITY, hi[c] = -INFINITY;
   for (uint32_t g = lane; g < ng; g += kWave) {
     float glo[3] = {INFINITY, INFINITY, INFINITY}, ghi[3] = {-INFINITY, -INFINITY, -INFINITY};
     const uint32_t t1 = min(nt, (g + 1) * TC_CLAS_GROUP_TRIANGLES);
@@ -173,24 +175,33 @@ __device__ __forceinline__ uint64_t u64(uint32_t lo, uint32_t hi) { return ((uin
 // Runs of records, grid-stride over tempInstantiateCounter; a frame with
 // fewer than kBatch records for each of the chip's resident waves takes
 // shorter runs (8192 records in runs of 1 on 40 waves a CU: 14 us, of 2 on 16
-// waves: 9.5 us).
-__global__ __launch_bounds__(kClasWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_clas_instantiate(KArgs a, uint32_t residentWaves) {
+// waves: 9.5 us).  With an insertion plan, one workgroup more makes its setup
+// and every record's Morton code is left for its keys.
+__global__ __launch_bounds__(kClasWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_clas_instantiate(KArgs a, uint32_t residentWaves, InsertPlan ip) {
   __shared__ ClasWave s_wave[kClasWaves];
+  if (ip.state && blockIdx.x == 0) {
+    static_assert(kClasWaves * kWave == kSortThreads && sizeof(s_wave) >= 4 * kInsertSetupWords, "setup workgroup");
+    insert_setup(a, ip, reinterpret_cast<uint32_t*>(s_wave));
+    return;
+  }
+  const uint32_t group = blockIdx.x - (ip.state ? 1 : 0), groups = gridDim.x - (ip.state ? 1 : 0);
   const tc_scene_building* b = a.build;
   const uint32_t n = min(b->tempInstantiateCounter, a.cfg.maxGeneratedClusters);
   const uint32_t lane = lane_id();
   ClasWave& w = s_wave[threadIdx.x / kWave];
   const tc_template_instantiate_info* infos = ptr<const tc_template_instantiate_info>(b->tempInstantiations);
   const uint64_t* dsts = ptr<const uint64_t>(b->tempClusterAddresses);
+  const uint32_t* instances = ptr<const uint32_t>(b->tempInstanceIDs);
   uint32_t* sizes = ptr<uint32_t>(b->tempClusterSizes);
-  const uint32_t waves = gridDim.x * kClasWaves;
+  const uint32_t waves = groups * kClasWaves;
   const uint32_t run = min(kBatch, max(1u, (n + residentWaves - 1) / residentWaves));
-  for (uint32_t r0 = uniform(blockIdx.x * kClasWaves + threadIdx.x / kWave) * run; r0 < n; r0 += waves * run) {
+  for (uint32_t r0 = uniform(group * kClasWaves + threadIdx.x / kWave) * run; r0 < n; r0 += waves * run) {
     const uint32_t cnt = min(run, n - r0);
     // lanes 0 .. cnt - 1 hold the run's records
     const bool held = lane < cnt;
     uint64_t dst = 0, src = 0, words = 0;
     uint32_t stride = 12, nv = 0, nt = 0, clusterID = 0;
+    float geo[6], box[6];  // of the lane's record: instance bounds, CLAS
     if (held) {
       const tc_template_instantiate_info info = gld_record(infos + r0 + lane);
       dst = gld(dsts + r0 + lane);
@@ -201,6 +212,11 @@ __global__ __launch_bounds__(kClasWaves * kWave) __attribute__((amdgpu_waves_per
       nv = min(T.numVertices, kMaxClusterVerts);
       nt = min(T.numTriangles, kMaxTemplateTris);
       clusterID = T.clusterID + info.clusterIdOffset;
+      if (ip.state) {
+        const tc_render_instance& ri = a.instances[gld(instances + r0 + lane)];
+#pragma unroll
+        for (int x = 0; x < 3; x++) geo[x] = gld(ri.geoLo + x), geo[3 + x] = gld(ri.geoHi + x);
+      }
     }
     const uint32_t ng = (nt + TC_CLAS_GROUP_TRIANGLES - 1) / TC_CLAS_GROUP_TRIANGLES;
     const uint32_t oT = (uint32_t)sizeof(tc_clas_header) + r16(ng * 24u), oV = oT + r16(nt * 4u), size = oV + r16(nv * 12u);
@@ -343,7 +359,14 @@ __global__ __launch_bounds__(kClasWaves * kWave) __attribute__((amdgpu_waves_per
                     "the header as three chunks");
       wave_sync();
       // the image to memory, 1 KB a step
-      if (in) gst(sizes + r0 + lane, size);
+      if (in) {
+        gst(sizes + r0 + lane, size);
+        if (ip.state) {
+          const float* h = w.f + 4 * (w.head[lane].y & 0xFFFF);
+#pragma unroll
+          for (int x = 0; x < 3; x++) box[x] = h[x], box[3 + x] = h[4 + x];
+        }
+      }
       {
         uint32_t before = done;
 #pragma unroll
@@ -361,6 +384,7 @@ __global__ __launch_bounds__(kClasWaves * kWave) __attribute__((amdgpu_waves_per
       wave_sync();
       done += k;
     }
+    if (ip.state && held) gst(ip.codes + r0 + lane, morton24_of(box, box + 3, geo, geo + 3));
   }
 }
 
@@ -370,8 +394,9 @@ constexpr uint32_t kWaveTrisPerLane = (kMaxClusterTris + kWave - 1) / kWave;
 // Transient builds (stands for the NV transient CLAS build,
 // renderer_raytrace_clusters_tess.cpp:625-655): triangles in record order
 // with the transient triangle index as primitive, all the record's
-// vertices.  One wave per CLAS, grid-stride over transBuildCounter.
-__global__ __launch_bounds__(64) void k_clas_build_transient(KArgs a) {
+// vertices.  One wave per CLAS, grid-stride over transBuildCounter.  With
+// `codes`, as k_clas_instantiate.
+__global__ __launch_bounds__(64) void k_clas_build_transient(KArgs a, uint32_t* codes) {
   __shared__ float s_v[kMaxClusterVerts * 3];
   __shared__ uint32_t s_t[kMaxClusterTris];
   const tc_scene_building* b = a.build;
@@ -430,8 +455,14 @@ __global__ __launch_bounds__(64) void k_clas_build_transient(KArgs a) {
       }
     }
     __syncthreads();
-    const uint32_t size = finish_block(dst, s_v, s_t, nt, nv, info.clusterID, vertex_base(b, info.vertexBuffer));
+    float lo[3], hi[3];
+    const uint32_t size = finish_block(dst, s_v, s_t, nt, nv, info.clusterID, vertex_base(b, info.vertexBuffer), lo, hi);
     if (lane == 0) gst(sizes + i, size);
+    if (codes && lane == 0) {
+      const tc_render_instance& ri = a.instances[gld(ptr<const uint32_t>(b->transInstanceIDs) + i)];
+      const uint32_t numTemp = min(b->tempInstantiateCounter, a.cfg.maxGeneratedClusters);
+      if (numTemp + i < a.cfg.maxGeneratedClusters) gst(codes + numTemp + i, morton24_of(lo, hi, ri.geoLo, ri.geoHi));
+    }
     __syncthreads();
   }
 }
@@ -440,24 +471,39 @@ __global__ __launch_bounds__(64) void k_clas_build_transient(KArgs a) {
 
 using namespace tc;
 
-extern "C" tc_status tc_clas_instantiate(const tc_bindings* b, tc_config config, tc_stream stream) {
+static tc_status launch_clas(const tc_bindings* b, tc_config config, tc_stream stream, const InsertPlan& ip) {
   KArgs a;
   tc_status s = make_args_public(b, config, a);
   if (s != TC_OK) return s;
   const uint32_t waves = std::min<uint32_t>((config.maxGeneratedClusters + 3) / 4,
                                             (uint32_t)num_cu_public() * tuning_snapshot().clasWavesPerCU);
   const uint32_t grid = (waves + kClasWaves - 1) / kClasWaves;
-  hipLaunchKernelGGL(k_clas_instantiate, dim3(grid), dim3(kClasWaves * kWave), 0, (hipStream_t)stream, a,
-                     (uint32_t)num_cu_public() * kClasResident);
+  hipLaunchKernelGGL(k_clas_instantiate, dim3(grid + (ip.state ? 1 : 0)), dim3(kClasWaves * kWave), 0, (hipStream_t)stream, a,
+                     (uint32_t)num_cu_public() * kClasResident, ip);
   return hipGetLastError() == hipSuccess ? TC_OK : TC_ERROR_LAUNCH;
 }
 
-extern "C" tc_status tc_clas_build_transient(const tc_bindings* b, tc_config config, tc_stream stream) {
+extern "C" tc_status tc_clas_instantiate(const tc_bindings* b, tc_config config, tc_stream stream) {
+  return launch_clas(b, config, stream, InsertPlan{});
+}
+
+static tc_status launch_transient(const tc_bindings* b, tc_config config, tc_stream stream, uint32_t* codes) {
   KArgs a;
   tc_status s = make_args_public(b, config, a);
   if (s != TC_OK) return s;
   if (!transient_builds(config.flags)) return TC_OK;
   uint32_t grid = std::min<uint32_t>(config.maxGeneratedClusters, (uint32_t)num_cu_public() * tuning_snapshot().clasWavesPerCU);
-  hipLaunchKernelGGL(k_clas_build_transient, dim3(grid), dim3(64), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(k_clas_build_transient, dim3(grid), dim3(64), 0, (hipStream_t)stream, a, codes);
   return hipGetLastError() == hipSuccess ? TC_OK : TC_ERROR_LAUNCH;
+}
+
+extern "C" tc_status tc_clas_build_transient(const tc_bindings* b, tc_config config, tc_stream stream) {
+  return launch_transient(b, config, stream, nullptr);
+}
+
+tc_status tc::clas_build_setup(const tc_bindings* b, tc_config config, tc_stream stream) {
+  if (!b || !b->workspace) return TC_ERROR_INVALID_ARGUMENT;
+  const InsertPlan ip = insert_plan(b, config);
+  const tc_status s = launch_clas(b, config, stream, ip);
+  return s != TC_OK ? s : launch_transient(b, config, stream, ip.codes);
 }

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "tc_kernels.h"
+#include "tc_insert.h"
 #include "tc_trace.h"
 
 namespace tc {
@@ -444,12 +445,9 @@ tc_status tc_renderer_build_accel(tc_renderer* rr, tc_stream stream) {
   tc_bindings b;
   tc_renderer_get_bindings(rr, &b);
   tc_status s;
-  if ((s = tc_clas_instantiate(&b, r->cfg, stream)) != TC_OK) return s;
-  if ((s = tc_clas_build_transient(&b, r->cfg, stream)) != TC_OK) return s;
-  if ((s = tc_blas_setup_insertion(&b, r->cfg, stream)) != TC_OK) return s;
-  if ((s = tc_blas_clusters_insert(&b, r->cfg, 0, stream)) != TC_OK) return s;
-  if ((s = tc_blas_clusters_insert(&b, r->cfg, 1, stream)) != TC_OK) return s;
-  return tc_accel_build(&b, r->cfg, &r->accel, r->xforms, stream);
+  if ((s = tc::clas_build_setup(&b, r->cfg, stream)) != TC_OK) return s;
+  if ((s = tc::insert_clusters(&b, r->cfg, stream)) != TC_OK) return s;
+  return tc::accel_build_inserted(&b, r->cfg, &r->accel, r->xforms, stream);
 }
 
 tc_status tc_renderer_trace(tc_renderer* rr, const tc_trace_params* params, tc_stream stream) {

@@ -1,6 +1,8 @@
 // tc_sort.h -- device radix sort and BLAS insertion kernels.
 #pragma once
 
+#include <algorithm>
+
 #include "tc_kernels.h"
 
 namespace tc {
@@ -37,9 +39,16 @@ void radix_sort_pairs(const SortBuffers& sb, const uint32_t* count, uint32_t bit
                       uint32_t* outIndex, const uint64_t* listField = nullptr);
 // The same over the 8-bit digits named by digitMask (bit d: key bits
 // [8d, 8d + 8)), lowest digit first; digits where every key agrees may be
-// left out.
+// left out.  pass0: the state's first pass for them, when something other than
+// an upsweep (0) has set the state up.
 void radix_sort_digits(const SortBuffers& sb, const uint32_t* count, uint32_t digitMask, hipStream_t stream,
-                       uint32_t* outIndex);
+                       uint32_t* outIndex, uint32_t pass0 = 0);
+
+// First epoch of the sort that follows state epoch `last` with P passes.
+__device__ __forceinline__ uint32_t sort_epoch0(uint32_t last, uint32_t P) {
+  const uint32_t e0 = last + 1;
+  return e0 + P > (1u << kEpochBits) ? 1u : e0;
+}
 
 __global__ void k_insert_seg_start(KArgs a, const uint64_t* keys, uint32_t* segStart, uint32_t capacity, int transient);
 __global__ void k_insert_scatter(KArgs a, const uint64_t* keys, const uint32_t* vals, const uint32_t* segStart,
