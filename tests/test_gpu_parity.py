@@ -505,3 +505,31 @@ def test_insertion_with_keys_matches_stages(instances, flags, capacity):
     assert out[0][8][0] >= (capacity or instances) and bool(flags) == (out[0][8][2] > 0)
     for x, y in zip(*out):
         assert x.tobytes() == y.tobytes()
+
+
+@pytest.mark.parametrize("fmt", ["r16", "r32"])
+@pytest.mark.parametrize("w,h", [(1, 1), (2, 1), (1, 3), (2, 2), (3, 5), (64, 7)])
+def test_height_map_edges(w, h, fmt):
+    """Samples across a height map's edges wrap texel by texel; waves whose
+    samples all lie inside read a row's two texels in one load.  Maps of one
+    and two texels (every sample wraps, or one in nine does not), odd sizes and
+    both formats against the oracle's vertices."""
+    rng = np.random.default_rng(10 * w + h)
+    heights = rng.random((h, w), np.float32)
+    tex = (scene.to_r16(heights), abi.TEXTURE_R16_UNORM) if fmt == "r16" else (heights, abi.TEXTURE_R32_FLOAT)
+    geo = scene.grid_patch(12, 12, 4.0, 4.0)
+    cam = scene.Camera(eye=(2.0, 3.0, -1.0), center=(2.0, 0.0, 2.0), width=160, height=90, near=0.05, far=100.0)
+    host = scene.HostScene([geo], [scene.Instance(0, np.eye(4), displacement_index=0, displacement_scale=0.3)], [tex], cam,
+                           3.0, "edges")
+    cfg = harness.small_config()
+    of = harness.OracleFrame(host, cfg)
+    of.run(host.frame())
+    ref = of.results()
+    g = harness.GpuFrame(host, cfg)
+    try:
+        g.run(host.frame())
+        res = g.results()
+    finally:
+        g.close()
+    assert ref.counters["partTriangleCounter"] > 100
+    harness.compare(res, ref)
