@@ -439,3 +439,23 @@ def test_ordered_and_general_slab_tests_agree(num):
     assert np.array_equal(regular[same].view(np.uint8), general[same].view(np.uint8))
     assert np.array_equal(regular.view(np.uint8), packets[0].view(np.uint8))
     assert np.array_equal(general.view(np.uint8), packets[1].view(np.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,height", [(1, 1), (33, 17), (96, 54), (160, 90), (250, 130), (320, 180), (408, 224), (640, 360)])
+def test_small_images_share_tiles(width, height):
+    """Small images deal a tile's rays over 16, 8, 4, 2 or one wave; hits and
+    decoded hits are those of the packet traversal (one wave a tile) byte for
+    byte, each pixel written once."""
+    host = scene.scene_grid_instances(num_instances=4, quads=24, patch_size=8.0, tex_size=64, tess_rate_pixels=6.0)
+    g = harness.GpuFrame(host, harness.small_config())
+    flags = abi.TRACE_CULL_BACK | abi.TRACE_SHADOW
+    try:
+        g.run(host.frame(), stages="accel")
+        gh, gd = g.trace(width, height, flags)
+        ph, pd = g.trace(width, height, flags | abi.TRACE_PACKETS)
+    finally:
+        g.close()
+    assert width < 96 or (ph["t"] > 0).mean() > 0.2, "camera must see geometry"
+    assert np.array_equal(gh.view(np.uint8), ph.view(np.uint8))
+    assert np.array_equal(gd.view(np.uint8), pd.view(np.uint8))

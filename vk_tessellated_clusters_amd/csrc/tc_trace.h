@@ -66,6 +66,7 @@ struct TraceArgs {
   tc_hit_decoded* decoded;
   uint32_t* hitVertices;
   TraceOrder* order;  // camera traces of a renderer, else null
+  uint32_t share;     // waves that share a tile's (or 64 explicit) rays, as a power of two
   uint32_t nodes32;   // nodes lie within 4 GB of their arrays' starts
 };
 

@@ -1015,7 +1015,26 @@ __device__ void decode_hit(const TraceArgs& a, const HitState& hs, tc_hit_decode
   out.depth = pp[2] / pp[3];
 }
 
-// One ray per lane, 64 rays per wave.  The primary and the shadow walk are
+// Waves a tile's (or 64 explicit rays') rays are dealt over, as a power of two.
+// A launch that leaves most of the chip's waves empty takes as long as its
+// longest wave, which visits the nodes of all its rays: with fewer rays a wave
+// that chain is shorter, and the leaf steps use the idle lanes all the same.
+// While the shared waves are resident together (16 a CU; 6 for explicit rays,
+// which also come in parallel bundles that want whole waves), down to four
+// rays a wave.  Camera rays at 160 x 90 / 320 x 180 / 480 x 270: 500 meshes 600 ->
+// 210, 595 -> 385, 648 -> 512 us, icosphere 124 -> 117, 132 -> 117, 142 -> 133,
+// but past that 640 x 360 150 -> 156 and 960 x 540 191 -> 227; 16384 vertical rays
+// onto whole clusters 12.4 -> 10.2 us and onto parts 26 -> 18, 65536 of them
+// 13.6 -> 14.9 and 28 -> 25.
+constexpr uint32_t kMaxShare = 4;
+static uint32_t tile_share(uint32_t waves, bool rays) {
+  const uint64_t limit = (uint64_t)num_cu_public() * (rays ? 6u : 16u);
+  uint32_t s = 0;
+  while (s < kMaxShare && ((uint64_t)waves << (s + 1)) <= limit) s++;
+  return s;
+}
+
+// One ray per lane, up to 64 rays per wave.  The primary and the shadow walk are
 // two rounds of one loop, so the traversal is one piece of code in the
 // instruction cache.  A wave's lanes stay together through both: lanes without
 // a ray (ragged tiles, rays past the end, misses in the shadow round) help in
@@ -1039,15 +1058,15 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 8))) void 
   TraceOrder* ord = !a.rays && a.order && tilesY <= kMaxOrderRows ? a.order : nullptr;
   const uint32_t* rowOrder = ord && ord->rows == tilesY ? ord->order : nullptr;
   if (ord && blockIdx.x == 0 && threadIdx.x == 0) ord->pendingRows = tilesY;
-  const uint32_t waves = gridDim.x * (T / kWave), numWaves = (a.numItems + kWave - 1) / kWave;
+  const uint32_t waves = gridDim.x * (T / kWave), perWave = kWave >> a.share, numWaves = (a.numItems + perWave - 1) / perWave;
   for (uint32_t wave = uniform(blockIdx.x * (T / kWave) + threadIdx.x / kWave); wave < numWaves; wave += waves) {
     const uint64_t t0 = ord ? __builtin_amdgcn_s_memrealtime() : 0;
     float o[3] = {0.f, 0.f, 0.f}, d[3] = {0.f, 0.f, 1.f}, tmin = 0.f, tmax = 0.f;
     bool live = false;
     uint32_t r = 0, timedRow = 0;
     if (a.rays) {
-      r = wave * kWave + lane;
-      live = r < a.numItems;
+      r = wave * perWave + lane;
+      live = lane < perWave && r < a.numItems;
       if (live) {
         const tc_ray ray = a.rays[r];
         for (int k = 0; k < 3; k++) o[k] = ray.origin[k], d[k] = ray.direction[k];
@@ -1056,10 +1075,13 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 8))) void 
       }
     } else {
       uint32_t tx, ty;
-      if (!strip_tile(wave, T / kWave, tilesX, tilesY, rowOrder, tx, ty)) continue;
+      // the waves that share a tile are eight workgroups apart, on one XCD
+      const uint32_t group = wave / (T / kWave), turn = group / kXcds, part = turn & ((1u << a.share) - 1u);
+      const uint32_t tile = ((turn >> a.share) * kXcds + group % kXcds) * (T / kWave) + wave % (T / kWave);
+      if (!strip_tile(tile, T / kWave, tilesX, tilesY, rowOrder, tx, ty)) continue;
       timedRow = ty;
-      const uint32_t x = tx * 8 + (lane & 7), y = ty * 8 + (lane >> 3);
-      live = x < a.width && y < a.height;
+      const uint32_t in = part * perWave + lane, x = tx * 8 + (in & 7), y = ty * 8 + (in >> 3);
+      live = lane < perWave && x < a.width && y < a.height;
       if (live) {
         r = y * a.width + x;
         primary_ray(a.view, x, y, a.width, a.height, o, d);
@@ -1216,7 +1238,8 @@ tc_status tc::trace_rays(const tc_bindings* b, tc_config config, const tc_accel*
   const tc_tuning tn = tuning_snapshot();
   const uint32_t T = tn.traceThreads;
   a.numItems = p->rays ? p->numRays : strip_waves((p->width + 7) / 8, (p->height + 7) / 8, T / kWave) * kWave;
-  const uint32_t grid = std::min<uint32_t>((a.numItems + T - 1) / T, (uint32_t)num_cu_public() * tn.traceBlocksPerCU);
+  a.share = (a.flags & TC_TRACE_PACKETS) ? 0u : tile_share((a.numItems + kWave - 1) / kWave, p->rays != nullptr);
+  const uint32_t grid = std::min<uint32_t>((((uint64_t)a.numItems << a.share) + T - 1) / T, (uint32_t)num_cu_public() * tn.traceBlocksPerCU);
   // resident waves: four per SIMD (128 VGPRs), four SIMDs per CU
   if ((uint64_t)grid * (T / kWave) > (uint64_t)kOrderRounds * num_cu_public() * 16u) a.order = nullptr;
   if (a.flags & TC_TRACE_PACKETS) {
