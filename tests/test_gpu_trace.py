@@ -459,3 +459,58 @@ def test_small_images_share_tiles(width, height):
     assert width < 96 or (ph["t"] > 0).mean() > 0.2, "camera must see geometry"
     assert np.array_equal(gh.view(np.uint8), ph.view(np.uint8))
     assert np.array_equal(gd.view(np.uint8), pd.view(np.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qx,qz,px", [(31, 16, 20.0), (40, 30, 20.0), (120, 90, 3.0), (760, 400, 0.7)])
+def test_refit_of_one_instance(qx, qz, px):
+    """Boxes and four-wide records of one instance whose leaves lie in one
+    chunk of the refit, in three, in about twenty (climbs meet in LDS) and in
+    more than 512 (in global memory): every node's boxes are its children's
+    (the leaves' from their CLAS headers), checked in whole arrays, and the
+    four-wide records of the first and of random nodes list the grandchildren."""
+    geo = scene.grid_patch(qx, qz, 76.0, 40.0)
+    cam = scene.Camera(eye=(38.0, 60.0, 19.0), center=(38.0, 0.0, 20.0), width=1920, height=1080, near=0.1, far=500.0)
+    host = scene.HostScene([geo], [scene.Instance(0, np.eye(4))], [], cam, px, "one")
+    tris = 2 * qx * qz
+    cfg = harness.small_config(maxPartTriangles=tris + 1024, maxGeneratedClusters=tris + 32768,
+                               maxGeneratedVertices=12 * tris + (1 << 16))
+    g = harness.GpuFrame(host, cfg)
+    try:
+        g.run(host.frame(), stages="accel")
+        arr = g.accel_arrays()
+        sb = arr["sb"]
+        n = int(arr["infos"][0]["clusterReferencesCount"])
+        off = (arr["blasLeaves"][:n] - np.uint64(sb.genClusterData)).astype(np.int64)
+        pool = g.r.copy(sb.genClusterData, int(off.max()) + 48).view(np.float32)
+    finally:
+        g.close()
+    print("CLAS", n, flush=True)
+    assert n > 0.9 * tris
+    nodes, wide = arr["blasNodes"][:n - 1], arr["blasNodes4"][:n - 1]
+    h = pool[(off // 4)[:, None] + np.arange(8)]
+    leaf_lo, leaf_hi = h[:, 0:3], h[:, 4:7]
+    lo = np.minimum(nodes["lo0"], nodes["lo1"])
+    hi = np.maximum(nodes["hi0"], nodes["hi1"])
+    seen = np.zeros(2 * n, np.int64)
+    for c in ("0", "1"):
+        word = nodes["child" + c]
+        leaf = (word & abi.BVH_LEAF) != 0
+        at = (word & ~np.uint32(abi.BVH_LEAF)).astype(np.int64)
+        want_lo = np.where(leaf[:, None], leaf_lo[np.where(leaf, at, 0)], lo[np.where(leaf, 0, at)])
+        want_hi = np.where(leaf[:, None], leaf_hi[np.where(leaf, at, 0)], hi[np.where(leaf, 0, at)])
+        assert np.array_equal(nodes["lo" + c], want_lo) and np.array_equal(nodes["hi" + c], want_hi)
+        np.add.at(seen, np.where(leaf, n + at, at), 1)
+    assert seen[0] == 0 and (seen[1:n - 1] == 1).all() and (seen[n:] == 1).all()
+    rng = np.random.default_rng(n)
+    for i in [0, *rng.integers(0, n - 1, 2000)]:
+        nd, want = nodes[i], []
+        for c in ("0", "1"):
+            ch = int(nd["child" + c])
+            if ch & abi.BVH_LEAF:
+                want.append((ch, tuple(nd["lo" + c]), tuple(nd["hi" + c])))
+            else:
+                want += [(int(nodes[ch]["child" + d]), tuple(nodes[ch]["lo" + d]), tuple(nodes[ch]["hi" + d])) for d in "01"]
+        got = [(int(wide[i]["child"][k]), tuple(wide[i]["lo"][:, k]), tuple(wide[i]["hi"][:, k])) for k in range(len(want))]
+        assert got == want
+        assert all(int(wide[i]["child"][k]) == abi.BVH4_EMPTY for k in range(len(want), 4))

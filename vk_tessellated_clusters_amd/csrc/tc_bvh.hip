@@ -261,54 +261,57 @@ __device__ __forceinline__ void collapse4(const tc_bvh_node* nodes, uint32_t i, 
 // climb waits on no global load.  A climb stops at the first node whose
 // range straddles chunks; the second arrival there lists the node as
 // pending for its instance (both children are then final).  The chunk's
-// four-wide records are written from LDS once every climb is done.
+// binary and four-wide records are written from LDS once every climb is done.
+// It moves about 290 bytes a CLAS (3.0 TB/s at 3.3 million) and took as long as
+// its waits: with 66 registers one workgroup of 16 waves filled a CU, with 54
+// two share it.  3.3 million CLAS 365 -> 304 us, 310,000 46.9 -> 39.8 us.
 //
 // k_blas_refit_top: one workgroup per instance climbs from its pending
-// nodes through the straddling nodes with global counters (continuing the
-// counts of the first launch) and workgroup-scope ordering, since every
-// climber of an instance is in that workgroup; each node's four-wide
-// record is written where the node is refit.  A pending node's range
-// holds exactly one chunk boundary (its split), so an instance has fewer
-// pending nodes than chunks it spans; its list starts at
-// (first >> kRefitChunkBits) + instance.
+// nodes through the straddling nodes; each node's records are written where
+// the node is refit.  A pending node's range holds exactly one chunk boundary
+// (its split), so an instance has fewer pending nodes than chunks it spans;
+// its list starts at (first >> kRefitChunkBits) + instance.
 constexpr uint32_t kRefitChunkBits = 10;
 constexpr uint32_t kRefitChunk = 1u << kRefitChunkBits;
 constexpr uint32_t kRefitThreads = kRefitChunk;
-constexpr uint32_t kRefitTopThreads = 1024;
+constexpr uint32_t kRefitTopThreads = 256;
 
-// Writes internal node `node` from its children's boxes (both final) and
-// returns its union box in `self`.
+// Writes internal node `node` from its children's boxes.
 __device__ __forceinline__ tc_bvh_node write_node(const BvhArgs& a, uint32_t node, uint32_t c0w, uint32_t c1w,
-                                                  const float lo[2][3], const float hi[2][3], tc_aabb& self) {
+                                                  const tc_aabb& b0, const tc_aabb& b1) {
   tc_bvh_node out;
-  for (int q = 0; q < 3; q++) {
-    out.lo0[q] = lo[0][q], out.hi0[q] = hi[0][q], out.lo1[q] = lo[1][q], out.hi1[q] = hi[1][q];
-  }
+  for (int q = 0; q < 3; q++) out.lo0[q] = b0.lo[q], out.hi0[q] = b0.hi[q], out.lo1[q] = b1.lo[q], out.hi1[q] = b1.hi[q];
   out.child0 = c0w;
   out.child1 = c1w;
   out._pad0 = out._pad1 = 0;
   gst_record(a.nodes + node, out);
-  for (int q = 0; q < 3; q++) self.lo[q] = fminf(lo[0][q], lo[1][q]), self.hi[q] = fmaxf(hi[0][q], hi[1][q]);
-  gst_record(a.nodeBox + node, self);  // read by straddling parents and the TLAS
   return out;
 }
 
-__global__ __launch_bounds__(kRefitThreads) void k_blas_refit(BvhArgs a) {
+// Place of a child's box in the chunk that starts at c0.
+__device__ __forceinline__ uint32_t box_at(uint32_t word, uint32_t first, uint32_t c0) {
+  return first + (word & ~TC_BVH_LEAF) - c0 + ((word & TC_BVH_LEAF) ? kRefitChunk : 0u);
+}
+
+__global__ __launch_bounds__(kRefitThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_blas_refit(BvhArgs a) {
   __shared__ uint32_t s_cnt[kRefitChunk];
-  __shared__ tc_aabb s_box[kRefitChunk];   // internal nodes' union boxes
-  __shared__ tc_aabb s_leaf[kRefitChunk];  // leaves' boxes
+  __shared__ tc_aabb s_box[2 * kRefitChunk + 1];  // internal nodes' union boxes, leaves' boxes, an empty one
   __shared__ uint32_t s_child[kRefitChunk][2];
   __shared__ uint32_t s_parent[kRefitChunk], s_leafParent[kRefitChunk], s_range[kRefitChunk];
   const tc_scene_building* b = a.build;
   const uint32_t n = min(b->blasClusterCounter, a.capacity);
   const uint32_t j = threadIdx.x;
+  if (j == 0)
+    for (int q = 0; q < 3; q++) s_box[2 * kRefitChunk].lo[q] = INFINITY, s_box[2 * kRefitChunk].hi[q] = -INFINITY;
   for (uint32_t c0 = blockIdx.x * kRefitChunk; c0 < n; c0 += gridDim.x * kRefitChunk) {
     const uint32_t c1 = min(c0 + kRefitChunk, n);
     const uint32_t k = c0 + j;
-    int64_t first = 0, last = 0;
+    uint32_t first = 0, last = 0;
     s_cnt[j] = 0;
     if (k < c1) {
-      blas_segment(a, (uint32_t)(a.sortedKeys[k] >> 32), n, first, last);
+      int64_t f, l;
+      blas_segment(a, (uint32_t)(a.sortedKeys[k] >> 32), n, f, l);
+      first = (uint32_t)f, last = (uint32_t)l;
       s_leafParent[j] = a.parent[a.capacity + k];
       // internal node k exists when k < last; the other entries are unread
       s_parent[j] = a.parent[k];
@@ -317,7 +320,7 @@ __global__ __launch_bounds__(kRefitThreads) void k_blas_refit(BvhArgs a) {
       s_child[j][1] = a.child[2 * k + 1];
       float lo[3], hi[3];
       leaf_box(a, k, lo, hi);
-      for (int q = 0; q < 3; q++) s_leaf[j].lo[q] = lo[q], s_leaf[j].hi[q] = hi[q];
+      for (int q = 0; q < 3; q++) s_box[kRefitChunk + j].lo[q] = lo[q], s_box[kRefitChunk + j].hi[q] = hi[q];
     }
     __syncthreads();
     if (k < c1 && first != last) {  // a single CLAS is its instance's root
@@ -329,13 +332,12 @@ __global__ __launch_bounds__(kRefitThreads) void k_blas_refit(BvhArgs a) {
           if (atomicAdd(&a.counter[node], 1u) == 1u) {
             const uint32_t inst = (uint32_t)(a.sortedKeys[k] >> 32);
             const uint32_t slot = atomicAdd(&a.pendingCount[inst], 1u);
-            a.pendingList[((uint32_t)first >> kRefitChunkBits) + inst + slot] = node;
+            a.pendingList[(first >> kRefitChunkBits) + inst + slot] = node;
           }
           break;
         }
         const uint32_t ln = node - c0;
-        // the arrival orders LDS only (s_box, s_cnt): no wait for the node
-        // stores, which no climber of this chunk reads
+        // the arrival orders LDS only (s_box, s_cnt)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         if (atomicAdd(&s_cnt[ln], 1u) == 0) break;  // first arrival stops
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
@@ -344,126 +346,192 @@ __global__ __launch_bounds__(kRefitThreads) void k_blas_refit(BvhArgs a) {
         const uint32_t cw[2] = {s_child[ln][0], s_child[ln][1]};
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-          const uint32_t g = (uint32_t)first + (cw[c] & ~TC_BVH_LEAF) - c0;
-          const tc_aabb& bx = (cw[c] & TC_BVH_LEAF) ? s_leaf[g] : s_box[g];
+          const tc_aabb& bx = s_box[box_at(cw[c], first, c0)];
           for (int q = 0; q < 3; q++) lo[c][q] = bx.lo[q], hi[c][q] = bx.hi[q];
         }
         tc_aabb self;
-        write_node(a, node, cw[0], cw[1], lo, hi, self);
+        for (int q = 0; q < 3; q++) self.lo[q] = fminf(lo[0][q], lo[1][q]), self.hi[q] = fmaxf(hi[0][q], hi[1][q]);
         s_box[ln] = self;
-        if ((int64_t)node == first) break;  // instance root
+        if (node == first) {  // instance root
+          gst_record(a.nodeBox + node, self);
+          break;
+        }
         node = s_parent[ln];
       }
     }
     __syncthreads();
-    // four-wide records of the chunk's local internal nodes, one per
-    // thread, from LDS (the grandchildren of a local node lie in the chunk)
-    if (k < c1 && (int64_t)k < last && s_range[j] >= c0 && s_range[j] < c1) {
+    // binary and four-wide records of the chunk's local internal nodes, one
+    // per thread, from LDS (the grandchildren of a local node lie in the
+    // chunk): neighbouring threads write neighbouring records, and the climbs,
+    // in which few lanes are left after a level or two, store nothing
+    if (k < c1 && k < last && s_range[j] >= c0 && s_range[j] < c1) {
       const uint32_t cw[2] = {s_child[j][0], s_child[j][1]};
-      Slot4 gs[2][2];
+      const uint32_t at[2] = {box_at(cw[0], first, c0), box_at(cw[1], first, c0)};
+      write_node(a, k, cw[0], cw[1], s_box[at[0]], s_box[at[1]]);
+      // slots as make4 orders them, by their boxes' places: the record leaves
+      // a vector at a time, so that the kernel keeps to 64 registers and two
+      // workgroups share a CU
+      const bool leaf0 = (cw[0] & TC_BVH_LEAF) != 0, leaf1 = (cw[1] & TC_BVH_LEAF) != 0;
+      const uint32_t a1w = leaf0 ? 0u : s_child[at[0]][1], b1w = leaf1 ? 0u : s_child[at[1]][1];
+      const uint32_t a0w = leaf0 ? cw[0] : s_child[at[0]][0], b0w = leaf1 ? cw[1] : s_child[at[1]][0];
+      uint32_t w[4], p[4];
+      w[0] = a0w;
+      w[1] = leaf0 ? b0w : a1w;
+      w[2] = leaf0 ? (leaf1 ? TC_BVH4_EMPTY : b1w) : b0w;
+      w[3] = leaf0 || leaf1 ? TC_BVH4_EMPTY : b1w;
 #pragma unroll
-      for (int c = 0; c < 2; c++) {
-        if (cw[c] & TC_BVH_LEAF) {
-          const tc_aabb& bx = s_leaf[(uint32_t)first + (cw[c] & ~TC_BVH_LEAF) - c0];
-          gs[c][0] = gs[c][1] = slot4(bx.lo, bx.hi, cw[c]);
-        } else {
-          const uint32_t g = (uint32_t)first + cw[c] - c0;
+      for (int q = 0; q < 4; q++) p[q] = w[q] == TC_BVH4_EMPTY ? 2 * kRefitChunk : box_at(w[q], first, c0);
+      float* out = reinterpret_cast<float*>(a.nodes4 + k);
 #pragma unroll
-          for (int d = 0; d < 2; d++) {
-            const uint32_t gw = s_child[g][d];
-            const uint32_t h = (uint32_t)first + (gw & ~TC_BVH_LEAF) - c0;
-            const tc_aabb& bx = (gw & TC_BVH_LEAF) ? s_leaf[h] : s_box[h];
-            gs[c][d] = slot4(bx.lo, bx.hi, gw);
-          }
-        }
+      for (int q = 0; q < 6; q++) {
+        typedef float f4 __attribute__((ext_vector_type(4)));
+        const auto side = [&](int i) { return q < 3 ? s_box[p[i]].lo[q % 3] : s_box[p[i]].hi[q % 3]; };
+        gst(reinterpret_cast<f4*>(out) + q, f4{side(0), side(1), side(2), side(3)});
       }
-      gst_record(a.nodes4 + k, make4((cw[0] & TC_BVH_LEAF) != 0, gs[0][0], gs[0][1], (cw[1] & TC_BVH_LEAF) != 0,
-                                     gs[1][0], gs[1][1]));
+      typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+      gst(reinterpret_cast<u4*>(out) + 6, u4{w[0], w[1], w[2], w[3]});
+      gst(reinterpret_cast<u4*>(out) + 7, u4{0u, 0u, 0u, 0u});
     }
     __syncthreads();
   }
 }
 
-// Arrivals of this launch are counted in LDS, one byte per internal node
-// (four per word), for instances of up to kRefitTopLdsNodes internal nodes;
-// the count the chunk launch left in the global counter is only read.
-// Larger instances count with global atomics.
-constexpr uint32_t kRefitTopLdsNodes = 131072;
-
-// Refit of straddling node `node` from its child words cw, with its
-// four-wide record: a leaf child's box comes from its CLAS, an internal
-// child's from its binary record, whose two slots are also the grandchildren
-// the four-wide record takes (the record's union is the child's node box,
-// to the bit).
-__device__ __forceinline__ void refit_top_node(const BvhArgs& a, uint32_t node, const uint32_t cw[2], int64_t first) {
-  float lo[2][3], hi[2][3];
-  Slot4 g[2][2];
-  bool leaf[2];
-#pragma unroll
-  for (int c = 0; c < 2; c++) {
-    const uint32_t ch = cw[c];
-    leaf[c] = (ch & TC_BVH_LEAF) != 0;
-    if (leaf[c]) {
-      leaf_box(a, (uint32_t)first + (ch & ~TC_BVH_LEAF), lo[c], hi[c]);
-      g[c][0] = g[c][1] = slot4(lo[c], hi[c], ch);
-    } else {
-      const tc_bvh_node m = gld_record(a.nodes + (uint32_t)first + ch);
-      for (int q = 0; q < 3; q++) lo[c][q] = fminf(m.lo0[q], m.lo1[q]), hi[c][q] = fmaxf(m.hi0[q], m.hi1[q]);
-      g[c][0] = slot4(m.lo0, m.hi0, m.child0);
-      g[c][1] = slot4(m.lo1, m.hi1, m.child1);
-    }
+// A child of a node being refit: an internal one's binary record (its union is
+// the child's box, and its two slots are the grandchildren of the four-wide
+// record), or a leaf's box twice.
+struct RefitChild {
+  Slot4 s[2];
+  uint32_t word;
+};
+__device__ __forceinline__ RefitChild refit_child(const tc_bvh_node& m, uint32_t word) {
+  RefitChild r;
+  r.s[0] = slot4(m.lo0, m.hi0, m.child0);
+  r.s[1] = slot4(m.lo1, m.hi1, m.child1);
+  r.word = word;
+  return r;
+}
+// A child that is final before this launch, from memory.
+__device__ __forceinline__ RefitChild refit_child_at(const BvhArgs& a, int64_t first, uint32_t word) {
+  RefitChild r;
+  if (word & TC_BVH_LEAF) {
+    float lo[3], hi[3];
+    leaf_box(a, (uint32_t)first + (word & ~TC_BVH_LEAF), lo, hi);
+    r.s[0] = r.s[1] = slot4(lo, hi, word);
+    r.word = word;
+  } else {
+    r = refit_child(gld_record(a.nodes + (uint32_t)first + word), word);
   }
-  tc_aabb self;
-  write_node(a, node, cw[0], cw[1], lo, hi, self);
-  gst_record(a.nodes4 + node, make4(leaf[0], g[0][0], g[0][1], leaf[1], g[1][0], g[1][1]));
+  return r;
+}
+__device__ __forceinline__ tc_aabb union_box(const Slot4& x, const Slot4& y) {
+  tc_aabb b;
+  for (int q = 0; q < 3; q++) b.lo[q] = fminf(x.lo[q], y.lo[q]), b.hi[q] = fmaxf(x.hi[q], y.hi[q]);
+  return b;
 }
 
+// Refit of straddling node `node`: its binary record (returned) and its
+// four-wide one.
+__device__ __forceinline__ tc_bvh_node refit_top_node(const BvhArgs& a, uint32_t node, int64_t first, const RefitChild& c0,
+                                                      const RefitChild& c1) {
+  const tc_bvh_node out =
+      write_node(a, node, c0.word, c1.word, union_box(c0.s[0], c0.s[1]), union_box(c1.s[0], c1.s[1]));
+  gst_record(a.nodes4 + node,
+             make4((c0.word & TC_BVH_LEAF) != 0, c0.s[0], c0.s[1], (c1.word & TC_BVH_LEAF) != 0, c1.s[0], c1.s[1]));
+  if ((int64_t)node == first) {  // instance root, read by the TLAS
+    tc_aabb self;
+    for (int q = 0; q < 3; q++) self.lo[q] = fminf(out.lo0[q], out.lo1[q]), self.hi[q] = fmaxf(out.hi0[q], out.hi1[q]);
+    gst_record(a.nodeBox + node, self);
+  }
+  return out;
+}
+
+// A climb goes up through nodes with one straddling child (the other is final)
+// and meets another climb at nodes with two: there the first to arrive leaves
+// its record in LDS, in a table by node, and stops.  What bounds a climb is its
+// chain of memory round trips, some 15 levels of them at an instance of 5000
+// CLAS: the topology and a final sibling's record are fetched together, a level
+// ahead, the record of the child just refit stays in registers, and no climb
+// reads a record that the launch has stored.  Measured: 64 instances of 4840
+// CLAS 42.7 -> 33.7 us, 500 meshes 30 -> 17 us, 5 instances of 5200 23 ->
+// 16.6 us, 64 instances of 51,000 160 -> 144 us.
+// More climbs than kTopMeets (half a million CLAS in one instance) meet in
+// global memory instead.
+constexpr uint32_t kTopMeets = 512;
+constexpr uint32_t kTopTable = 2 * kTopMeets;
+
 __global__ __launch_bounds__(kRefitTopThreads) void k_blas_refit_top(BvhArgs a) {
-  __shared__ uint32_t s_arrive[kRefitTopLdsNodes / 4];
+  __shared__ uint32_t s_node[kTopTable], s_meet[kTopTable];
+  __shared__ __align__(16) tc_bvh_node s_rec[kTopMeets];
   const uint32_t inst = blockIdx.x;
   if (inst >= a.numInstances) return;
   const tc_scene_building* b = a.build;
   const uint32_t n = min(b->blasClusterCounter, a.capacity);
   const tc_blas_build_info& bi = ptr<const tc_blas_build_info>(b->blasBuildInfos)[inst];
-  if (bi.clusterReferencesCount < 2) return;
+  const uint32_t count = a.pendingCount[inst];
+  if (bi.clusterReferencesCount < 2 || count == 0) return;
   const int64_t first = (int64_t)((bi.clusterReferences - b->blasClusterAddresses) / 8);
   if (first >= (int64_t)n) return;
-  const uint32_t count = a.pendingCount[inst];
   const uint32_t base = ((uint32_t)first >> kRefitChunkBits) + inst;
-  const bool ldsCount = bi.clusterReferencesCount - 1 <= kRefitTopLdsNodes;
-  if (ldsCount)
-    for (uint32_t w = threadIdx.x; w < (bi.clusterReferencesCount + 2) / 4; w += kRefitTopThreads) s_arrive[w] = 0;
+  const bool meetLds = count <= kTopMeets;
+  if (meetLds)
+    for (uint32_t w = threadIdx.x; w < kTopTable; w += kRefitTopThreads) s_node[w] = ~0u, s_meet[w] = 0;
   __syncthreads();
   for (uint32_t t = threadIdx.x; t < count; t += kRefitTopThreads) {
     uint32_t node = a.pendingList[base + t];
     // A node's child words and parent (written by the hierarchy launch) and
-    // the chunk launch's arrivals there are final, so the parent's load
-    // together with the node's child records: one round trip a level.
-    uint32_t cw[2] = {gld(a.child + 2 * node), gld(a.child + 2 * node + 1)};
-    uint32_t up = gld(a.parent + node);
+    // the chunk launch's arrivals there are final.
+    uint32_t up = gld(a.parent + node);  // (the root's is not followed)
+    uint32_t w0 = gld(a.child + 2 * node), w1 = gld(a.child + 2 * node + 1), nup = 0, prior = 0;
+    RefitChild c0 = refit_child_at(a, first, w0), c1 = refit_child_at(a, first, w1);
+    if ((int64_t)node != first) {
+      w0 = gld(a.child + 2 * up), w1 = gld(a.child + 2 * up + 1);
+      nup = gld(a.parent + up);
+      prior = gld(a.counter + up);
+    }
     while (true) {
       const bool root = (int64_t)node == first;
-      uint32_t ncw[2] = {0u, 0u}, nup = 0u, prior = 0u;
-      if (!root) {
-        ncw[0] = gld(a.child + 2 * up), ncw[1] = gld(a.child + 2 * up + 1);
-        nup = gld(a.parent + up);
-        prior = ldsCount ? gld(a.counter + up) : 0u;
-      }
-      refit_top_node(a, node, cw, first);
+      const uint32_t self = node - (uint32_t)first;
+      const bool right = w1 == self;  // (an internal child's word is its index)
+      const uint32_t sib = right ? w0 : w1;
+      const bool final = !root && meetLds && prior != 0, leaf = (sib & TC_BVH_LEAF) != 0;
+      // the sibling's record, if it is final, and the next level's topology,
+      // before this level's stores
+      const tc_bvh_node sibRec = gld_record(a.nodes + (uint32_t)first + (final && !leaf ? sib : 0u));
+      const uint32_t at = root || (int64_t)up == first ? node : nup;
+      const uint32_t x0 = gld(a.child + 2 * at), x1 = gld(a.child + 2 * at + 1), xup = gld(a.parent + at),
+                     xprior = gld(a.counter + at);
+      const tc_bvh_node rec = refit_top_node(a, node, first, c0, c1);
       if (root) break;
-      node = up;
-      cw[0] = ncw[0], cw[1] = ncw[1];
-      up = nup;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-      uint32_t before;
-      if (ldsCount) {
-        const uint32_t rel = node - (uint32_t)first, sh = 8 * (rel & 3);
-        before = ((atomicAdd(&s_arrive[rel >> 2], 1u << sh) >> sh) & 0xFFu) + prior;
+      RefitChild other;
+      if (final) {
+        other = refit_child(sibRec, sib);
+        if (leaf) other = refit_child_at(a, first, sib);
+      } else if (!meetLds) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (atomicAdd(&a.counter[up], 1u) == 0) break;  // first arrival stops
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        other = refit_child_at(a, first, sib);
       } else {
-        before = atomicAdd(&a.counter[node], 1u);
+        uint32_t h = (up * 2654435761u) >> (32 - 10);
+        static_assert(kTopTable == 1u << 10, "the hash's bits");
+        while (true) {  // at most kTopMeets - 1 nodes have two climbs
+          const uint32_t seen = atomicCAS(&s_node[h], ~0u, up);
+          if (seen == ~0u || seen == up) break;
+          h = (h + 1) & (kTopTable - 1);
+        }
+        // the climb's own record: it stays in place once the climb stops
+        s_rec[t] = rec;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        const uint32_t met = atomicExch(&s_meet[h], t + 1);
+        if (met == 0) break;  // first arrival stops
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        other = refit_child(s_rec[met - 1], sib);
       }
-      if (before == 0) break;  // first arrival stops
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+      const RefitChild mine = refit_child(rec, self);
+      c0 = right ? other : mine, c1 = right ? mine : other;
+      node = up;
+      up = nup;
+      w0 = x0, w1 = x1, nup = xup, prior = xprior;
     }
   }
 }
