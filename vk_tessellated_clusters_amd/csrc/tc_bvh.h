@@ -17,12 +17,12 @@ struct BvhArgs {
   const uint32_t* sortedVals;
   uint64_t* leafAddr;  // CLAS address per sorted position (blasLeaves)
   uint64_t* leafInfo;  // its header's counts | clusterID << 32 (blasLeafInfo)
-  uint32_t* child;     // 2 per internal node, relative to the instance start
-  uint32_t* parent;    // [0, capacity) internal nodes, [capacity, 2 capacity) leaves
-  uint32_t* counter;   // refit arrival counters
-  uint32_t* rangeEnd;  // per internal node: the far end of its key range (global position)
-  uint32_t* pendingCount;  // per instance: straddling nodes listed by the chunk refit
-  uint32_t* pendingList;   // their node indices, per instance from (first >> 10) + instance
+  // internal nodes whose key range straddles chunks (the others' entries are
+  // not written)
+  uint32_t* child;        // 2 per node, relative to the instance start
+  uint32_t* parent;       // of such a node, unless it is a root
+  uint32_t* counter;      // its children that are final before the climbs
+  uint32_t* pendingList;  // per chunk boundary: the node split there, when both its children are final, or ~0
   tc_bvh_node* nodes;  // blasNodes
   tc_bvh4_node* nodes4;  // blasNodes4
   tc_aabb* nodeBox;    // union box of every internal node
@@ -43,7 +43,7 @@ struct BvhArgs {
 };
 
 struct AccelLayout {
-  uint64_t blasNodes, blasLeaves, nodeBox, child, parent, counter, rangeEnd, pendingCount, pendingList;
+  uint64_t blasNodes, blasLeaves, nodeBox, child, parent, counter, pendingList;
   uint64_t blasNodes4, tlasNodes4, blasLeafInfo;
   uint64_t tlasInstances, tlasNodes, tlasNodeBox, tlasLeafBox, tlasChild, tlasParent, tlasCounter, tlasKeys, tlasVals,
       tlasRoot;

@@ -119,7 +119,7 @@ __device__ __forceinline__ int delta(const uint64_t* keys, int64_t i, int64_t j,
 // Karras (2012) radix tree for the segment [first, last] of sorted keys;
 // thread handles internal node `g` (global index first + local j).
 __device__ __forceinline__ void karras_node(const uint64_t* keys, int64_t first, int64_t last, int64_t i, uint32_t* child,
-                                            uint32_t* parent, uint32_t leafParentBase, uint32_t* rangeEnd = nullptr) {
+                                            uint32_t* parent, uint32_t leafParentBase) {
   const int d = (delta(keys, i, i + 1, first, last) - delta(keys, i, i - 1, first, last)) >= 0 ? 1 : -1;
   const int dmin = delta(keys, i, i - d, first, last);
   int64_t lmax = 2;
@@ -137,7 +137,6 @@ __device__ __forceinline__ void karras_node(const uint64_t* keys, int64_t first,
   } while (t > 1);
   const int64_t gamma = i + s * d + min(d, 0);
   const int64_t lo = min(i, j), hi = max(i, j);
-  if (rangeEnd) rangeEnd[i] = (uint32_t)j;
   // children: leaf flag + position relative to `first`, or internal node
   const uint32_t c0 = (lo == gamma) ? (TC_BVH_LEAF | (uint32_t)(gamma - first)) : (uint32_t)(gamma - first);
   const uint32_t c1 = (hi == gamma + 1) ? (TC_BVH_LEAF | (uint32_t)(gamma + 1 - first)) : (uint32_t)(gamma + 1 - first);
@@ -162,31 +161,16 @@ __device__ __forceinline__ void blas_segment(const BvhArgs& a, uint32_t inst, ui
   last = first + (int64_t)bi.clusterReferencesCount - 1;
 }
 
-// One thread per sorted position k: internal node k of its instance (when
-// k < last) and the sorted CLAS address.
-__global__ void k_blas_hierarchy(BvhArgs a) {
-  const tc_scene_building* b = a.build;
-  const uint32_t n = min(b->blasClusterCounter, a.capacity);
-  const uint64_t* refs = ptr<const uint64_t>(b->blasClusterAddresses);
-  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-    const uint32_t inst = (uint32_t)(a.sortedKeys[k] >> 32);
-    int64_t first, last;
-    blas_segment(a, inst, n, first, last);
-    a.leafAddr[k] = refs[a.sortedVals[k]];
-    a.counter[k] = 0;
-    if ((int64_t)k < last) karras_node(a.sortedKeys, first, last, k, a.child, a.parent, a.capacity, a.rangeEnd);
-  }
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.numInstances; i += gridDim.x * blockDim.x)
-    a.pendingCount[i] = 0;
-}
-
 // Box of sorted leaf k from its CLAS header; also writes the leaf's info
-// word (counts | clusterID << 32) from the same header.  The refit stages
-// every leaf once; the leaves of straddling nodes are read again.
-__device__ __forceinline__ void leaf_box(const BvhArgs& a, uint32_t k, float lo[3], float hi[3]) {
-  const tc_clas_header h = gld_record(ptr<const tc_clas_header>(a.leafAddr[k]));
+// word (counts | clusterID << 32) from the same header.  The chunk launch
+// stages every leaf once; the leaves of straddling nodes are read again.
+__device__ __forceinline__ void leaf_box_at(const BvhArgs& a, uint32_t k, uint64_t addr, float lo[3], float hi[3]) {
+  const tc_clas_header h = gld_record(ptr<const tc_clas_header>(addr));
   for (int c = 0; c < 3; c++) lo[c] = h.lo[c], hi[c] = h.hi[c];
-  a.leafInfo[k] = (uint64_t)h.counts | (uint64_t)h.clusterID << 32;
+  gst(a.leafInfo + k, (uint64_t)h.counts | (uint64_t)h.clusterID << 32);
+}
+__device__ __forceinline__ void leaf_box(const BvhArgs& a, uint32_t k, float lo[3], float hi[3]) {
+  leaf_box_at(a, k, gld(a.leafAddr + k), lo, hi);
 }
 
 // One slot of a four-wide record: a box and its child word.
@@ -249,28 +233,31 @@ __device__ __forceinline__ void collapse4(const tc_bvh_node* nodes, uint32_t i, 
   gst_record(out + i, collapse4_of(gld_record(nodes + i), nodes));
 }
 
-// Bottom-up refit in two launches, with no device-scope fence.
+// The tree of every instance and its boxes in two launches, with no
+// device-scope fence.
 //
-// k_blas_refit: a workgroup owns a chunk of kRefitChunk sorted positions,
-// one thread per position.  It first stages the chunk's topology (child
-// words, parents, range ends of the internal nodes, the leaves' parents)
-// and its leaves' boxes (from their CLAS headers, which also give the leaf
-// info words) in LDS, all loads in parallel.  Then every leaf climbs; the
-// second arrival at a node writes it.  Nodes whose key range lies inside
-// the chunk are read and counted in LDS (workgroup-scope ordering), so a
-// climb waits on no global load.  A climb stops at the first node whose
-// range straddles chunks; the second arrival there lists the node as
-// pending for its instance (both children are then final).  The chunk's
-// binary and four-wide records are written from LDS once every climb is done.
-// It moves about 290 bytes a CLAS (3.0 TB/s at 3.3 million) and took as long as
-// its waits: with 66 registers one workgroup of 16 waves filled a CU, with 54
-// two share it.  3.3 million CLAS 365 -> 304 us, 310,000 46.9 -> 39.8 us.
+// k_blas_build: a workgroup owns a chunk of kRefitChunk sorted positions, one
+// thread per position.  It stages the chunk's keys and its leaves' boxes (from
+// their CLAS headers, which also give the leaf info words) in LDS; thread k
+// finds internal node k (Karras 2012) from the keys there, reading global keys
+// only where a range leaves the chunk.  Nodes whose key range lies inside the
+// chunk have their parents and children there as well, so topology, arrival
+// counts and boxes of the climbs from the leaves stay in LDS.  The binary and
+// four-wide records are written once every climb is done.  A node whose range
+// straddles chunks is described in memory by its thread: child words, which of
+// its children are final (leaves, or ranges inside one chunk), and the parent
+// of those that are not; with two final children it is pending, the entry of
+// the one chunk boundary that its range holds (its split).
+// With the tree in a launch before, 36 bytes a CLAS of topology went through
+// memory and every search waited for some twenty loads of keys one after
+// another: both took 60 us at 310,000 CLAS in 64 instances, 409 us at 3.3
+// million, 30 us at 8192 in one; now 48, 361 and 26 us.  In the last, staging
+// takes 3.2 us, the searches 9.6, the climbs 5.9 and the records 5.5.
+// Two workgroups of 16 waves share a CU (64 registers, 74 KB).
 //
-// k_blas_refit_top: one workgroup per instance climbs from its pending
-// nodes through the straddling nodes; each node's records are written where
-// the node is refit.  A pending node's range holds exactly one chunk boundary
-// (its split), so an instance has fewer pending nodes than chunks it spans;
-// its list starts at (first >> kRefitChunkBits) + instance.
+// k_blas_refit_top: one workgroup per instance climbs from its pending nodes
+// through the straddling nodes; each node's records are written where the node
+// is refit.
 constexpr uint32_t kRefitChunkBits = 10;
 constexpr uint32_t kRefitChunk = 1u << kRefitChunkBits;
 constexpr uint32_t kRefitThreads = kRefitChunk;
@@ -293,13 +280,17 @@ __device__ __forceinline__ uint32_t box_at(uint32_t word, uint32_t first, uint32
   return first + (word & ~TC_BVH_LEAF) - c0 + ((word & TC_BVH_LEAF) ? kRefitChunk : 0u);
 }
 
-__global__ __launch_bounds__(kRefitThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_blas_refit(BvhArgs a) {
+__global__ __launch_bounds__(kRefitThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_blas_build(BvhArgs a) {
+  constexpr uint32_t kNone = ~0u;
+  __shared__ uint32_t s_key[kRefitChunk + 2];  // Morton codes of positions c0 - 1 .. c1
   __shared__ uint32_t s_cnt[kRefitChunk];
   __shared__ tc_aabb s_box[2 * kRefitChunk + 1];  // internal nodes' union boxes, leaves' boxes, an empty one
   __shared__ uint32_t s_child[kRefitChunk][2];
-  __shared__ uint32_t s_parent[kRefitChunk], s_leafParent[kRefitChunk], s_range[kRefitChunk];
+  __shared__ uint32_t s_parent[kRefitChunk], s_leafParent[kRefitChunk];  // in the chunk, or kNone
   const tc_scene_building* b = a.build;
   const uint32_t n = min(b->blasClusterCounter, a.capacity);
+  const uint64_t* refs = ptr<const uint64_t>(b->blasClusterAddresses);
+  const uint32_t* codes = reinterpret_cast<const uint32_t*>(a.sortedKeys);  // the keys' low words
   const uint32_t j = threadIdx.x;
   if (j == 0)
     for (int q = 0; q < 3; q++) s_box[2 * kRefitChunk].lo[q] = INFINITY, s_box[2 * kRefitChunk].hi[q] = -INFINITY;
@@ -308,55 +299,88 @@ __global__ __launch_bounds__(kRefitThreads) __attribute__((amdgpu_waves_per_eu(8
     const uint32_t k = c0 + j;
     uint32_t first = 0, last = 0;
     s_cnt[j] = 0;
+    s_parent[j] = s_leafParent[j] = kNone;
+    if (j == 0) {
+      s_key[0] = c0 ? (uint32_t)gld(a.sortedKeys + c0 - 1) : 0u;
+      s_key[c1 - c0 + 1] = c1 < n ? (uint32_t)gld(a.sortedKeys + c1) : 0u;
+    }
     if (k < c1) {
+      const uint64_t key = gld(a.sortedKeys + k);
+      const uint64_t addr = gld(refs + gld(a.sortedVals + k));
+      s_key[j + 1] = (uint32_t)key;
       int64_t f, l;
-      blas_segment(a, (uint32_t)(a.sortedKeys[k] >> 32), n, f, l);
+      blas_segment(a, (uint32_t)(key >> 32), n, f, l);
       first = (uint32_t)f, last = (uint32_t)l;
-      s_leafParent[j] = a.parent[a.capacity + k];
-      // internal node k exists when k < last; the other entries are unread
-      s_parent[j] = a.parent[k];
-      s_range[j] = a.rangeEnd[k];
-      s_child[j][0] = a.child[2 * k + 0];
-      s_child[j][1] = a.child[2 * k + 1];
+      gst(a.leafAddr + k, addr);
       float lo[3], hi[3];
-      leaf_box(a, k, lo, hi);
+      leaf_box_at(a, k, addr, lo, hi);
       for (int q = 0; q < 3; q++) s_box[kRefitChunk + j].lo[q] = lo[q], s_box[kRefitChunk + j].hi[q] = hi[q];
     }
     __syncthreads();
-    if (k < c1 && first != last) {  // a single CLAS is its instance's root
-      uint32_t node = s_leafParent[j];
-      while (true) {
-        const bool local = node >= c0 && node < c1 && s_range[node - c0] >= c0 && s_range[node - c0] < c1;
-        if (!local) {
-          // straddling: the second arrival lists it for the second launch
-          if (atomicAdd(&a.counter[node], 1u) == 1u) {
-            const uint32_t inst = (uint32_t)(a.sortedKeys[k] >> 32);
-            const uint32_t slot = atomicAdd(&a.pendingCount[inst], 1u);
-            a.pendingList[(first >> kRefitChunkBits) + inst + slot] = node;
-          }
-          break;
-        }
-        const uint32_t ln = node - c0;
+    // internal node k exists when k < last (a single CLAS is its instance's root)
+    bool local = false;
+    if (k < c1 && k >= first && k < last) {
+      const uint32_t ki = s_key[j + 1];
+      const int f = (int)first, l = (int)last, i = (int)k;
+      // common prefix of the keys at i and x: of the Morton codes, as the keys
+      // of an instance share their high words; equal codes by position; -1
+      // outside the instance
+      const auto prefix = [&](int x) {
+        if (x < f || x > l) return -1;
+        const uint32_t o = (uint32_t)x + 1 - c0;
+        const uint32_t v = ki ^ (o <= c1 - c0 + 1 ? s_key[o] : gld(codes + 2 * (uint64_t)x));
+        return v ? __clz(v) : 32 + __clz((uint32_t)i ^ (uint32_t)x);
+      };
+      const int next = prefix(i + 1), prev = prefix(i - 1);
+      const int d = next - prev >= 0 ? 1 : -1, dmin = d > 0 ? prev : next;
+      int far = 2;
+      while (prefix(i + far * d) > dmin) far *= 2;
+      int len = 0;
+      for (int t = far / 2; t >= 1; t /= 2)
+        if (prefix(i + (len + t) * d) > dmin) len += t;
+      const int dnode = prefix(i + len * d);
+      int s = 0, t = len;
+      do {
+        t = (t + 1) / 2;
+        if (prefix(i + (s + t) * d) > dnode) s += t;
+      } while (t > 1);
+      const uint32_t gamma = (uint32_t)(i + s * d + min(d, 0));
+      const uint32_t lo = (uint32_t)min(i, i + len * d), hi = (uint32_t)max(i, i + len * d);
+      const bool leaf0 = lo == gamma, leaf1 = hi == gamma + 1;
+      const uint32_t w0 = (leaf0 ? TC_BVH_LEAF : 0u) | (gamma - first), w1 = (leaf1 ? TC_BVH_LEAF : 0u) | (gamma + 1 - first);
+      local = lo >= c0 && hi < c1;
+      if (local) {
+        s_child[j][0] = w0, s_child[j][1] = w1;
+        (leaf0 ? s_leafParent : s_parent)[gamma - c0] = j;
+        (leaf1 ? s_leafParent : s_parent)[gamma + 1 - c0] = j;
+      } else {
+        const bool final0 = lo >> kRefitChunkBits == gamma >> kRefitChunkBits;
+        const bool final1 = (gamma + 1) >> kRefitChunkBits == hi >> kRefitChunkBits;
+        gst(a.child + 2 * k, w0);
+        gst(a.child + 2 * k + 1, w1);
+        gst(a.counter + k, (final0 ? 1u : 0u) + (final1 ? 1u : 0u));
+        if (!final0) gst(a.parent + gamma, k);
+        if (!final1) gst(a.parent + gamma + 1, k);
+        if (((gamma + 1) & (kRefitChunk - 1)) == 0) gst(a.pendingList + ((gamma + 1) >> kRefitChunkBits), final0 && final1 ? k : kNone);
+      }
+    }
+    __syncthreads();
+    if (k < c1 && first != last) {
+      uint32_t ln = s_leafParent[j];
+      while (ln != kNone) {
         // the arrival orders LDS only (s_box, s_cnt)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         if (atomicAdd(&s_cnt[ln], 1u) == 0) break;  // first arrival stops
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        // a local node's children (leaves or internal nodes) lie in the chunk
-        float lo[2][3], hi[2][3];
-        const uint32_t cw[2] = {s_child[ln][0], s_child[ln][1]};
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-          const tc_aabb& bx = s_box[box_at(cw[c], first, c0)];
-          for (int q = 0; q < 3; q++) lo[c][q] = bx.lo[q], hi[c][q] = bx.hi[q];
-        }
+        const tc_aabb &b0 = s_box[box_at(s_child[ln][0], first, c0)], &b1 = s_box[box_at(s_child[ln][1], first, c0)];
         tc_aabb self;
-        for (int q = 0; q < 3; q++) self.lo[q] = fminf(lo[0][q], lo[1][q]), self.hi[q] = fmaxf(hi[0][q], hi[1][q]);
+        for (int q = 0; q < 3; q++) self.lo[q] = fminf(b0.lo[q], b1.lo[q]), self.hi[q] = fmaxf(b0.hi[q], b1.hi[q]);
         s_box[ln] = self;
-        if (node == first) {  // instance root
-          gst_record(a.nodeBox + node, self);
+        if (c0 + ln == first) {  // instance root
+          gst_record(a.nodeBox + first, self);
           break;
         }
-        node = s_parent[ln];
+        ln = s_parent[ln];
       }
     }
     __syncthreads();
@@ -364,7 +388,7 @@ __global__ __launch_bounds__(kRefitThreads) __attribute__((amdgpu_waves_per_eu(8
     // per thread, from LDS (the grandchildren of a local node lie in the
     // chunk): neighbouring threads write neighbouring records, and the climbs,
     // in which few lanes are left after a level or two, store nothing
-    if (k < c1 && k < last && s_range[j] >= c0 && s_range[j] < c1) {
+    if (local) {
       const uint32_t cw[2] = {s_child[j][0], s_child[j][1]};
       const uint32_t at[2] = {box_at(cw[0], first, c0), box_at(cw[1], first, c0)};
       write_node(a, k, cw[0], cw[1], s_box[at[0]], s_box[at[1]]);
@@ -467,19 +491,20 @@ __global__ __launch_bounds__(kRefitTopThreads) void k_blas_refit_top(BvhArgs a) 
   const tc_scene_building* b = a.build;
   const uint32_t n = min(b->blasClusterCounter, a.capacity);
   const tc_blas_build_info& bi = ptr<const tc_blas_build_info>(b->blasBuildInfos)[inst];
-  const uint32_t count = a.pendingCount[inst];
-  if (bi.clusterReferencesCount < 2 || count == 0) return;
+  if (bi.clusterReferencesCount < 2) return;
   const int64_t first = (int64_t)((bi.clusterReferences - b->blasClusterAddresses) / 8);
   if (first >= (int64_t)n) return;
-  const uint32_t base = ((uint32_t)first >> kRefitChunkBits) + inst;
+  // chunk boundaries inside the instance, with a pending node or none each
+  const uint32_t base = ((uint32_t)first >> kRefitChunkBits) + 1;
+  const uint32_t count = (((uint32_t)first + bi.clusterReferencesCount - 1) >> kRefitChunkBits) + 1 - base;
+  if (count == 0) return;
   const bool meetLds = count <= kTopMeets;
   if (meetLds)
     for (uint32_t w = threadIdx.x; w < kTopTable; w += kRefitTopThreads) s_node[w] = ~0u, s_meet[w] = 0;
   __syncthreads();
   for (uint32_t t = threadIdx.x; t < count; t += kRefitTopThreads) {
-    uint32_t node = a.pendingList[base + t];
-    // A node's child words and parent (written by the hierarchy launch) and
-    // the chunk launch's arrivals there are final.
+    uint32_t node = gld(a.pendingList + base + t);
+    if (node == ~0u) continue;
     uint32_t up = gld(a.parent + node);  // (the root's is not followed)
     uint32_t w0 = gld(a.child + 2 * node), w1 = gld(a.child + 2 * node + 1), nup = 0, prior = 0;
     RefitChild c0 = refit_child_at(a, first, w0), c1 = refit_child_at(a, first, w1);
@@ -829,11 +854,9 @@ AccelLayout accel_layout(uint32_t capacity, uint32_t numInstances) {
   put(L.blasLeafInfo, c * 8);
   put(L.nodeBox, c * sizeof(tc_aabb));
   put(L.child, 2 * c * 4);
-  put(L.parent, 2 * c * 4);
+  put(L.parent, c * 4);
   put(L.counter, c * 4);
-  put(L.rangeEnd, c * 4);
-  put(L.pendingCount, n * 4);
-  put(L.pendingList, (c / kRefitChunk + n + 2) * 4);
+  put(L.pendingList, (c / kRefitChunk + 2) * 4);
   put(L.tlasInstances, n * sizeof(tc_tlas_instance));
   put(L.tlasNodes, n * sizeof(tc_bvh_node));
   put(L.tlasNodes4, n * sizeof(tc_bvh4_node));
@@ -917,8 +940,6 @@ static tc_status accel_build(const tc_bindings* b, tc_config config, const tc_ac
   a.child = reinterpret_cast<uint32_t*>(m + L.child);
   a.parent = reinterpret_cast<uint32_t*>(m + L.parent);
   a.counter = reinterpret_cast<uint32_t*>(m + L.counter);
-  a.rangeEnd = reinterpret_cast<uint32_t*>(m + L.rangeEnd);
-  a.pendingCount = reinterpret_cast<uint32_t*>(m + L.pendingCount);
   a.pendingList = reinterpret_cast<uint32_t*>(m + L.pendingList);
   a.nodes = reinterpret_cast<tc_bvh_node*>(m + L.blasNodes);
   a.nodes4 = reinterpret_cast<tc_bvh4_node*>(m + L.blasNodes4);
@@ -934,7 +955,7 @@ static tc_status accel_build(const tc_bindings* b, tc_config config, const tc_ac
   a.tlasRoot = reinterpret_cast<uint32_t*>(m + L.tlasRoot);
 
   const uint32_t grid = std::min<uint32_t>((capacity + 255) / 256, (uint32_t)num_cu_public() * tuning_snapshot().bvhBlocksPerCU);
-  // BLAS: keys, sort by (instance, Morton), hierarchy, refit
+  // BLAS: keys, sort by (instance, Morton), trees and boxes
   if (!inserted) hipLaunchKernelGGL(k_blas_keys, dim3(grid), dim3(256), 0, st, a);
   uint32_t res = 0;
   // digits 0-2: the 24-bit Morton code; digits 4-5: the instance, where there
@@ -944,8 +965,7 @@ static tc_status accel_build(const tc_bindings* b, tc_config config, const tc_ac
                     inserted ? ip.insertPasses : 0);
   a.sortedKeys = sb.keys[res];
   a.sortedVals = sb.vals[res];
-  hipLaunchKernelGGL(k_blas_hierarchy, dim3(grid), dim3(256), 0, st, a);
-  hipLaunchKernelGGL(k_blas_refit, dim3(std::min<uint32_t>((capacity + kRefitChunk - 1) / kRefitChunk, (uint32_t)num_cu_public() * 4)),
+  hipLaunchKernelGGL(k_blas_build, dim3(std::min<uint32_t>((capacity + kRefitChunk - 1) / kRefitChunk, (uint32_t)num_cu_public() * 4)),
                      dim3(kRefitThreads), 0, st, a);
   hipLaunchKernelGGL(k_blas_refit_top, dim3(a.numInstances), dim3(kRefitTopThreads), 0, st, a);
   // TLAS over instances, with key and value arrays of its own
