@@ -17,12 +17,10 @@ struct BvhArgs {
   const uint32_t* sortedVals;
   uint64_t* leafAddr;  // CLAS address per sorted position (blasLeaves)
   uint64_t* leafInfo;  // its header's counts | clusterID << 32 (blasLeafInfo)
-  // internal nodes whose key range straddles chunks (the others' entries are
-  // not written)
-  uint32_t* child;        // 2 per node, relative to the instance start
-  uint32_t* parent;       // of such a node, unless it is a root
-  uint32_t* counter;      // its children that are final before the climbs
-  uint32_t* pendingList;  // per chunk boundary: the node split there, when both its children are final, or ~0
+  // of instances that lie in several chunks of the build, per position
+  uint32_t* waitEnd;    // the subtree that ends there and waits for a sibling from outside its chunk, or 0
+  uint32_t* waitBegin;  // ... that begins there
+  uint64_t* meet;       // the climb that waits at the boundary before it, or 0 (instances of very many chunks)
   tc_bvh_node* nodes;  // blasNodes
   tc_bvh4_node* nodes4;  // blasNodes4
   tc_aabb* nodeBox;    // union box of every internal node
@@ -43,7 +41,7 @@ struct BvhArgs {
 };
 
 struct AccelLayout {
-  uint64_t blasNodes, blasLeaves, nodeBox, child, parent, counter, pendingList;
+  uint64_t blasNodes, blasLeaves, nodeBox, waitEnd, waitBegin, meet;
   uint64_t blasNodes4, tlasNodes4, blasLeafInfo;
   uint64_t tlasInstances, tlasNodes, tlasNodeBox, tlasLeafBox, tlasChild, tlasParent, tlasCounter, tlasKeys, tlasVals,
       tlasRoot;

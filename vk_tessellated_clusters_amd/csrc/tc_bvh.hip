@@ -9,11 +9,10 @@
 //           single-pass launch per digit) over the three Morton digits and
 //           the one or two instance digits (stable, CLAS order breaks ties);
 //   build   Karras' binary radix tree over each instance's key segment
-//           (internal nodes of instance i live at [s_i, s_i + n_i - 1));
-//   refit   bottom-up with one arrival counter per internal node, in LDS
-//           for nodes whose key range lies inside one workgroup's chunk of
-//           sorted positions, in global memory for the few that straddle;
-//           a node's four-wide record is written with it;
+//           (internal nodes of instance i live at [s_i, s_i + n_i - 1)) with
+//           its boxes, from the leaves up, in LDS for subtrees inside one
+//           workgroup's chunk of sorted positions; a node's four-wide record is
+//           written with it;
 //   TLAS    the same builder over the instances' world-space boxes, with a
 //           30-bit Morton code (morton_of) per instance.
 #include <algorithm>
@@ -233,35 +232,38 @@ __device__ __forceinline__ void collapse4(const tc_bvh_node* nodes, uint32_t i, 
   gst_record(out + i, collapse4_of(gld_record(nodes + i), nodes));
 }
 
-// The tree of every instance and its boxes in two launches, with no
-// device-scope fence.
+// The tree of every instance and its boxes in two launches, from the leaves up
+// (Apetrei 2014) with Karras' (2012) node numbers, and with no device-scope
+// fence.
+//
+// A subtree covers sorted positions [l, r].  Keys l - 1 and l share a prefix of
+// some length, and so do keys r and r + 1; the longer of the two says whether
+// its sibling begins at r + 1 (it is a left child, node number r) or ends at
+// l - 1 (a right child, number l), so the boundary between the two names their
+// meeting place.  Of two siblings the second to arrive there makes their
+// parent, whose outer prefixes are the siblings'.  No node is searched for.
 //
 // k_blas_build: a workgroup owns a chunk of kRefitChunk sorted positions, one
-// thread per position.  It stages the chunk's keys and its leaves' boxes (from
-// their CLAS headers, which also give the leaf info words) in LDS; thread k
-// finds internal node k (Karras 2012) from the keys there, reading global keys
-// only where a range leaves the chunk.  Nodes whose key range lies inside the
-// chunk have their parents and children there as well, so topology, arrival
-// counts and boxes of the climbs from the leaves stay in LDS.  The binary and
-// four-wide records are written once every climb is done.  A node whose range
-// straddles chunks is described in memory by its thread: child words, which of
-// its children are final (leaves, or ranges inside one chunk), and the parent
-// of those that are not; with two final children it is pending, the entry of
-// the one chunk boundary that its range holds (its split).
-// With the tree in a launch before, 36 bytes a CLAS of topology went through
-// memory and every search waited for some twenty loads of keys one after
-// another: both took 60 us at 310,000 CLAS in 64 instances, 409 us at 3.3
-// million, 30 us at 8192 in one; now 48, 361 and 26 us.  In the last, staging
-// takes 3.2 us, the searches 9.6, the climbs 5.9 and the records 5.5.
-// Two workgroups of 16 waves share a CU (64 registers, 74 KB).
+// thread per position.  It stages the leaves' boxes (from their CLAS headers,
+// which also give the leaf info words) and the prefixes in LDS, the leaves
+// climb there, and the binary and four-wide records are written once every
+// climb is done.  Subtrees whose sibling reaches out of the chunk, some ten per
+// chunk boundary, are noted at their ends for the second launch.
+// With Karras' searches in a launch before, 36 bytes a CLAS of topology went
+// through memory, and one workgroup of 66 registers filled a CU; both took 67 us
+// at 310,000 CLAS in 64 instances, 470 us at 3.3 million, 31 us at 8192 in one,
+// with the searches in this launch 48, 360 and 25 us, and now 44, 314 and 18 us:
+// 290 bytes a CLAS at 3.0 TB/s at the largest, waits and the records' strided
+// stores (a fifth) at the smallest.  Two workgroups of 16 waves share a CU.
 //
-// k_blas_refit_top: one workgroup per instance climbs from its pending nodes
-// through the straddling nodes; each node's records are written where the node
-// is refit.
+// k_blas_refit_top: one workgroup per instance that lies in several chunks goes
+// on with the climbs.
 constexpr uint32_t kRefitChunkBits = 10;
 constexpr uint32_t kRefitChunk = 1u << kRefitChunkBits;
 constexpr uint32_t kRefitThreads = kRefitChunk;
 constexpr uint32_t kRefitTopThreads = 256;
+constexpr uint32_t kTopClimbs = 512;  // that meet in LDS
+constexpr uint32_t kTopTable = 2 * kTopClimbs;
 
 // Writes internal node `node` from its children's boxes.
 __device__ __forceinline__ tc_bvh_node write_node(const BvhArgs& a, uint32_t node, uint32_t c0w, uint32_t c1w,
@@ -280,115 +282,108 @@ __device__ __forceinline__ uint32_t box_at(uint32_t word, uint32_t first, uint32
   return first + (word & ~TC_BVH_LEAF) - c0 + ((word & TC_BVH_LEAF) ? kRefitChunk : 0u);
 }
 
+// Length of the common prefix of the keys at positions x and y of one
+// instance, plus one: of their Morton codes (the keys' high words are the
+// instance), of the positions where the codes are equal.
+__device__ __forceinline__ uint32_t key_prefix(uint32_t cx, uint32_t cy, uint32_t x, uint32_t y) {
+  const uint32_t v = cx ^ cy;
+  return 1u + (v ? __clz(v) : 32u + __clz(x ^ y));
+}
+
+// A subtree that waits for a sibling from outside its chunk: its other end,
+// from the chunk's start, and the prefix there.
+__device__ __forceinline__ uint32_t pack_wait(uint32_t far, uint32_t outer) { return 1u << 31 | outer << 16 | far; }
+
 __global__ __launch_bounds__(kRefitThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_blas_build(BvhArgs a) {
-  constexpr uint32_t kNone = ~0u;
-  __shared__ uint32_t s_key[kRefitChunk + 2];  // Morton codes of positions c0 - 1 .. c1
-  __shared__ uint32_t s_cnt[kRefitChunk];
+  constexpr uint32_t kNone = ~0u, kDone = ~0u;
   __shared__ tc_aabb s_box[2 * kRefitChunk + 1];  // internal nodes' union boxes, leaves' boxes, an empty one
   __shared__ uint32_t s_child[kRefitChunk][2];
-  __shared__ uint32_t s_parent[kRefitChunk], s_leafParent[kRefitChunk];  // in the chunk, or kNone
+  __shared__ uint32_t s_meet[kRefitChunk + 1];  // per boundary: 0, the subtree that waits there, or kDone
+  __shared__ uint8_t s_prefix[kRefitChunk + 4];  // per boundary: key_prefix of its two sides, 0 at an instance's ends
   const tc_scene_building* b = a.build;
   const uint32_t n = min(b->blasClusterCounter, a.capacity);
   const uint64_t* refs = ptr<const uint64_t>(b->blasClusterAddresses);
-  const uint32_t* codes = reinterpret_cast<const uint32_t*>(a.sortedKeys);  // the keys' low words
   const uint32_t j = threadIdx.x;
   if (j == 0)
     for (int q = 0; q < 3; q++) s_box[2 * kRefitChunk].lo[q] = INFINITY, s_box[2 * kRefitChunk].hi[q] = -INFINITY;
   for (uint32_t c0 = blockIdx.x * kRefitChunk; c0 < n; c0 += gridDim.x * kRefitChunk) {
-    const uint32_t c1 = min(c0 + kRefitChunk, n);
+    const uint32_t c1 = min(c0 + kRefitChunk, n), cnt = c1 - c0;
     const uint32_t k = c0 + j;
     uint32_t first = 0, last = 0;
-    s_cnt[j] = 0;
-    s_parent[j] = s_leafParent[j] = kNone;
-    if (j == 0) {
-      s_key[0] = c0 ? (uint32_t)gld(a.sortedKeys + c0 - 1) : 0u;
-      s_key[c1 - c0 + 1] = c1 < n ? (uint32_t)gld(a.sortedKeys + c1) : 0u;
-    }
+    bool valid = false;
+    s_child[j][0] = kNone;
+    s_meet[j] = 0;
+    if (j == 0) s_meet[kRefitChunk] = 0;
     if (k < c1) {
-      const uint64_t key = gld(a.sortedKeys + k);
+      const uint64_t key = gld(a.sortedKeys + k), before = gld(a.sortedKeys + (k ? k - 1 : 0u)),
+                     after = gld(a.sortedKeys + (k + 1 < n ? k + 1 : k));
       const uint64_t addr = gld(refs + gld(a.sortedVals + k));
-      s_key[j + 1] = (uint32_t)key;
       int64_t f, l;
       blas_segment(a, (uint32_t)(key >> 32), n, f, l);
       first = (uint32_t)f, last = (uint32_t)l;
+      valid = k >= first && k <= last;
+      s_prefix[j] = valid && k != first && before >> 32 == key >> 32
+                        ? (uint8_t)key_prefix((uint32_t)before, (uint32_t)key, k - 1, k)
+                        : (uint8_t)0;
+      if (k + 1 == c1)
+        s_prefix[cnt] = valid && k != last && k + 1 < n && after >> 32 == key >> 32
+                            ? (uint8_t)key_prefix((uint32_t)key, (uint32_t)after, k, k + 1)
+                            : (uint8_t)0;
       gst(a.leafAddr + k, addr);
       float lo[3], hi[3];
       leaf_box_at(a, k, addr, lo, hi);
       for (int q = 0; q < 3; q++) s_box[kRefitChunk + j].lo[q] = lo[q], s_box[kRefitChunk + j].hi[q] = hi[q];
     }
     __syncthreads();
-    // internal node k exists when k < last (a single CLAS is its instance's root)
-    bool local = false;
-    if (k < c1 && k >= first && k < last) {
-      const uint32_t ki = s_key[j + 1];
-      const int f = (int)first, l = (int)last, i = (int)k;
-      // common prefix of the keys at i and x: of the Morton codes, as the keys
-      // of an instance share their high words; equal codes by position; -1
-      // outside the instance
-      const auto prefix = [&](int x) {
-        if (x < f || x > l) return -1;
-        const uint32_t o = (uint32_t)x + 1 - c0;
-        const uint32_t v = ki ^ (o <= c1 - c0 + 1 ? s_key[o] : gld(codes + 2 * (uint64_t)x));
-        return v ? __clz(v) : 32 + __clz((uint32_t)i ^ (uint32_t)x);
-      };
-      const int next = prefix(i + 1), prev = prefix(i - 1);
-      const int d = next - prev >= 0 ? 1 : -1, dmin = d > 0 ? prev : next;
-      int far = 2;
-      while (prefix(i + far * d) > dmin) far *= 2;
-      int len = 0;
-      for (int t = far / 2; t >= 1; t /= 2)
-        if (prefix(i + (len + t) * d) > dmin) len += t;
-      const int dnode = prefix(i + len * d);
-      int s = 0, t = len;
-      do {
-        t = (t + 1) / 2;
-        if (prefix(i + (s + t) * d) > dnode) s += t;
-      } while (t > 1);
-      const uint32_t gamma = (uint32_t)(i + s * d + min(d, 0));
-      const uint32_t lo = (uint32_t)min(i, i + len * d), hi = (uint32_t)max(i, i + len * d);
-      const bool leaf0 = lo == gamma, leaf1 = hi == gamma + 1;
-      const uint32_t w0 = (leaf0 ? TC_BVH_LEAF : 0u) | (gamma - first), w1 = (leaf1 ? TC_BVH_LEAF : 0u) | (gamma + 1 - first);
-      local = lo >= c0 && hi < c1;
-      if (local) {
-        s_child[j][0] = w0, s_child[j][1] = w1;
-        (leaf0 ? s_leafParent : s_parent)[gamma - c0] = j;
-        (leaf1 ? s_leafParent : s_parent)[gamma + 1 - c0] = j;
-      } else {
-        const bool final0 = lo >> kRefitChunkBits == gamma >> kRefitChunkBits;
-        const bool final1 = (gamma + 1) >> kRefitChunkBits == hi >> kRefitChunkBits;
-        gst(a.child + 2 * k, w0);
-        gst(a.child + 2 * k + 1, w1);
-        gst(a.counter + k, (final0 ? 1u : 0u) + (final1 ? 1u : 0u));
-        if (!final0) gst(a.parent + gamma, k);
-        if (!final1) gst(a.parent + gamma + 1, k);
-        if (((gamma + 1) & (kRefitChunk - 1)) == 0) gst(a.pendingList + ((gamma + 1) >> kRefitChunkBits), final0 && final1 ? k : kNone);
-      }
-    }
-    __syncthreads();
-    if (k < c1 && first != last) {
-      uint32_t ln = s_leafParent[j];
-      while (ln != kNone) {
-        // the arrival orders LDS only (s_box, s_cnt)
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        if (atomicAdd(&s_cnt[ln], 1u) == 0) break;  // first arrival stops
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        const tc_aabb &b0 = s_box[box_at(s_child[ln][0], first, c0)], &b1 = s_box[box_at(s_child[ln][1], first, c0)];
-        tc_aabb self;
-        for (int q = 0; q < 3; q++) self.lo[q] = fminf(b0.lo[q], b1.lo[q]), self.hi[q] = fmaxf(b0.hi[q], b1.hi[q]);
-        s_box[ln] = self;
-        if (c0 + ln == first) {  // instance root
-          gst_record(a.nodeBox + first, self);
+    if (valid && first != last) {  // (a single CLAS is its instance's root)
+      uint32_t l = j, r = j;
+      while (true) {
+        const uint32_t dl = s_prefix[l], dr = s_prefix[r + 1];
+        if ((dl | dr) == 0) break;  // the instance's root, written where it was made
+        const bool left = dr > dl;
+        const uint32_t at = left ? r + 1 : l;
+        const uint32_t mine = 1u + (left ? l : r) + (left ? 1u << 16 : 0u);
+        if (at == 0 || at == cnt) {  // the sibling lies in another chunk
+          s_meet[at] = mine;
           break;
         }
-        ln = s_parent[ln];
+        // the meeting orders LDS only (s_box, s_meet)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        const uint32_t other = atomicExch(&s_meet[at], mine);
+        if (other == 0) break;  // first to arrive
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        s_meet[at] = kDone;
+        if (left)
+          r = (other - 1) & 0xFFFFu;
+        else
+          l = (other - 1) & 0xFFFFu;
+        const uint32_t ul = s_prefix[l], ur = s_prefix[r + 1];
+        const bool leaf0 = l + 1 == at, leaf1 = r == at, root = (ul | ur) == 0;
+        const tc_aabb &b0 = s_box[at - 1 + (leaf0 ? kRefitChunk : 0u)], &b1 = s_box[at + (leaf1 ? kRefitChunk : 0u)];
+        tc_aabb self;
+        for (int q = 0; q < 3; q++) self.lo[q] = fminf(b0.lo[q], b1.lo[q]), self.hi[q] = fmaxf(b0.hi[q], b1.hi[q]);
+        const uint32_t node = !root && ur > ul ? r : l;
+        s_box[node] = self;
+        s_child[node][0] = (leaf0 ? TC_BVH_LEAF : 0u) | (c0 + at - 1 - first);
+        s_child[node][1] = (leaf1 ? TC_BVH_LEAF : 0u) | (c0 + at - first);
+        if (root) gst_record(a.nodeBox + first, self);
       }
     }
     __syncthreads();
-    // binary and four-wide records of the chunk's local internal nodes, one
-    // per thread, from LDS (the grandchildren of a local node lie in the
+    // the subtrees that end or begin at this position and wait for a sibling
+    // from outside (an instance inside the chunk has none)
+    const uint32_t chunks = (last >> kRefitChunkBits) - (first >> kRefitChunkBits);
+    if (valid && chunks != 0) {
+      const uint32_t me = s_meet[j + 1], mb = s_meet[j];
+      const uint32_t fe = (me - 1) & 0xFFFFu, fb = (mb - 1) & 0xFFFFu;
+      gst(a.waitEnd + k, me != 0 && me != kDone && (me - 1) >> 16 != 0 ? pack_wait(fe, s_prefix[fe]) : 0u);
+      gst(a.waitBegin + k, mb != 0 && mb != kDone && (mb - 1) >> 16 == 0 ? pack_wait(fb, s_prefix[fb + 1]) : 0u);
+      if (chunks > kTopClimbs) gst(a.meet + k, (uint64_t)0);
+    }
+    // binary and four-wide records of the chunk's internal nodes, one per thread, from LDS (the grandchildren of a local node lie in the
     // chunk): neighbouring threads write neighbouring records, and the climbs,
     // in which few lanes are left after a level or two, store nothing
-    if (local) {
+    if (s_child[j][0] != kNone) {
       const uint32_t cw[2] = {s_child[j][0], s_child[j][1]};
       const uint32_t at[2] = {box_at(cw[0], first, c0), box_at(cw[1], first, c0)};
       write_node(a, k, cw[0], cw[1], s_box[at[0]], s_box[at[1]]);
@@ -435,15 +430,15 @@ __device__ __forceinline__ RefitChild refit_child(const tc_bvh_node& m, uint32_t
   return r;
 }
 // A child that is final before this launch, from memory.
-__device__ __forceinline__ RefitChild refit_child_at(const BvhArgs& a, int64_t first, uint32_t word) {
+__device__ __forceinline__ RefitChild refit_child_at(const BvhArgs& a, uint32_t first, uint32_t word) {
   RefitChild r;
   if (word & TC_BVH_LEAF) {
     float lo[3], hi[3];
-    leaf_box(a, (uint32_t)first + (word & ~TC_BVH_LEAF), lo, hi);
+    leaf_box(a, first + (word & ~TC_BVH_LEAF), lo, hi);
     r.s[0] = r.s[1] = slot4(lo, hi, word);
     r.word = word;
   } else {
-    r = refit_child(gld_record(a.nodes + (uint32_t)first + word), word);
+    r = refit_child(gld_record(a.nodes + first + word), word);
   }
   return r;
 }
@@ -455,13 +450,13 @@ __device__ __forceinline__ tc_aabb union_box(const Slot4& x, const Slot4& y) {
 
 // Refit of straddling node `node`: its binary record (returned) and its
 // four-wide one.
-__device__ __forceinline__ tc_bvh_node refit_top_node(const BvhArgs& a, uint32_t node, int64_t first, const RefitChild& c0,
+__device__ __forceinline__ tc_bvh_node refit_top_node(const BvhArgs& a, uint32_t node, uint32_t first, const RefitChild& c0,
                                                       const RefitChild& c1) {
   const tc_bvh_node out =
       write_node(a, node, c0.word, c1.word, union_box(c0.s[0], c0.s[1]), union_box(c1.s[0], c1.s[1]));
   gst_record(a.nodes4 + node,
              make4((c0.word & TC_BVH_LEAF) != 0, c0.s[0], c0.s[1], (c1.word & TC_BVH_LEAF) != 0, c1.s[0], c1.s[1]));
-  if ((int64_t)node == first) {  // instance root, read by the TLAS
+  if (node == first) {  // instance root, read by the TLAS
     tc_aabb self;
     for (int q = 0; q < 3; q++) self.lo[q] = fminf(out.lo0[q], out.lo1[q]), self.hi[q] = fmaxf(out.hi0[q], out.hi1[q]);
     gst_record(a.nodeBox + node, self);
@@ -469,94 +464,95 @@ __device__ __forceinline__ tc_bvh_node refit_top_node(const BvhArgs& a, uint32_t
   return out;
 }
 
-// A climb goes up through nodes with one straddling child (the other is final)
-// and meets another climb at nodes with two: there the first to arrive leaves
-// its record in LDS, in a table by node, and stops.  What bounds a climb is its
-// chain of memory round trips, some 15 levels of them at an instance of 5000
-// CLAS: the topology and a final sibling's record are fetched together, a level
-// ahead, the record of the child just refit stays in registers, and no climb
-// reads a record that the launch has stored.  Measured: 64 instances of 4840
-// CLAS 42.7 -> 33.7 us, 500 meshes 30 -> 17 us, 5 instances of 5200 23 ->
-// 16.6 us, 64 instances of 51,000 160 -> 144 us.
-// More climbs than kTopMeets (half a million CLAS in one instance) meet in
-// global memory instead.
-constexpr uint32_t kTopMeets = 512;
-constexpr uint32_t kTopTable = 2 * kTopMeets;
-
+// The climbs of an instance, one from each chunk boundary where the subtrees on
+// both sides wait for each other.  Higher up, a sibling is a subtree that waits
+// (read with its record ahead of this level's stores: one round trip a level),
+// or another climb's: two climbs meet in LDS, where the first leaves its
+// record, far end and outer prefix in its slot and the slot's number in a table
+// by boundary.  More climbs than kTopClimbs (half a million CLAS in one
+// instance) meet in global memory.
+// Bound by some 16 levels of a round trip and the stores before it.  64
+// instances of up to 130,000 CLAS 42.7 -> 28.6 us, 500 meshes 30 -> 15.5, 5
+// instances of 5200 23 -> 15, 64 instances of 51,000 160 -> 122 us.  With a climb
+// for every waiting subtree instead, which needs no look-ups, 288 us and 1547 us:
+// most lanes of a wave stop at their first meeting.
 __global__ __launch_bounds__(kRefitTopThreads) void k_blas_refit_top(BvhArgs a) {
-  __shared__ uint32_t s_node[kTopTable], s_meet[kTopTable];
-  __shared__ __align__(16) tc_bvh_node s_rec[kTopMeets];
+  __shared__ uint32_t s_at[kTopTable];    // boundary, or ~0
+  __shared__ uint32_t s_slot[kTopTable];  // 0, or the slot that waits there + 1
+  __shared__ __align__(16) tc_bvh_node s_rec[kTopClimbs];  // (_pad0: far end, _pad1: outer prefix)
   const uint32_t inst = blockIdx.x;
   if (inst >= a.numInstances) return;
   const tc_scene_building* b = a.build;
   const uint32_t n = min(b->blasClusterCounter, a.capacity);
   const tc_blas_build_info& bi = ptr<const tc_blas_build_info>(b->blasBuildInfos)[inst];
   if (bi.clusterReferencesCount < 2) return;
-  const int64_t first = (int64_t)((bi.clusterReferences - b->blasClusterAddresses) / 8);
-  if (first >= (int64_t)n) return;
-  // chunk boundaries inside the instance, with a pending node or none each
-  const uint32_t base = ((uint32_t)first >> kRefitChunkBits) + 1;
-  const uint32_t count = (((uint32_t)first + bi.clusterReferencesCount - 1) >> kRefitChunkBits) + 1 - base;
+  const int64_t first64 = (int64_t)((bi.clusterReferences - b->blasClusterAddresses) / 8);
+  if (first64 >= (int64_t)n) return;
+  const uint32_t first = (uint32_t)first64, last = min(first + bi.clusterReferencesCount, n) - 1;
+  const uint32_t chunk0 = first >> kRefitChunkBits, count = (last >> kRefitChunkBits) - chunk0;
   if (count == 0) return;
-  const bool meetLds = count <= kTopMeets;
-  if (meetLds)
-    for (uint32_t w = threadIdx.x; w < kTopTable; w += kRefitTopThreads) s_node[w] = ~0u, s_meet[w] = 0;
+  const bool lds = count <= kTopClimbs;
+  if (lds)
+    for (uint32_t w = threadIdx.x; w < kTopTable; w += kRefitTopThreads) s_at[w] = ~0u, s_slot[w] = 0;
   __syncthreads();
   for (uint32_t t = threadIdx.x; t < count; t += kRefitTopThreads) {
-    uint32_t node = gld(a.pendingList + base + t);
-    if (node == ~0u) continue;
-    uint32_t up = gld(a.parent + node);  // (the root's is not followed)
-    uint32_t w0 = gld(a.child + 2 * node), w1 = gld(a.child + 2 * node + 1), nup = 0, prior = 0;
-    RefitChild c0 = refit_child_at(a, first, w0), c1 = refit_child_at(a, first, w1);
-    if ((int64_t)node != first) {
-      w0 = gld(a.child + 2 * up), w1 = gld(a.child + 2 * up + 1);
-      nup = gld(a.parent + up);
-      prior = gld(a.counter + up);
-    }
+    uint32_t at = (chunk0 + 1 + t) << kRefitChunkBits;
+    const uint32_t we = gld(a.waitEnd + at - 1), wb = gld(a.waitBegin + at);
+    if (we == 0 || wb == 0) continue;
+    uint32_t l = at - kRefitChunk + (we & 0xFFFFu), r = at + (wb & 0xFFFFu);
+    uint32_t dl = we >> 16 & 0xFFu, dr = wb >> 16 & 0xFFu;
+    RefitChild c0 = refit_child_at(a, first, (l + 1 == at ? TC_BVH_LEAF : 0u) | (at - 1 - first));
+    RefitChild c1 = refit_child_at(a, first, (r == at ? TC_BVH_LEAF : 0u) | (at - first));
     while (true) {
-      const bool root = (int64_t)node == first;
-      const uint32_t self = node - (uint32_t)first;
-      const bool right = w1 == self;  // (an internal child's word is its index)
-      const uint32_t sib = right ? w0 : w1;
-      const bool final = !root && meetLds && prior != 0, leaf = (sib & TC_BVH_LEAF) != 0;
-      // the sibling's record, if it is final, and the next level's topology,
-      // before this level's stores
-      const tc_bvh_node sibRec = gld_record(a.nodes + (uint32_t)first + (final && !leaf ? sib : 0u));
-      const uint32_t at = root || (int64_t)up == first ? node : nup;
-      const uint32_t x0 = gld(a.child + 2 * at), x1 = gld(a.child + 2 * at + 1), xup = gld(a.parent + at),
-                     xprior = gld(a.counter + at);
-      const tc_bvh_node rec = refit_top_node(a, node, first, c0, c1);
+      const bool root = (dl | dr) == 0, left = dr > dl;
+      const uint32_t node = !root && left ? r : l;  // (the root's l is `first`)
+      at = left ? r + 1 : l;
+      // the sibling's end there: its node's number, or its leaf
+      const uint32_t p = root ? first : (left ? at : at - 1);
+      const uint32_t wait = gld((left ? a.waitBegin : a.waitEnd) + p);
+      const tc_bvh_node sibRec = gld_record(a.nodes + p);
+      const tc_bvh_node made = refit_top_node(a, node, first, c0, c1);
       if (root) break;
-      RefitChild other;
-      if (final) {
-        other = refit_child(sibRec, sib);
-        if (leaf) other = refit_child_at(a, first, sib);
-      } else if (!meetLds) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        if (atomicAdd(&a.counter[up], 1u) == 0) break;  // first arrival stops
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        other = refit_child_at(a, first, sib);
-      } else {
-        uint32_t h = (up * 2654435761u) >> (32 - 10);
+      uint32_t far, outer;
+      RefitChild sib;
+      if (wait != 0) {
+        far = (p & ~(kRefitChunk - 1)) + (wait & 0xFFFFu), outer = wait >> 16 & 0xFFu;
+        sib = refit_child(sibRec, p - first);
+        if (far == p) sib = refit_child_at(a, first, TC_BVH_LEAF | (p - first));
+      } else if (lds) {
+        uint32_t h = (at * 2654435761u) >> (32 - 10);
         static_assert(kTopTable == 1u << 10, "the hash's bits");
-        while (true) {  // at most kTopMeets - 1 nodes have two climbs
-          const uint32_t seen = atomicCAS(&s_node[h], ~0u, up);
-          if (seen == ~0u || seen == up) break;
+        while (true) {  // at most kTopClimbs - 1 boundaries
+          const uint32_t seen = atomicCAS(&s_at[h], ~0u, at);
+          if (seen == ~0u || seen == at) break;
           h = (h + 1) & (kTopTable - 1);
         }
-        // the climb's own record: it stays in place once the climb stops
-        s_rec[t] = rec;
+        // the climb's own slot: it stays in place once the climb stops
+        tc_bvh_node own = made;
+        own._pad0 = left ? l : r, own._pad1 = left ? dl : dr;
+        s_rec[t] = own;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        const uint32_t met = atomicExch(&s_meet[h], t + 1);
-        if (met == 0) break;  // first arrival stops
+        const uint32_t met = atomicExch(&s_slot[h], t + 1);
+        if (met == 0) break;  // first to arrive
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        other = refit_child(s_rec[met - 1], sib);
+        const tc_bvh_node rec = s_rec[met - 1];
+        far = rec._pad0, outer = rec._pad1;
+        sib = refit_child(rec, p - first);
+      } else {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        const uint64_t met = atomicExch(reinterpret_cast<unsigned long long*>(a.meet + at),
+                                        1ull << 63 | (unsigned long long)(left ? dl : dr) << 32 | (left ? l : r));
+        if (met == 0) break;  // first to arrive
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        far = (uint32_t)met, outer = (uint32_t)(met >> 32) & 0xFFu;
+        sib = refit_child_at(a, first, p - first);  // (a climb's subtree is no leaf)
       }
-      const RefitChild mine = refit_child(rec, self);
-      c0 = right ? other : mine, c1 = right ? mine : other;
-      node = up;
-      up = nup;
-      w0 = x0, w1 = x1, nup = xup, prior = xprior;
+      const RefitChild mine = refit_child(made, node - first);
+      c0 = left ? mine : sib, c1 = left ? sib : mine;
+      if (left)
+        r = far, dr = outer;
+      else
+        l = far, dl = outer;
     }
   }
 }
@@ -853,10 +849,9 @@ AccelLayout accel_layout(uint32_t capacity, uint32_t numInstances) {
   put(L.blasLeaves, c * 8);
   put(L.blasLeafInfo, c * 8);
   put(L.nodeBox, c * sizeof(tc_aabb));
-  put(L.child, 2 * c * 4);
-  put(L.parent, c * 4);
-  put(L.counter, c * 4);
-  put(L.pendingList, (c / kRefitChunk + 2) * 4);
+  put(L.waitEnd, c * 4);
+  put(L.waitBegin, c * 4);
+  put(L.meet, c * 8);
   put(L.tlasInstances, n * sizeof(tc_tlas_instance));
   put(L.tlasNodes, n * sizeof(tc_bvh_node));
   put(L.tlasNodes4, n * sizeof(tc_bvh4_node));
@@ -937,10 +932,9 @@ static tc_status accel_build(const tc_bindings* b, tc_config config, const tc_ac
   a.vals = sb.vals[0];
   a.leafAddr = reinterpret_cast<uint64_t*>(m + L.blasLeaves);
   a.leafInfo = reinterpret_cast<uint64_t*>(m + L.blasLeafInfo);
-  a.child = reinterpret_cast<uint32_t*>(m + L.child);
-  a.parent = reinterpret_cast<uint32_t*>(m + L.parent);
-  a.counter = reinterpret_cast<uint32_t*>(m + L.counter);
-  a.pendingList = reinterpret_cast<uint32_t*>(m + L.pendingList);
+  a.waitEnd = reinterpret_cast<uint32_t*>(m + L.waitEnd);
+  a.waitBegin = reinterpret_cast<uint32_t*>(m + L.waitBegin);
+  a.meet = reinterpret_cast<uint64_t*>(m + L.meet);
   a.nodes = reinterpret_cast<tc_bvh_node*>(m + L.blasNodes);
   a.nodes4 = reinterpret_cast<tc_bvh4_node*>(m + L.blasNodes4);
   a.nodeBox = reinterpret_cast<tc_aabb*>(m + L.nodeBox);
