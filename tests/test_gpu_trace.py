@@ -514,3 +514,42 @@ def test_refit_of_one_instance(qx, qz, px):
         got = [(int(wide[i]["child"][k]), tuple(wide[i]["lo"][:, k]), tuple(wide[i]["hi"][:, k])) for k in range(len(want))]
         assert got == want
         assert all(int(wide[i]["child"][k]) == abi.BVH4_EMPTY for k in range(len(want), 4))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 3, 63, 65, 257, 512, 513, 1024])
+def test_small_tlas_trees(n):
+    """One-workgroup TLAS builds over instance counts at the edges of its rank
+    shares (several threads, two and one thread to an instance): every instance
+    is a leaf once, inner boxes are the unions below them, the four-wide records
+    list the grandchildren."""
+    host = lattice_scene(n)
+    g = harness.GpuFrame(host, harness.small_config())
+    try:
+        g.run(host.frame(), stages="accel")
+        arr = g.accel_arrays()
+    finally:
+        g.close()
+    if n == 1:
+        assert arr["tlasRoot"] == abi.BVH_LEAF
+        return
+    nodes = arr["tlasNodes"][:n - 1]
+    seen, inner = [], set()
+
+    def visit(word):
+        assert word < n - 1 and word not in inner
+        inner.add(word)
+        nd = nodes[word]
+        for c in ("0", "1"):
+            ch = int(nd["child" + c])
+            if ch & abi.BVH_LEAF:
+                seen.append(ch & ~abi.BVH_LEAF)
+            else:
+                lo, hi = visit(ch)
+                assert np.array_equal(nd["lo" + c], lo) and np.array_equal(nd["hi" + c], hi)
+        return np.minimum(nd["lo0"], nd["lo1"]), np.maximum(nd["hi0"], nd["hi1"])
+
+    assert arr["tlasRoot"] == 0
+    visit(0)
+    assert sorted(seen) == list(range(n)) and len(inner) == n - 1
+    check_wide(nodes, arr["tlasNodes4"][:n - 1])

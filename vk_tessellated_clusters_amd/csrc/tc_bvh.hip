@@ -557,8 +557,8 @@ __global__ __launch_bounds__(kRefitTopThreads) void k_blas_refit_top(BvhArgs a) 
   }
 }
 
-// TLAS record and world box of instance i.
-__device__ void tlas_prep_one(const BvhArgs& a, const float* xforms /* 24 floats per instance */, uint32_t i) {
+// TLAS record and world box (returned as well) of instance i.
+__device__ __forceinline__ tc_aabb tlas_prep_one(const BvhArgs& a, const float* xforms /* 24 floats per instance */, uint32_t i) {
   const tc_blas_build_info bi = ptr<const tc_blas_build_info>(a.build->blasBuildInfos)[i];
   const uint32_t first = (uint32_t)((bi.clusterReferences - a.build->blasClusterAddresses) / 8);
   const uint32_t cnt = bi.clusterReferencesCount;
@@ -601,6 +601,7 @@ __device__ void tlas_prep_one(const BvhArgs& a, const float* xforms /* 24 floats
     wb.lo[q] = wlo[q] - e, wb.hi[q] = whi[q] + e;
   }
   a.tlasLeafBox[i] = wb;
+  return wb;
 }
 
 // Per-instance TLAS records and world boxes (one thread per instance).
@@ -714,32 +715,38 @@ __global__ void k_tlas_root(BvhArgs a) {
 
 // The whole TLAS in one workgroup for up to kTlasRankSort instances, one
 // thread per instance: records and world boxes, scene bounds and keys, the
-// rank sort, hierarchy, refit and four-wide view, the steps the launches
-// above make, separated by workgroup barriers instead of kernel boundaries.
+// rank sort, the tree with its boxes from the leaves up (as k_blas_build), and
+// the binary and four-wide records.  One workgroup's chain of waits: of 28.8 us
+// at 500 instances the ranks took 6.9 (a key of LDS after another), Karras'
+// searches 4.0, the climbs with their record stores 6.8, reading the boxes back
+// 1.9.  Every thread now ranks four keys at a time, with several threads to an
+// instance where there are fewer than half as many as threads: 500 instances
+// 29.9 -> 24.3 us, 64 14.5 -> 9.5, 20 10.9 -> 7.3, 8 9.4 -> 6.8.
 __global__ __launch_bounds__(kTlasRankSort) void k_tlas_build_small(BvhArgs a, const float* xforms) {
   __shared__ float s_b[6][kTlasRankSort / kWave];
-  __shared__ uint64_t s_key[kTlasRankSort], s_sorted[kTlasRankSort];
-  __shared__ uint32_t s_val[kTlasRankSort], s_cnt[kTlasRankSort];
-  __shared__ uint32_t s_child[2 * kTlasRankSort], s_parent[2 * kTlasRankSort];
-  __shared__ tc_aabb s_leaf[kTlasRankSort], s_box[kTlasRankSort];  // by instance, by internal node
+  __shared__ __align__(16) uint64_t s_key[kTlasRankSort + 4];
+  __shared__ uint64_t s_sorted[kTlasRankSort];
+  __shared__ uint32_t s_rank[kTlasRankSort], s_val[kTlasRankSort];
+  __shared__ uint32_t s_child[kTlasRankSort][2], s_meet[kTlasRankSort];
+  __shared__ uint8_t s_prefix[kTlasRankSort + 4];
+  __shared__ tc_aabb s_leaf[kTlasRankSort], s_box[kTlasRankSort];  // by sorted position, by internal node
   const uint32_t n = a.numInstances, i = threadIdx.x, lane = lane_id(), wave = threadIdx.x / kWave;
-  if (i < n) tlas_prep_one(a, xforms, i);
-  if (i == 0) {
-    a.tlasRoot[0] = n == 1 ? (TC_BVH_LEAF | 0u) : 0u;
-    a.tlasRoot[1] = n;
-  }
-  __syncthreads();
-  // scene bounds of the instance box centres (k_tlas_keys)
   tc_aabb bx;
   bool empty = true;
   float c[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
   if (i < n) {
-    bx = a.tlasLeafBox[i];
-    s_leaf[i] = bx;
+    bx = tlas_prep_one(a, xforms, i);
     empty = !(bx.lo[0] <= bx.hi[0]);
     if (!empty)
       for (int q = 0; q < 3; q++) c[q] = c[3 + q] = (bx.lo[q] + bx.hi[q]) * 0.5f;
   }
+  if (i == 0) {
+    a.tlasRoot[0] = n == 1 ? (TC_BVH_LEAF | 0u) : 0u;
+    a.tlasRoot[1] = n;
+  }
+  s_rank[i] = 0;
+  s_meet[i] = 0;
+  // scene bounds of the instance box centres (k_tlas_keys)
 #pragma unroll
   for (int q = 0; q < 3; q++) {
     for (int d = 1; d < kWave; d <<= 1) {
@@ -755,59 +762,78 @@ __global__ __launch_bounds__(kTlasRankSort) void k_tlas_build_small(BvhArgs a, c
     for (int q = 0; q < 3; q++) slo[q] = fminf(slo[q], s_b[q][w]), shi[q] = fmaxf(shi[q], s_b[3 + q][w]);
   // keys (empty instances sort last and are never entered), then ranks
   if (i < n) s_key[i] = empty ? (0xFFFFFFFFull << 32) | i : ((uint64_t)morton_of(bx.lo, bx.hi, slo, shi) << 32) | i;
+  if (i < 4) s_key[n + i] = ~0ull;  // above every key
+  __syncthreads();
+  {
+    // thread i ranks key i % span among its share of the keys
+    uint32_t span = kWave;
+    while (span < n) span *= 2;
+    const uint32_t me = i % span, share = ((n + kTlasRankSort / span - 1) / (kTlasRankSort / span) + 3u) & ~3u;
+    const uint32_t j0 = i / span * share, j1 = min(j0 + share, (n + 3u) & ~3u);
+    if (me < n && j0 < j1) {
+      const uint64_t k = s_key[me];
+      uint32_t rank = 0;
+      for (uint32_t j = j0; j < j1; j += 4) {
+        const ulonglong2 x = *reinterpret_cast<const ulonglong2*>(s_key + j), y = *reinterpret_cast<const ulonglong2*>(s_key + j + 2);
+        rank += (x.x < k ? 1u : 0u) + (x.y < k ? 1u : 0u) + (y.x < k ? 1u : 0u) + (y.y < k ? 1u : 0u);
+      }
+      atomicAdd(&s_rank[me], rank);
+    }
+  }
   __syncthreads();
   if (i < n) {
+    const uint32_t rank = s_rank[i];
     const uint64_t k = s_key[i];
-    uint32_t rank = 0;
-    for (uint32_t j = 0; j < n; j++) rank += s_key[j] < k ? 1u : 0u;
     a.tlasKeys[rank] = k;
     a.tlasVals[rank] = i;
     s_sorted[rank] = k;
     s_val[rank] = i;
+    s_leaf[rank] = bx;
   }
   __syncthreads();
-  // hierarchy over the sorted keys (as k_tlas_hierarchy), refit (as
-  // tlas_refit_leaf) and four-wide view, with the topology, counters and
-  // boxes in LDS: a climb waits on no global load
   if (i < n) {
-    s_cnt[i] = 0;
-    if (i + 1 < n) karras_node(s_sorted, 0, (int64_t)n - 1, i, s_child, s_parent, n);
+    s_prefix[i] = i ? (uint8_t)(1 + __clzll(s_sorted[i - 1] ^ s_sorted[i])) : (uint8_t)0;
+    if (i + 1 == n) s_prefix[n] = 0;
   }
   __syncthreads();
-  // a TLAS leaf names its instance: the sorted position's value
-  const auto leaf_word = [&](uint32_t w) { return (w & TC_BVH_LEAF) ? (TC_BVH_LEAF | s_val[w & ~TC_BVH_LEAF]) : w; };
-  const auto box_of = [&](uint32_t w) -> const tc_aabb& {
-    return (w & TC_BVH_LEAF) ? s_leaf[s_val[w & ~TC_BVH_LEAF]] : s_box[w];
-  };
-  if (i < n && n > 1) {
-    uint32_t node = s_parent[n + i];
+  const auto box_of = [&](uint32_t w) -> const tc_aabb& { return (w & TC_BVH_LEAF) ? s_leaf[w & ~TC_BVH_LEAF] : s_box[w]; };
+  if (i < n) {
+    uint32_t l = i, r = i;
     while (true) {
+      const uint32_t dl = s_prefix[l], dr = s_prefix[r + 1];
+      if ((dl | dr) == 0) break;  // the root (or the only instance)
+      const bool left = dr > dl;
+      const uint32_t at = left ? r + 1 : l;
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-      if (atomicAdd(&s_cnt[node], 1u) == 0) break;
+      const uint32_t other = atomicExch(&s_meet[at], 1u + (left ? l : r));
+      if (other == 0) break;  // first to arrive
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-      const uint32_t cw[2] = {s_child[2 * node], s_child[2 * node + 1]};
-      float lo[2][3], hi[2][3];
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const tc_aabb& bx = box_of(cw[c]);
-        for (int q = 0; q < 3; q++) lo[c][q] = bx.lo[q], hi[c][q] = bx.hi[q];
-      }
-      tc_bvh_node out;
-      for (int q = 0; q < 3; q++) out.lo0[q] = lo[0][q], out.hi0[q] = hi[0][q], out.lo1[q] = lo[1][q], out.hi1[q] = hi[1][q];
-      out.child0 = leaf_word(cw[0]);
-      out.child1 = leaf_word(cw[1]);
-      out._pad0 = out._pad1 = 0;
-      gst_record(a.tlasNodes + node, out);
+      if (left)
+        r = other - 1;
+      else
+        l = other - 1;
+      const uint32_t ul = s_prefix[l], ur = s_prefix[r + 1];
+      const uint32_t w0 = (l + 1 == at ? TC_BVH_LEAF : 0u) | (at - 1), w1 = (r == at ? TC_BVH_LEAF : 0u) | at;
+      const tc_aabb &b0 = box_of(w0), &b1 = box_of(w1);
       tc_aabb self;
-      for (int q = 0; q < 3; q++) self.lo[q] = fminf(lo[0][q], lo[1][q]), self.hi[q] = fmaxf(hi[0][q], hi[1][q]);
+      for (int q = 0; q < 3; q++) self.lo[q] = fminf(b0.lo[q], b1.lo[q]), self.hi[q] = fmaxf(b0.hi[q], b1.hi[q]);
+      const uint32_t node = ur > ul ? r : l;  // (the root's l is 0)
       s_box[node] = self;
-      if (node == 0) break;
-      node = s_parent[node];
+      s_child[node][0] = w0, s_child[node][1] = w1;
     }
   }
   __syncthreads();
   if (i + 1 < n) {
-    const uint32_t cw[2] = {s_child[2 * i], s_child[2 * i + 1]};
+    // a TLAS leaf names its instance: the sorted position's value
+    const auto leaf_word = [&](uint32_t w) { return (w & TC_BVH_LEAF) ? (TC_BVH_LEAF | s_val[w & ~TC_BVH_LEAF]) : w; };
+    const uint32_t cw[2] = {s_child[i][0], s_child[i][1]};
+    const tc_aabb &b0 = box_of(cw[0]), &b1 = box_of(cw[1]);
+    tc_bvh_node out;
+    for (int q = 0; q < 3; q++) out.lo0[q] = b0.lo[q], out.hi0[q] = b0.hi[q], out.lo1[q] = b1.lo[q], out.hi1[q] = b1.hi[q];
+    out.child0 = leaf_word(cw[0]);
+    out.child1 = leaf_word(cw[1]);
+    out._pad0 = out._pad1 = 0;
+    gst_record(a.tlasNodes + i, out);
     Slot4 gs[2][2];
 #pragma unroll
     for (int c = 0; c < 2; c++) {
@@ -817,7 +843,7 @@ __global__ __launch_bounds__(kTlasRankSort) void k_tlas_build_small(BvhArgs a, c
       } else {
 #pragma unroll
         for (int d = 0; d < 2; d++) {
-          const uint32_t gw = s_child[2 * cw[c] + d];
+          const uint32_t gw = s_child[cw[c]][d];
           const tc_aabb& bx = box_of(gw);
           gs[c][d] = slot4(bx.lo, bx.hi, leaf_word(gw));
         }
