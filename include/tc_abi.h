@@ -602,7 +602,7 @@ typedef struct tc_tuning {
   uint32_t clasWavesPerCU;         /* CLAS build, one wave per CLAS */
   uint32_t traceBlocksPerCU;       /* traversal workgroups per CU */
   uint32_t traceThreads;           /* traversal workgroup size */
-  uint32_t bvhBlocksPerCU;         /* BVH keys / hierarchy / collapse */
+  uint32_t bvhBlocksPerCU;         /* BVH keys of tc_accel_build */
   /* Sleeps before a wait of the persistent split gives up and flags the
    * frame (TC_READBACK_ERROR_SPLIT_WAIT); default 2^24, and 0 in
    * tc_set_tuning restores it.  Not a performance knob: only failure-path

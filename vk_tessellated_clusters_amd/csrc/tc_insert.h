@@ -13,8 +13,9 @@
 //     their final places and counts the keys' Morton digits, so neither the
 //     scatter, the key launch (which read every header again) nor an upsweep is
 //     left.
-// Launches from the CLAS to the hierarchy: one instance 10 -> 4, up to 256
-// instances 10 -> 5, more 13 -> 7.
+// Launches from the CLAS to the tree: one instance 10 -> 4, up to 256 instances
+// 10 -> 5, more 13 -> 7.  Frames: icosphere at 320 x 180 260 -> 242 us, grid64 1012
+// -> 986, 500 meshes 1610 -> 1582, patch field at 3840 x 2160 6747 -> 6550.
 #pragma once
 
 #include "tc_sort.h"
