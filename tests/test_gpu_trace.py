@@ -553,3 +553,36 @@ def test_small_tlas_trees(n):
     visit(0)
     assert sorted(seen) == list(range(n)) and len(inner) == n - 1
     check_wide(nodes, arr["tlasNodes4"][:n - 1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quads,px,vertices", [(1, 40.0, 2), (1, 40.0, 1 << 22), (12, 2.0, 1 << 22)])
+def test_tlas_of_one_instance(quads, px, vertices):
+    """The TLAS of one instance with no CLAS (its vertices are over the
+    capacity), a single one (the BLAS root is a leaf) and 288: its record's
+    fields, and the traced frame against the oracle's."""
+    geo = scene.grid_patch(quads, quads, 1.0, 1.0)
+    cam = scene.Camera(eye=(0.5, 2.0, 0.5), center=(0.5, 0.0, 0.5), up=(0.0, 0.0, -1.0), width=96, height=56, near=0.01,
+                       far=100.0)
+    host = scene.HostScene([geo], [scene.Instance(0, np.eye(4))], [], cam, px, "one")
+    cfg = harness.small_config(maxGeneratedVertices=vertices)
+    of = harness.OracleFrame(host, cfg)
+    of.run(host.frame())
+    oh, od = of.trace(96, 56, 0)
+    g = harness.GpuFrame(host, cfg)
+    try:
+        g.run(host.frame(), stages="accel")
+        arr = g.accel_arrays()
+        gh, gd = g.trace(96, 56, 0)
+    finally:
+        g.close()
+    n = int(of.sb.blasClusterCounter)
+    assert n == (0 if vertices == 2 else 2 * quads * quads if quads > 1 else 1)
+    ti, acc = arr["tlasInstances"][0], arr["accel"]
+    assert arr["tlasRoot"] == abi.BVH_LEAF
+    assert int(ti["numClusters"]) == n and int(ti["flags"]) == 1
+    assert int(ti["blasRoot"]) == (abi.BVH_LEAF if n == 1 else 0)
+    assert int(ti["blasNodes"]) == acc.blasNodes and int(ti["blasLeaves"]) == acc.blasLeaves
+    assert np.array_equal(ti["objectToWorld"], np.eye(4, dtype=np.float32).reshape(-1)[:12])
+    assert (gh["t"] >= 0).any() == (n > 0)
+    compare_hits(gh, oh, gd, od)

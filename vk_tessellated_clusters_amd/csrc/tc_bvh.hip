@@ -464,6 +464,53 @@ __device__ __forceinline__ tc_bvh_node refit_top_node(const BvhArgs& a, uint32_t
   return out;
 }
 
+// TLAS record and world box (returned as well) of instance i.
+__device__ __forceinline__ tc_aabb tlas_prep_one(const BvhArgs& a, const float* xforms /* 24 floats per instance */, uint32_t i) {
+  const tc_blas_build_info bi = ptr<const tc_blas_build_info>(a.build->blasBuildInfos)[i];
+  const uint32_t first = (uint32_t)((bi.clusterReferences - a.build->blasClusterAddresses) / 8);
+  const uint32_t cnt = bi.clusterReferencesCount;
+  tc_tlas_instance t;
+  for (int q = 0; q < 12; q++) t.objectToWorld[q] = xforms[24 * i + q], t.worldToObject[q] = xforms[24 * i + 12 + q];
+  t.blasNodes = reinterpret_cast<uint64_t>(a.nodes + first);
+  t.blasLeaves = reinterpret_cast<uint64_t>(a.leafAddr + first);
+  t.blasRoot = cnt == 1 ? TC_BVH_LEAF : 0u;
+  t.numClusters = cnt;
+  t.flags = 1;
+  t._pad = 0;
+  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  if (cnt == 1) {
+    // a single CLAS is the root and has no parent to refit: its box and info here
+    const tc_clas_header h = *ptr<const tc_clas_header>(a.leafAddr[first]);
+    for (int q = 0; q < 3; q++) lo[q] = h.lo[q], hi[q] = h.hi[q];
+    a.leafInfo[first] = (uint64_t)h.counts | (uint64_t)h.clusterID << 32;
+  } else if (cnt > 1) {
+    const tc_aabb bx = a.nodeBox[first];
+    for (int q = 0; q < 3; q++) lo[q] = bx.lo[q], hi[q] = bx.hi[q];
+  }
+  a.tlasInst[i] = t;
+  // world box of the object box corners
+  float wlo[3] = {INFINITY, INFINITY, INFINITY}, whi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  if (cnt > 0)
+    for (int c = 0; c < 8; c++) {
+      const float p[3] = {(c & 1) ? hi[0] : lo[0], (c & 2) ? hi[1] : lo[1], (c & 4) ? hi[2] : lo[2]};
+      for (int r = 0; r < 3; r++) {
+        const float* m = t.objectToWorld + 4 * r;
+        const float w = ((m[0] * p[0] + m[1] * p[1]) + m[2] * p[2]) + m[3];
+        wlo[r] = fminf(wlo[r], w);
+        whi[r] = fmaxf(whi[r], w);
+      }
+    }
+  // widen by a few ULP-scale steps so rounding of the transformed corners
+  // never cuts off a hit found in object space
+  tc_aabb wb;
+  for (int q = 0; q < 3; q++) {
+    const float e = cnt > 0 ? 1e-6f * fmaxf(fmaxf(fabsf(wlo[q]), fabsf(whi[q])), 1e-3f) : 0.0f;
+    wb.lo[q] = wlo[q] - e, wb.hi[q] = whi[q] + e;
+  }
+  a.tlasLeafBox[i] = wb;
+  return wb;
+}
+
 // The climbs of an instance, one from each chunk boundary where the subtrees on
 // both sides wait for each other.  Higher up, a sibling is a subtree that waits
 // (read with its record ahead of this level's stores: one round trip a level),
@@ -476,12 +523,10 @@ __device__ __forceinline__ tc_bvh_node refit_top_node(const BvhArgs& a, uint32_t
 // instances of 5200 23 -> 15, 64 instances of 51,000 160 -> 122 us.  With a climb
 // for every waiting subtree instead, which needs no look-ups, 288 us and 1547 us:
 // most lanes of a wave stop at their first meeting.
-__global__ __launch_bounds__(kRefitTopThreads) void k_blas_refit_top(BvhArgs a) {
+__device__ __forceinline__ void climb_instance(const BvhArgs& a, uint32_t inst) {
   __shared__ uint32_t s_at[kTopTable];    // boundary, or ~0
   __shared__ uint32_t s_slot[kTopTable];  // 0, or the slot that waits there + 1
   __shared__ __align__(16) tc_bvh_node s_rec[kTopClimbs];  // (_pad0: far end, _pad1: outer prefix)
-  const uint32_t inst = blockIdx.x;
-  if (inst >= a.numInstances) return;
   const tc_scene_building* b = a.build;
   const uint32_t n = min(b->blasClusterCounter, a.capacity);
   const tc_blas_build_info& bi = ptr<const tc_blas_build_info>(b->blasBuildInfos)[inst];
@@ -557,51 +602,20 @@ __global__ __launch_bounds__(kRefitTopThreads) void k_blas_refit_top(BvhArgs a) 
   }
 }
 
-// TLAS record and world box (returned as well) of instance i.
-__device__ __forceinline__ tc_aabb tlas_prep_one(const BvhArgs& a, const float* xforms /* 24 floats per instance */, uint32_t i) {
-  const tc_blas_build_info bi = ptr<const tc_blas_build_info>(a.build->blasBuildInfos)[i];
-  const uint32_t first = (uint32_t)((bi.clusterReferences - a.build->blasClusterAddresses) / 8);
-  const uint32_t cnt = bi.clusterReferencesCount;
-  tc_tlas_instance t;
-  for (int q = 0; q < 12; q++) t.objectToWorld[q] = xforms[24 * i + q], t.worldToObject[q] = xforms[24 * i + 12 + q];
-  t.blasNodes = reinterpret_cast<uint64_t>(a.nodes + first);
-  t.blasLeaves = reinterpret_cast<uint64_t>(a.leafAddr + first);
-  t.blasRoot = cnt == 1 ? TC_BVH_LEAF : 0u;
-  t.numClusters = cnt;
-  t.flags = 1;
-  t._pad = 0;
-  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-  if (cnt == 1) {
-    // a single CLAS is the root and has no parent to refit: its box and info here
-    const tc_clas_header h = *ptr<const tc_clas_header>(a.leafAddr[first]);
-    for (int q = 0; q < 3; q++) lo[q] = h.lo[q], hi[q] = h.hi[q];
-    a.leafInfo[first] = (uint64_t)h.counts | (uint64_t)h.clusterID << 32;
-  } else if (cnt > 1) {
-    const tc_aabb bx = a.nodeBox[first];
-    for (int q = 0; q < 3; q++) lo[q] = bx.lo[q], hi[q] = bx.hi[q];
+// The climbs; a single instance's workgroup also writes the TLAS, which is that
+// instance alone.  Its launch would cost more than its work: frames of one
+// instance 208.9 -> 206.4 us (320 x 180), 406.4 -> 402.7 us (1280 x 720); depth
+// step on 512^2 rays 343.0 -> 339.8 us.
+__global__ __launch_bounds__(kRefitTopThreads) void k_blas_refit_top(BvhArgs a, const float* xforms) {
+  if (blockIdx.x >= a.numInstances) return;
+  climb_instance(a, blockIdx.x);
+  if (a.numInstances != 1) return;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    tlas_prep_one(a, xforms, 0);
+    a.tlasRoot[0] = TC_BVH_LEAF;
+    a.tlasRoot[1] = 1;
   }
-  a.tlasInst[i] = t;
-  // world box of the object box corners
-  float wlo[3] = {INFINITY, INFINITY, INFINITY}, whi[3] = {-INFINITY, -INFINITY, -INFINITY};
-  if (cnt > 0)
-    for (int c = 0; c < 8; c++) {
-      const float p[3] = {(c & 1) ? hi[0] : lo[0], (c & 2) ? hi[1] : lo[1], (c & 4) ? hi[2] : lo[2]};
-      for (int r = 0; r < 3; r++) {
-        const float* m = t.objectToWorld + 4 * r;
-        const float w = ((m[0] * p[0] + m[1] * p[1]) + m[2] * p[2]) + m[3];
-        wlo[r] = fminf(wlo[r], w);
-        whi[r] = fmaxf(whi[r], w);
-      }
-    }
-  // widen by a few ULP-scale steps so rounding of the transformed corners
-  // never cuts off a hit found in object space
-  tc_aabb wb;
-  for (int q = 0; q < 3; q++) {
-    const float e = cnt > 0 ? 1e-6f * fmaxf(fmaxf(fabsf(wlo[q]), fabsf(whi[q])), 1e-3f) : 0.0f;
-    wb.lo[q] = wlo[q] - e, wb.hi[q] = whi[q] + e;
-  }
-  a.tlasLeafBox[i] = wb;
-  return wb;
 }
 
 // Per-instance TLAS records and world boxes (one thread per instance).
@@ -704,16 +718,15 @@ __global__ void k_tlas_collapse4(BvhArgs a) {
 // instances the one-workgroup TLAS build (k_tlas_build_small) takes
 constexpr uint32_t kTlasRankSort = 1024;
 
-// TLAS root word (internal node 0, or the single instance) and the TLAS
-// element count read by the sort
+// TLAS root word (internal node 0) and the TLAS element count read by the sort
 __global__ void k_tlas_root(BvhArgs a) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
-    a.tlasRoot[0] = a.numInstances == 1 ? (TC_BVH_LEAF | 0u) : 0u;
+    a.tlasRoot[0] = 0;
     a.tlasRoot[1] = a.numInstances;
   }
 }
 
-// The whole TLAS in one workgroup for up to kTlasRankSort instances, one
+// The whole TLAS in one workgroup for 2 to kTlasRankSort instances, one
 // thread per instance: records and world boxes, scene bounds and keys, the
 // rank sort, the tree with its boxes from the leaves up (as k_blas_build), and
 // the binary and four-wide records.  One workgroup's chain of waits: of 28.8 us
@@ -741,7 +754,7 @@ __global__ __launch_bounds__(kTlasRankSort) void k_tlas_build_small(BvhArgs a, c
       for (int q = 0; q < 3; q++) c[q] = c[3 + q] = (bx.lo[q] + bx.hi[q]) * 0.5f;
   }
   if (i == 0) {
-    a.tlasRoot[0] = n == 1 ? (TC_BVH_LEAF | 0u) : 0u;
+    a.tlasRoot[0] = 0;
     a.tlasRoot[1] = n;
   }
   s_rank[i] = 0;
@@ -987,7 +1000,8 @@ static tc_status accel_build(const tc_bindings* b, tc_config config, const tc_ac
   a.sortedVals = sb.vals[res];
   hipLaunchKernelGGL(k_blas_build, dim3(std::min<uint32_t>((capacity + kRefitChunk - 1) / kRefitChunk, (uint32_t)num_cu_public() * 4)),
                      dim3(kRefitThreads), 0, st, a);
-  hipLaunchKernelGGL(k_blas_refit_top, dim3(a.numInstances), dim3(kRefitTopThreads), 0, st, a);
+  hipLaunchKernelGGL(k_blas_refit_top, dim3(a.numInstances), dim3(kRefitTopThreads), 0, st, a, instanceXforms);
+  if (a.numInstances == 1) return hipGetLastError() == hipSuccess ? TC_OK : TC_ERROR_LAUNCH;
   // TLAS over instances, with key and value arrays of its own
   a.tlasKeys = reinterpret_cast<uint64_t*>(m + L.tlasKeys);
   a.tlasVals = reinterpret_cast<uint32_t*>(m + L.tlasVals);
