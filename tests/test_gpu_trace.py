@@ -556,6 +556,26 @@ def test_small_tlas_trees(n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("width,height", [(480, 270), (568, 320), (592, 328), (600, 340)])
+def test_halved_tiles_beyond_residency(width, height):
+    """Tiles halved over more waves than are resident together, at both sides
+    of the rule's line (24 waves a CU): hits and decoded hits are those of the
+    packet traversal byte for byte."""
+    host = scene.scene_grid_instances(num_instances=4, quads=24, patch_size=8.0, tex_size=64, tess_rate_pixels=6.0)
+    g = harness.GpuFrame(host, harness.small_config())
+    flags = abi.TRACE_CULL_BACK | abi.TRACE_SHADOW
+    try:
+        g.run(host.frame(), stages="accel")
+        gh, gd = g.trace(width, height, flags)
+        ph, pd = g.trace(width, height, flags | abi.TRACE_PACKETS)
+    finally:
+        g.close()
+    assert (ph["t"] > 0).mean() > 0.2, "camera must see geometry"
+    assert np.array_equal(gh.view(np.uint8), ph.view(np.uint8))
+    assert np.array_equal(gd.view(np.uint8), pd.view(np.uint8))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("quads,px,vertices", [(1, 40.0, 2), (1, 40.0, 1 << 22), (12, 2.0, 1 << 22)])
 def test_tlas_of_one_instance(quads, px, vertices):
     """The TLAS of one instance with no CLAS (its vertices are over the

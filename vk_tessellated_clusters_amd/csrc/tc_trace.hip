@@ -273,12 +273,15 @@ __device__ __forceinline__ bool clas_hit(const WoopRay& r, const char* clas, uin
 // 143 < kStackDepth.
 constexpr uint32_t kLdsStack = 16;
 constexpr uint32_t kStackDepth = 160;
-// The node loop hands over to a leaf step when fewer lanes than this still
-// search (and some lane holds a leaf): the step costs what its leaves cost,
-// so it need not wait for stragglers.  4107 -> 3950 us at the 3840 x 2160
-// patch frame, 148 -> 131 us at a 320 x 180 icosphere and no difference at
-// grid64 against waiting for all; 16 and more lose at grid64 (488 -> 492-510 us).
-constexpr uint32_t kMinSearch = 8;
+// The node loop hands over to a leaf step when fewer than one in this many of
+// the lanes still in their BLAS search (the others hold a leaf): the step costs
+// what its leaves cost, so it need not wait for stragglers.  A share, not a
+// count, so that the waves of small and of ragged launches, which have few rays,
+// do not take their steps with half of them: against fewer than 8 lanes
+// icosphere 320 x 180 113 -> 91 us, grid64 480 -> 468, 500 meshes 832 -> 814,
+// 3840 x 2160 patches 3730 -> 3697.  1/2 and 1/12 lose at the small images (96
+// and 98 us), 1/8 and all at the patches (3750 and 3844).
+constexpr uint32_t kSearchShare = 4;
 constexpr uint32_t kDone = 0xFFFFFFFFu;
 
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
@@ -726,7 +729,7 @@ __device__ __forceinline__ bool trace_wave(const TraceArgs& a, WaveLds& w, RaySt
       while (true) {
         const uint64_t searching = ballot((int32_t)b >= 0);
         if (!searching) break;
-        if ((uint32_t)__popcll(searching) < kMinSearch && ballot((int32_t)b < 0 && b != kDone)) break;
+        if ((uint32_t)__popcll(searching) * kSearchShare < (uint32_t)__popcll(ballot(b != kDone))) break;
         if ((int32_t)b >= 0) b = visit_node(a.blasNodes4, first, b, ordered, ray, near, tmin, best.t, stack);
       }
       const bool has = (int32_t)b < 0 && b != kDone;
@@ -1021,16 +1024,19 @@ __device__ void decode_hit(const TraceArgs& a, const HitState& hs, tc_hit_decode
 // that chain is shorter, and the leaf steps use the idle lanes all the same.
 // While the shared waves are resident together (16 a CU; 6 for explicit rays,
 // which also come in parallel bundles that want whole waves), down to four
-// rays a wave.  Camera rays at 160 x 90 / 320 x 180 / 480 x 270: 500 meshes 600 ->
-// 210, 595 -> 385, 648 -> 512 us, icosphere 124 -> 117, 132 -> 117, 142 -> 133,
-// but past that 640 x 360 150 -> 156 and 960 x 540 191 -> 227; 16384 vertical rays
-// onto whole clusters 12.4 -> 10.2 us and onto parts 26 -> 18, 65536 of them
-// 13.6 -> 14.9 and 28 -> 25.
+// rays a wave: 160 x 90 / 320 x 180 camera rays onto 500 meshes 600 -> 244, 595 ->
+// 349 us, onto an icosphere 124 -> 92, 132 -> 98.  The first halving up to 24 a
+// CU: 480 x 270 / 560 x 315 500 meshes 562 -> 462, 548 -> 430, icosphere 138 -> 119,
+// 129 -> 121, 64 grids 207 -> 169, 222 -> 191; past it 640 x 360 150 -> 156 and
+// 960 x 540 191 -> 227.  (The further halvings up to 24 a CU, at 256 x 144: 500
+// meshes 359 -> 279, but icosphere 94 -> 102 and 25 meshes 108 -> 121.)  16384
+// vertical rays onto whole clusters 12.4 -> 10.2 us and onto parts 26 -> 18, 65536
+// of them 13.6 -> 14.9 and 28 -> 25.
 constexpr uint32_t kMaxShare = 4;
 static uint32_t tile_share(uint32_t waves, bool rays) {
-  const uint64_t limit = (uint64_t)num_cu_public() * (rays ? 6u : 16u);
+  const uint64_t cus = num_cu_public();
   uint32_t s = 0;
-  while (s < kMaxShare && ((uint64_t)waves << (s + 1)) <= limit) s++;
+  while (s < kMaxShare && ((uint64_t)waves << (s + 1)) <= cus * (rays ? 6u : s == 0 ? 24u : 16u)) s++;
   return s;
 }
 
