@@ -288,6 +288,15 @@ __global__ __launch_bounds__(kClasWaves * kWave) __attribute__((amdgpu_waves_per
           w.f[va[j]] = vx[j][0], w.f[va[j] + 1] = vx[j][1], w.f[va[j] + 2] = vx[j][2];
 #pragma unroll
         for (uint32_t j = 0; j < kRoundTris / 64; j++) w.u[ta[j]] = tw[j];
+      } else {
+        // a record of vertices or of triangles alone, in its own round
+        const uint4 rv = w.vert[done], rt = w.tri[done];
+        for (uint32_t i = lane; i < numV; i += kWave) {
+          const gfloat3 f = gld3(ptr<const float>(u64(rv.x, rv.y) + (uint64_t)i * rv.z));
+          float* v = w.f + rv.w + 3 * i;
+          v[0] = f.x, v[1] = f.y, v[2] = f.z;
+        }
+        for (uint32_t i = lane; i < numT; i += kWave) w.u[rt.z + i] = gld(ptr<const uint32_t>(u64(rt.x, rt.y)) + i);
       }
       wave_sync();
       // group boxes
