@@ -79,3 +79,36 @@ def test_clas_without_triangles(empty_templates, quads, px):
         g.close()
     assert ref.counters["tempInstantiateCounter"] >= 4 * 2 * (-(-quads // 8)) ** 2 * 3 // 4
     harness.compare(res, ref)
+
+
+@pytest.mark.parametrize("num", [300, 60000])
+def test_trace_past_blocks_without_triangles(empty_templates, num):
+    """Leaf steps whose lanes hold blocks without triangles beside others.
+    Vertical rays take the general slab test, which an inverted box passes, so
+    they enter such blocks in every tree; an instance of one such block alone
+    is entered by all rays.  Few rays (shared waves) and many (whole waves), in
+    one order and mixed: hits and decoded hits are the oracle's."""
+    host = mixed_scene(24, 2.0)
+    cfg = harness.small_config()
+    rng = np.random.default_rng(num)
+    rays = np.zeros(num, abi.RAY_DT)
+    rays["origin"] = rng.uniform(-1.0, 15.0, (num, 3))
+    rays["origin"][:, 1] = 6.0
+    kind = np.arange(num) % 3
+    rays["direction"] = np.where((kind == 0)[:, None], (0.0, -1.0, 0.0),
+                                 rng.uniform(-0.4, 0.4, (num, 3)) * (1, 0, 1) + (0.003, -1.0, 0.002))
+    rays["tMin"], rays["tMax"] = 0.0, 100.0
+    of = harness.OracleFrame(host, cfg)
+    of.run(host.frame())
+    g = harness.GpuFrame(host, cfg)
+    try:
+        g.run(host.frame(), stages="accel")
+        for order in (np.argsort(kind, kind="stable"), np.arange(num)):
+            some = np.ascontiguousarray(rays[order])
+            oh, od = of.trace(0, 0, 0, rays=some)
+            assert (oh["t"] > 0).mean() > 0.3, "rays must meet the surface"
+            for flags in (0, abi.TRACE_PRIVATE_STACK, abi.TRACE_PACKETS):
+                gh, gd = g.trace(0, 0, flags, rays=some)
+                harness.compare_hits(gh, oh, gd, od)
+    finally:
+        g.close()

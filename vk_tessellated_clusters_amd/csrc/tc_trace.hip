@@ -524,7 +524,9 @@ __device__ __forceinline__ void leaf_step(WaveLds& w, bool has, const char* clas
   const uint32_t total = __builtin_amdgcn_readlane(end, 63);
   if (lane < 16) w.heads[lane] = 0;
   wave_sync();
-  const uint64_t holders = ballot(has);
+  // a block without triangles has no pairs: its first is its successor's, so it
+  // takes no entry and no bit
+  const uint64_t holders = ballot(npairs != 0);
   if (has) {
     const uint64_t addr = reinterpret_cast<uint64_t>(clas);
     w.rayO[lane] = make_float4(ray.o[0], ray.o[1], ray.o[2], tmax);
@@ -532,9 +534,11 @@ __device__ __forceinline__ void leaf_step(WaveLds& w, bool has, const char* clas
     w.rayS[lane] = make_float4(ray.Sx, ray.Sy, ray.Sz,
                                __uint_as_float((uint32_t)(ray.kx | ray.ky << 2 | ray.kz << 4) | nt << 8 | ng << 16));
     w.leaf[lane] = make_uint4((uint32_t)addr, (uint32_t)(addr >> 32), ~0u, ~0u);
-    w.lanes[mask_prefix(holders)] = lane | ng << 8 | first << 16;
-    __hip_atomic_fetch_or(reinterpret_cast<uint32_t*>(w.heads) + (first >> 5), 1u << (first & 31), __ATOMIC_RELAXED,
-                          __HIP_MEMORY_SCOPE_WAVEFRONT);
+    if (npairs != 0) {
+      w.lanes[mask_prefix(holders)] = lane | ng << 8 | first << 16;
+      __hip_atomic_fetch_or(reinterpret_cast<uint32_t*>(w.heads) + (first >> 5), 1u << (first & 31), __ATOMIC_RELAXED,
+                            __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
   }
   wave_sync();
   // Which way the group boxes are tested, by what the two cost in units of
