@@ -606,3 +606,58 @@ def test_tlas_of_one_instance(quads, px, vertices):
     assert np.array_equal(ti["objectToWorld"], np.eye(4, dtype=np.float32).reshape(-1)[:12])
     assert (gh["t"] >= 0).any() == (n > 0)
     compare_hits(gh, oh, gd, od)
+
+
+def big_cluster_patch(n, q):
+    """n x n clusters of q x q quads over [0, n]^2 (more triangles than the
+    pipeline's 128 a cluster), with a bumpy surface."""
+    ii, jj = np.meshgrid(np.arange(q + 1), np.arange(q + 1), indexing="xy")
+    a = (jj[:-1, :-1] * (q + 1) + ii[:-1, :-1]).reshape(-1)
+    tri = np.stack([np.stack([a, a + q + 1, a + 1], 1), np.stack([a + 1, a + q + 1, a + q + 2], 1)], 1).reshape(-1, 3)
+    nv, nt = (q + 1) ** 2, 2 * q * q
+    clusters, bboxes, pos = np.zeros(n * n, abi.CLUSTER_DT), np.zeros(n * n, abi.BBOX_DT), []
+    for c in range(n * n):
+        x, z = c % n + ii.reshape(-1) / q, c // n + jj.reshape(-1) / q
+        p = np.stack([x, 0.1 * np.sin(7.0 * x) * np.cos(5.0 * z), z], 1)
+        clusters[c] = (nv, nt, c * nt, c * nv, 3 * c * nt)
+        bboxes[c] = (p.min(0), p.max(0), 0.0, 1.0)
+        pos.append(p)
+    pos = np.ascontiguousarray(np.concatenate(pos), np.float32)
+    g = scene.Geometry(pos, np.tile(np.float32([0, 1, 0]), (len(pos), 1)), np.ascontiguousarray(pos[:, ::2] / n), clusters,
+                       np.tile(tri.astype(np.uint8).reshape(-1), n * n), bboxes)
+    g.lo, g.hi = pos.min(0), pos.max(0)
+    return g
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q,num", [(8, 60000), (10, 300), (10, 60000), (11, 60000)])
+def test_blocks_of_more_than_32_groups(q, num):
+    """Clusters of 200 and 242 triangles (templates may hold that many) give
+    blocks of 25 and 31 group pairs: a wave of parallel rays deals out more
+    pairs than 64 lanes of whole pipeline clusters (8 x 8 quads) have.  Hits
+    are the oracle's."""
+    geo = big_cluster_patch(6, q)
+    cam = scene.Camera(eye=(3.0, 4.0, 3.0), center=(3.0, 0.0, 3.0), up=(0.0, 0.0, -1.0), width=96, height=56, near=0.01,
+                       far=100.0)
+    insts = [scene.Instance(0, scene.rigid_transform(0.2, [0.0, 0.3 * k, 0.0])) for k in range(2)]
+    host = scene.HostScene([geo], insts, [], cam, 4000.0, "big")
+    cfg = harness.small_config()
+    rng = np.random.default_rng(num)
+    rays = np.zeros(num, abi.RAY_DT)
+    rays["origin"] = rng.uniform(0.0, 6.0, (num, 3))
+    rays["origin"][:, 1] = 5.0
+    rays["direction"] = (0.01, -1.0, 0.02)
+    rays["direction"][num // 2:] = (0.0, -1.0, 0.0)
+    rays["tMin"], rays["tMax"] = 0.0, 100.0
+    of = harness.OracleFrame(host, cfg)
+    of.run(host.frame())
+    oh, od = of.trace(0, 0, 0, rays=rays)
+    assert of.sb.tempInstantiateCounter == 2 * 36 and (oh["t"] > 0).mean() > 0.5
+    g = harness.GpuFrame(host, cfg)
+    try:
+        g.run(host.frame(), stages="accel")
+        got = [g.trace(0, 0, f, rays=rays) for f in (0, abi.TRACE_PRIVATE_STACK)]
+    finally:
+        g.close()
+    for gh, gd in got:
+        harness.compare_hits(gh, oh, gd, od)

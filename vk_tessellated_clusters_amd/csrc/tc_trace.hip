@@ -454,6 +454,10 @@ __device__ __forceinline__ uint32_t visit_node(const tc_bvh4_node* nodes, uint32
 
 // LDS of one wave: the lanes' stacks and the state of a leaf step.
 constexpr uint32_t kLeafQueue = 144;  // 15 left over + 128 of one step, rounded up
+// Group pairs of a block, at most: its header counts 255 triangles
+// (tc_cluster_template_order takes 256; clusters of the pipeline have 128 and
+// 16 pairs).
+constexpr uint32_t kBlockPairs = (255 + 2 * TC_CLAS_GROUP_TRIANGLES - 1) / (2 * TC_CLAS_GROUP_TRIANGLES);
 struct WaveLds {
   uint32_t stack[kLdsStack * kWave];
   float4 rayO[kWave];          // origin, closest hit so far
@@ -461,7 +465,7 @@ struct WaveLds {
   float4 rayS[kWave];          // shear, permutation | triangles << 8 | groups << 16
   uint4 leaf[kWave];           // CLAS address, (ordered t, primitive) of the closest hit
   float4 won[kWave];           // that hit's V, W, determinant and triangle word
-  uint64_t heads[16];          // bit per group-box pair: the first of its lane
+  uint64_t heads[kBlockPairs]; // bit per group-box pair: the first of its lane
   uint32_t lanes[kWave];       // lanes with leaves, in order: lane | groups << 8 | first pair << 16
   uint16_t queue[kLeafQueue];  // groups entered: lane | group << 6
 };
@@ -519,10 +523,10 @@ __device__ __forceinline__ void leaf_step(WaveLds& w, bool has, const char* clas
                                           float tmin, float tmax, bool cullBack, bool anyHit) {
   const uint32_t lane = lane_id();
   const uint32_t nt = (uint32_t)info & 0xFF, ng = ((uint32_t)info >> 16) & 0xFF;
-  const uint32_t npairs = has ? (ng + 1) >> 1 : 0;
+  const uint32_t npairs = has ? min((ng + 1) >> 1, kBlockPairs) : 0;
   const uint32_t end = wave_scan_dpp(npairs), first = end - npairs;
   const uint32_t total = __builtin_amdgcn_readlane(end, 63);
-  if (lane < 16) w.heads[lane] = 0;
+  if (lane < kBlockPairs) w.heads[lane] = 0;
   wave_sync();
   // a block without triangles has no pairs: its first is its successor's, so it
   // takes no entry and no bit
@@ -555,7 +559,8 @@ __device__ __forceinline__ void leaf_step(WaveLds& w, bool has, const char* clas
   most = max(most, (uint32_t)__builtin_amdgcn_update_dpp(0, most, 0x142, 0xa, 0xf, false));
   most = max(most, (uint32_t)__builtin_amdgcn_update_dpp(0, most, 0x143, 0xc, 0xf, false));
   most = __builtin_amdgcn_readlane(most, 63);
-  const bool own = (most == 1 ? 1 : (most + 1) & ~1u) + 2 <= 2 * ((total + kWave - 1) / kWave);
+  // (A lane's own groups are bits of one word.)
+  const bool own = most <= 16 && (most == 1 ? 1 : (most + 1) & ~1u) + 2 <= 2 * ((total + kWave - 1) / kWave);
   uint32_t mask = 0;  // own: this lane's groups entered and not queued yet
   if (own) {
     const float4* gq = reinterpret_cast<const float4*>(clas + sizeof(tc_clas_header));
