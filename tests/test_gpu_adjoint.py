@@ -161,3 +161,40 @@ def test_gradient_of_scattered_rays(rays):
     assert rays == 32 or np.count_nonzero(want) > rays * rays / 4
     k = max(256.0, 12.0 * rays * rays / SIZE ** 2 * 16)
     assert (np.abs(got - want) <= 2 * k * 2.0 ** -24 * np.abs(want) + 1e-30).all()
+
+
+@pytest.mark.parametrize("rays", [7, 64, 181, 182, 255, 256, 362, 363])
+def test_gradient_by_ray_count_matches_fp64(rays):
+    """Workgroups of 128, 256, 512 and 1024 rays, at both sides of each line
+    (32, 64 and 128 thousand rays on 256 CUs) and for fewer rays than one
+    workgroup: the gradient of the rays in row order and in random order (whose
+    texels overflow the tables) against the FP64 adjoint, within the bounds of
+    test_gradient_matches_fp64_adjoint."""
+    import torch
+    from vk_tessellated_clusters_amd import diff, scene
+    hmap = (0.5 * scene.fbm_height(SIZE, 7, 4)).astype(np.float32)
+    r = diff.DepthRenderer(torch.from_numpy(hmap).cuda(), rays=rays)
+    rng = np.random.default_rng(rays)
+    g = (rng.random(rays * rays) + 0.5).astype(np.float32)
+    perm = rng.permutation(rays * rays)
+    try:
+        r.render()
+        st = r.host_state()
+        rows = r.adjoint(torch.from_numpy(g).cuda())
+        dperm = torch.from_numpy(perm).cuda()
+        for name, width in (("rays", abi.RAY_DT.itemsize), ("hits", abi.HIT_DT.itemsize)):
+            b = getattr(r, name).view(-1, width)
+            b.copy_(b[dperm].clone())
+        hv = r.hit_vertices.view(-1, 4)
+        hv.copy_(hv[dperm].clone())
+        mixed = r.adjoint(torch.from_numpy(g[perm]).cuda())
+        torch.cuda.synchronize()
+    finally:
+        r.close()
+    assert (st["hits"]["t"] >= 0).mean() > 0.5  # (vertical rays on the lines of 7 x 7 lie in box planes and miss)
+    (ref,) = Problem(st["rays"], st["hits"], st["hitVertices"], st["tape"], [hmap], st["xforms"]).adjoint64(g)
+    scale = np.abs(ref).max()
+    assert scale > 0
+    for got in (rows, mixed):
+        err = np.abs(got.double().cpu().numpy() - ref)
+        assert (err <= 1e-3 * np.abs(ref) + 1e-5 * scale).all(), (err / (np.abs(ref) + 1e-5 * scale)).max()
