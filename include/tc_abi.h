@@ -599,10 +599,10 @@ typedef struct tc_tuning {
   uint32_t classifyBlocksPerCU;    /* cluster_classify, 256-thread workgroups */
   uint32_t splitBlocksPerCU;       /* triangle_split, 64-thread workgroups */
   uint32_t instantiateBlocksPerCU; /* template instantiate, 256-thread workgroups */
-  uint32_t clasWavesPerCU;         /* CLAS build, one wave per CLAS */
+  uint32_t clasWavesPerCU;         /* CLAS build, waves at most: runs of 1 to 16 templates, a transient CLAS each */
   uint32_t traceBlocksPerCU;       /* traversal workgroups per CU */
   uint32_t traceThreads;           /* traversal workgroup size */
-  uint32_t bvhBlocksPerCU;         /* BVH keys of tc_accel_build */
+  uint32_t bvhBlocksPerCU;         /* BVH keys of tc_accel_build (a renderer's frame has no such launch) */
   /* Sleeps before a wait of the persistent split gives up and flags the
    * frame (TC_READBACK_ERROR_SPLIT_WAIT); default 2^24, and 0 in
    * tc_set_tuning restores it.  Not a performance knob: only failure-path

@@ -143,3 +143,12 @@ def test_noalloc_tessellate_rejects_oversized_configs():
         assert L.tc_frame_tessellate_noalloc(C.byref(b), cfg, 0, None) == abi.TC_ERROR_CAPACITY, field
     bad = abi.default_config(clusterTriangleCount=0)
     assert L.tc_frame_tessellate_noalloc(C.byref(b), bad, 0, None) == abi.TC_ERROR_INVALID_ARGUMENT
+
+
+def test_autotuner_varies_what_frames_read():
+    """The tuner times whole frames, so every shape it tries has to reach
+    one: the wait limit is no shape, and the key launch of tc_accel_build is
+    not part of a renderer's frame."""
+    from vk_tessellated_clusters_amd import autotune
+    fields = {n for n, _ in abi.Tuning._fields_}
+    assert set(autotune.CANDIDATES) == fields - {"splitWaitLimit", "bvhBlocksPerCU"}

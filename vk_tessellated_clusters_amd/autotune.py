@@ -11,6 +11,8 @@ import ctypes as C
 
 from . import abi
 
+# Shapes that a renderer's frame reads (bvhBlocksPerCU is the key launch of
+# tc_accel_build, which frames do not make).
 CANDIDATES = {
     "classifyBlocksPerCU": [2, 3, 4, 5, 8],
     "splitBlocksPerCU": [2, 4, 8, 16],
@@ -18,7 +20,6 @@ CANDIDATES = {
     "clasWavesPerCU": [16, 32, 64, 128],
     "traceThreads": [64, 128, 256],
     "traceBlocksPerCU": [32, 64, 128, 256, 512],
-    "bvhBlocksPerCU": [4, 8, 16],
 }
 
 
