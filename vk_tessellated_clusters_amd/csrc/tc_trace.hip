@@ -64,7 +64,9 @@ __device__ __forceinline__ void setup_ray(WoopRay& r, const float o[3], const fl
   r.Sz = pick3(r.inv[0], r.inv[1], r.inv[2], r.kz);  // 1 / dz
 }
 
-// conservative slab test; returns entry distance or +inf
+// Slab test; returns the entry distance or +inf.  A ray that lies in a plane of
+// the box (parallel to it, its origin on it) has 0 * inf in that slab, which
+// counts as the other plane's infinity: it misses.
 __device__ __forceinline__ float box_hit(const WoopRay& r, const float lo[3], const float hi[3], float tmin, float tmax) {
   float tn = tmin, tf = tmax;
 #pragma unroll
@@ -266,13 +268,16 @@ __device__ __forceinline__ bool clas_hit(const WoopRay& r, const char* clas, uin
 // visits every other level, so a ray holds at most 3 * (ceil(dT / 2) +
 // ceil(dB / 2)) entries and two sentinels for binary depths dT (TLAS) and dB
 // (BLAS).  A Karras tree's depth is at most its distinct key bits plus the
-// index bits that break ties.  TLAS keys are a 30-bit Morton code above the
-// instance index, so dT <= 30 + 16 = 46 (2^16 instances); a BLAS covers one
-// instance's segment, whose keys differ only in the 24-bit Morton code, so
-// dB <= 24 + 23 = 47 (2^23 references).  That is at most 3 * (23 + 24) + 2 =
-// 143 < kStackDepth.
+// index bits that break ties.  TLAS keys are a 30-bit Morton code, all ones for
+// empty instances (one more bit that differs), above the instance index of at
+// most 16 bits; a BLAS covers one instance's segment, whose keys differ only in
+// the 24-bit Morton code, and its positions have at most 31 bits (the 32nd marks
+// a leaf).
 constexpr uint32_t kLdsStack = 16;
 constexpr uint32_t kStackDepth = 160;
+constexpr uint32_t kTlasDepth = 30 + 1 + 16, kBlasDepth = 24 + 31;
+constexpr uint32_t kMostEntries = 3 * ((kTlasDepth + 1) / 2 + (kBlasDepth + 1) / 2);
+static_assert(kMostEntries + 2 <= kStackDepth, "entries and sentinels of the deepest trees");
 // The node loop hands over to a leaf step when fewer than one in this many of
 // the lanes still in their BLAS search (the others hold a leaf): the step costs
 // what its leaves cost, so it need not wait for stragglers.  A share, not a
@@ -784,6 +789,7 @@ __device__ __forceinline__ bool trace_wave(const TraceArgs& a, WaveLds& w, RaySt
 // wave.  Suited to coherent rays: camera rays in 8 x 8 pixel tiles and their
 // shadow rays.
 constexpr uint32_t kPacketStack = 160;
+static_assert(kMostEntries <= kPacketStack, "entries of the deepest trees");
 constexpr uint32_t kBlasEntry = 1u << 30;  // packet stack: marks BLAS entries
 
 __device__ __forceinline__ float wave_min_f(float v) {
