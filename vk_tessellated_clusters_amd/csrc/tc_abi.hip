@@ -656,9 +656,10 @@ extern "C" {
 // file-scope array instead of the caller's workspace.  Each device holds
 // its own copy from module load to process end.  It starts zeroed, as
 // tc_workspace_init leaves a workspace; after that nothing needs clearing
-// between calls: every stage's prologue resets the ticket and opens a new
-// epoch, and status words of earlier epochs read as unpublished.  Calls
-// that overlap on one device race on it.
+// between calls: the sequence's first launch resets every stage's ticket and
+// opens the epochs of all stages (with the persistent split each stage's
+// prologue opens its own), and status words of earlier epochs read as
+// unpublished.  Calls that overlap on one device race on it.
 constexpr uint32_t kScratchTiles = 16384;
 constexpr uint64_t kScratchBytes = kWsHeaderBytes + (uint64_t)kMaxCounters * kScratchTiles * 8;
 static __device__ __align__(256) uint64_t scratch[kScratchBytes / 8];

@@ -388,14 +388,14 @@ __global__ void k_insert_scatter(KArgs a, const uint64_t* keys, const uint32_t* 
 // ---------------------------------------- insertion and BLAS keys together
 
 // A pass over the CLAS of both lists (templates, then transient builds) by a
-// digit of their instance: as k_sort_pass, whose tiles it has.  FIRST reads the
-// lists, the second pass the (instance, position) pairs that the first one
-// wrote.  LAST writes the reference lists: instance digits alone order them,
-// so the place of a CLAS is its place among all references.  Past two tiles a
-// CU a workgroup takes several, so that no more of them add their Morton counts
-// and sizes to the totals.  Bound by its chain of waits (ticket, lists, walk,
-// totals), so tiles are small while they are few: 125k CLAS 29 us in tiles of
-// 2048 and 23 us in tiles of 512.
+// digit of their instance: as k_sort_pass, but in tiles of 256 to 2048 CLAS by
+// their number (insert_rounds).  FIRST reads the lists, the second pass the
+// (instance, position) pairs that the first one wrote.  LAST writes the
+// reference lists: instance digits alone order them, so the place of a CLAS is
+// its place among all references.  Past two tiles a CU a workgroup takes several,
+// so that no more of them add their Morton counts and sizes to the totals.  Bound
+// by its chain of waits (ticket, lists, walk, totals), so tiles are small while
+// they are few: 125k CLAS 29 us in tiles of 2048 and 23 us in tiles of 512.
 template <bool FIRST, bool LAST>
 __global__ __launch_bounds__(kSortThreads) void k_insert_pass(KArgs a, InsertPlan ip, uint64_t* pairs, uint64_t* keys,
                                                               uint32_t* vals) {

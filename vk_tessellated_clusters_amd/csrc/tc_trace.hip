@@ -5,8 +5,8 @@
 // glsl:128-236, 338-339 (decode, depth) and render_shading.glsl:263-274
 // (shadow rays).  One ray per lane over the four-wide views of the TLAS and
 // the BLAS; the lane's stack (LDS, overflowing into private memory) holds
-// TLAS and BLAS entries (the BLAS entries of the instance being walked lie
-// above the depth it was entered at).  Triangles use the watertight test of
+// TLAS and BLAS entries (those of the instance being walked lie above a
+// sentinel).  Triangles use the watertight test of
 // Woop, Benthin and Wald (JCGT 2013) with an FP64 recomputation of zero edge
 // functions; closest-hit ties are broken by (instance, cluster, primitive)
 // so the result does not depend on traversal order.
@@ -512,7 +512,7 @@ __device__ __forceinline__ bool key_less(float t, uint32_t i, uint32_t c, uint32
 
 // Intersects the CLAS blocks that the wave's lanes hold (`has`), sharing the
 // work over all 64 lanes; the whole wave calls it.  The traversal is bound by
-// VALU issue (82 % busy at grid64), and what it issues is mostly idle lanes:
+// VALU issue (74 % busy at grid64), and what it issues is mostly idle lanes:
 // about 22 of 64 lanes arrive with a leaf, their blocks hold 2 to 32 groups,
 // and when each lane tested its own block's triangles 15 of 64 lanes were at
 // work.  So every lane puts its ray in LDS, the group boxes of all blocks are
