@@ -22,14 +22,6 @@
 
 namespace tc {
 
-__device__ __forceinline__ uint32_t expand_bits(uint32_t v) {
-  v = (v | (v << 16)) & 0x030000FFu;
-  v = (v | (v << 8)) & 0x0300F00Fu;
-  v = (v | (v << 4)) & 0x030C30C3u;
-  v = (v | (v << 2)) & 0x09249249u;
-  return v;
-}
-
 // 30-bit Morton code of the box centre, normalised to [lo, hi]
 __host__ __device__ __forceinline__ uint32_t morton_of(const float* blo, const float* bhi, const float* lo,
                                                        const float* hi) {
@@ -464,7 +456,7 @@ __device__ __forceinline__ tc_bvh_node refit_top_node(const BvhArgs& a, uint32_t
   return out;
 }
 
-// TLAS record and world box (returned as well) of instance i.
+// TLAS record (written) and world box of instance i.
 __device__ __forceinline__ tc_aabb tlas_prep_one(const BvhArgs& a, const float* xforms /* 24 floats per instance */, uint32_t i) {
   const tc_blas_build_info bi = ptr<const tc_blas_build_info>(a.build->blasBuildInfos)[i];
   const uint32_t first = (uint32_t)((bi.clusterReferences - a.build->blasClusterAddresses) / 8);
@@ -507,7 +499,6 @@ __device__ __forceinline__ tc_aabb tlas_prep_one(const BvhArgs& a, const float* 
     const float e = cnt > 0 ? 1e-6f * fmaxf(fmaxf(fabsf(wlo[q]), fabsf(whi[q])), 1e-3f) : 0.0f;
     wb.lo[q] = wlo[q] - e, wb.hi[q] = whi[q] + e;
   }
-  a.tlasLeafBox[i] = wb;
   return wb;
 }
 
@@ -621,7 +612,7 @@ __global__ __launch_bounds__(kRefitTopThreads) void k_blas_refit_top(BvhArgs a, 
 // Per-instance TLAS records and world boxes (one thread per instance).
 __global__ void k_tlas_prep(BvhArgs a, const float* xforms) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < a.numInstances) tlas_prep_one(a, xforms, i);
+  if (i < a.numInstances) a.tlasLeafBox[i] = tlas_prep_one(a, xforms, i);
 }
 
 // Scene bounds and TLAS keys over instances (one workgroup).
@@ -797,8 +788,6 @@ __global__ __launch_bounds__(kTlasRankSort) void k_tlas_build_small(BvhArgs a, c
   if (i < n) {
     const uint32_t rank = s_rank[i];
     const uint64_t k = s_key[i];
-    a.tlasKeys[rank] = k;
-    a.tlasVals[rank] = i;
     s_sorted[rank] = k;
     s_val[rank] = i;
     s_leaf[rank] = bx;

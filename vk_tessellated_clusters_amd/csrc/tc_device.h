@@ -648,13 +648,6 @@ __device__ __forceinline__ void atomic_store_agent(uint64_t* p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Takes the next tile ticket (whole wave; returns a wave-uniform value).
-__device__ __forceinline__ uint32_t take_ticket(WsHeader* h) {
-  uint32_t t = 0;
-  if (lane_id() == 0) t = __hip_atomic_fetch_add(&h->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return uniform(t);
-}
-
 // The next ticket of a launch with numTiles tiles, or numTiles once they
 // are all taken.  Tickets only grow, so a read at or past numTiles means no
 // work is left, and the workgroups of an empty launch (a split pass with
